@@ -25,6 +25,25 @@ def scan_of(N, nz, rot_shift=0.0, n_frames=2, n_views=22, **kw):
     return s
 
 
+@pytest.mark.parametrize("N,nz,shift", [(16, 1, 0.0), (17, 3, 0.0), (33, 4, 2.5), (31, 5, -3.0),
+                                        (40, 8, 0.5), (26, 9, 7.0), (64, 17, 0.0)])
+def test_fbp_groups_and_edges(N, nz, shift):
+    """Within 1e-5 of the largest value of the FP64 numpy statement (the
+    output is FP32, its sums FP64), for every remainder of the slice groups
+    and of the filter's output groups."""
+    print(f"fbp N={N} nz={nz} shift={shift}", flush=True)
+    scan = scan_of(N, nz, shift)
+    st = tb.Stage(scan)
+    off = np.random.default_rng(4).normal(0, 0.01, (N, nz)).astype(np.float32)
+    st.set_offset(off)
+    st.init_fbp()
+    got = st.object()
+    ref = stage_fbp_reference(scan, st, off)
+    st.close()
+    assert np.abs(ref).max() > 0
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+
+
 @pytest.mark.parametrize("scale", [0.0, 1e-42, 1e-30, 1e-12, 1.0, 1e12, 1e20])
 @pytest.mark.parametrize("shape", [(1, 1, 5), (2, 3, 17), (3, 2, 19)])
 def test_prior_cost_over_the_float_range(scale, shape):

@@ -21,7 +21,8 @@ namespace tb {
 __global__ void k_transpose_in(KP, const float *, const float *, double);
 __global__ void k_to_ref_layout(KP, const float *, float *);
 __global__ void k_fwd_interleave(KP, float4 *);
-__global__ void k_fbp_filter(KP, float *);
+__global__ void k_fbp_filter(KP, float *, int);
+template <int NZ>
 __global__ void k_fbp_back(KP, const float *);
 __global__ void k_forward(KP, const int *, const float4 *, float *, int);
 __global__ void k_upsample(const float *, float *, int, int, int, int, int);
@@ -853,10 +854,18 @@ extern "C" int tb_init_fbp(tb_stage *st) {
     return fail("tb_init_fbp: %d detector bins exceed the filter's LDS row", st->N_r);
   KP P = st->kp();
   float *q = nullptr;
-  HIPCHK(dalloc(&q, (size_t)st->N_z * st->N_p * st->N_r));
-  hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, st->N_z), dim3(256),
-                     st->N_r * sizeof(double), st->stream, P, q);
-  hipLaunchKernelGGL(k_fbp_back, dim3(grid_for(st->nobj())), dim3(256), 0, st->stream, P, q);
+  const int ngroups = (st->N_z + kFwdZ - 1) / kFwdZ;
+  // the filter's taps and as many detector rows of a group as 48 KB hold
+  const size_t taps = 2 * (size_t)((st->N_r + 2 * kFbpF + 1) / 2);
+  const int per = (int)std::max<size_t>(1, std::min<size_t>(kFwdZ, 6144 / st->N_r));
+  const size_t lds = (taps + (size_t)per * st->N_r) * sizeof(double);
+  HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_fbp_filter),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  HIPCHK(dalloc(&q, (size_t)ngroups * kFwdZ * st->N_p * st->N_r));
+  hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, ngroups), dim3(512), lds, st->stream, P, q, per);
+  const dim3 grid((unsigned)((st->nxy() + 255) / 256 * st->N_time * ngroups));
+  if (st->N_z <= 4) hipLaunchKernelGGL(k_fbp_back<4>, grid, dim3(256), 0, st->stream, P, q);
+  else hipLaunchKernelGGL(k_fbp_back<8>, grid, dim3(256), 0, st->stream, P, q);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess) err = hipStreamSynchronize(st->stream);
   (void)hipFree(q);

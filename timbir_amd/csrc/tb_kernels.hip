@@ -242,62 +242,123 @@ __global__ __launch_bounds__(kFwdT) void k_forward(KP P, const int *__restrict__
 //   k_fbp_back: x[f][z][pixel] = (pi / n_f) sum over the n_f views of frame
 //     f of q at the pixel's ray, linearly interpolated between bin centres;
 //     zero outside the reconstruction mask.
+//
+// Bound: FP64 arithmetic and the L1 reads of q.  The filter keeps the kernel's
+// odd taps in LDS (no division per tap), takes `per` slices of a view at once
+// and gives a thread kFbpF outputs of one parity, which share each sample and
+// all but one tap.  The back-projection's geometry (ray, bin, fraction)
+// depends on the pixel and view alone: a thread evaluates it once for NZ
+// slices, whose filtered rows lie side by side in q[group][v][r][kFwdZ].  With
+// a division per tap and a thread per voxel the two took 1.34 and 6.62 ms for
+// 512 x 512 x 16 slices x 8 frames and 1024 views, in this form 0.25 and 0.97.
 // ---------------------------------------------------------------------------
-__global__ void k_fbp_filter(KP P, float *__restrict__ q) {
-  extern __shared__ double s_p[];  // one detector row
-  const int v = blockIdx.x, z = blockIdx.y;
-  for (int r = threadIdx.x; r < P.N_r; r += blockDim.x) {
-    double acc = 0.0;
-    for (int m = 0; m < P.mz; m++) {
-      const size_t o = sidx(P, z, v, r, m);
-      acc += (double)P.y[o] - (double)P.d[(size_t)r * P.N_t + z * P.mz + m];
-    }
-    s_p[r] = acc / P.mz;
+__global__ __launch_bounds__(512) void k_fbp_filter(KP P, float *__restrict__ q, int per) {
+  extern __shared__ double s_h[];  // the taps, then `per` detector rows
+  const int v = blockIdx.x, g = blockIdx.y;
+  const int half = (P.N_r + 2 * kFbpF + 1) / 2;
+  double *s_p = s_h + 2 * half;
+  // s_h[half + i]: tap of offset 2 i + 1
+  for (int i = threadIdx.x; i < 2 * half; i += blockDim.x) {
+    const double n = 2.0 * (i - half) + 1.0;
+    s_h[i] = -1.0 / (kPi * kPi) / (n * n);
   }
-  __syncthreads();
   const double h = P.delta_r;
-  const double k_odd = -1.0 / (kPi * kPi);
-  for (int r = threadIdx.x; r < P.N_r; r += blockDim.x) {
-    double acc = 0.25 * s_p[r];
-    // odd offsets n = r - k
-    for (int k = (r & 1) ^ 1; k < P.N_r; k += 2) {
-      const double n = (double)(r - k);
-      acc += k_odd * s_p[k] / (n * n);
+  float *out = q + ((size_t)g * P.N_p + v) * P.N_r * kFwdZ;
+  // item: outputs r0, r0 + 2, .. of one parity, from the samples of the other
+  const int items = 2 * ((P.N_r + 2 * kFbpF - 1) / (2 * kFbpF));
+  const int nz = min(kFwdZ, P.N_z - g * kFwdZ);
+  for (int z0 = 0; z0 < nz; z0 += per) {
+    const int ns = min(per, nz - z0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < ns * P.N_r; i += blockDim.x) {
+      const int sl = i / P.N_r, r = i - sl * P.N_r, z = g * kFwdZ + z0 + sl;
+      double acc = 0.0;
+      for (int m = 0; m < P.mz; m++)
+        acc += (double)P.y[sidx(P, z, v, r, m)] - (double)P.d[(size_t)r * P.N_t + z * P.mz + m];
+      s_p[i] = acc / P.mz;
     }
-    q[((size_t)z * P.N_p + v) * P.N_r + r] = (float)(acc / h);
+    __syncthreads();
+    for (int it = threadIdx.x; it < ns * items; it += blockDim.x) {
+      const int sl = it / items, i1 = it - sl * items;
+      const double *sp = s_p + sl * P.N_r;
+      const int r0 = (i1 >> 1) * 2 * kFbpF + (i1 & 1);
+      double acc[kFbpF], t[kFbpF];
+#pragma unroll
+      for (int u = 0; u < kFbpF; u++) acc[u] = r0 + 2 * u < P.N_r ? 0.25 * sp[r0 + 2 * u] : 0.0;
+      // odd offsets r0 + 2 u - k = 2 (i0 - half + u) + 1
+      const int k0 = (r0 & 1) ^ 1;
+      int i0 = (r0 < k0 ? -1 : (r0 - k0 - 1) / 2) + half;
+#pragma unroll
+      for (int u = 0; u < kFbpF; u++) t[u] = s_h[i0 + u];
+      for (int k = k0; k < P.N_r; k += 2) {
+        const double x = sp[k];
+#pragma unroll
+        for (int u = 0; u < kFbpF; u++) acc[u] = fma(t[u], x, acc[u]);
+#pragma unroll
+        for (int u = kFbpF - 1; u > 0; u--) t[u] = t[u - 1];
+        i0--;
+        t[0] = s_h[max(i0, 0)];
+      }
+#pragma unroll
+      for (int u = 0; u < kFbpF; u++)
+        if (r0 + 2 * u < P.N_r) out[(size_t)(r0 + 2 * u) * kFwdZ + z0 + sl] = (float)(acc[u] / h);
+    }
   }
 }
 
-__global__ void k_fbp_back(KP P, const float *__restrict__ q) {
-  const size_t Nxy = (size_t)P.N_x * P.N_y;
-  const size_t n = (size_t)P.N_time * P.N_z * Nxy;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    const size_t pix = i % Nxy;
-    const int z = (int)((i / Nxy) % P.N_z), f = (int)(i / (Nxy * P.N_z));
-    const int row = (int)(pix / P.N_x), col = (int)(pix % P.N_x);
-    float out = 0.0f;
-    const int vb = P.view_off[f], nv = P.view_off[f + 1] - vb;
-    if (P.mask[pix] && nv > 0) {
+// thread: one pixel of one frame, NZ slices (blocks: frame, group, run of pixels)
+template <int NZ>
+__global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q) {
+  const int Nxy = P.N_x * P.N_y;
+  const int ngroups = (P.N_z + kFwdZ - 1) / kFwdZ;
+  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, f = fg / ngroups, g = fg - f * ngroups;
+  const int vb = P.view_off[f], nv = P.view_off[f + 1] - vb;
+  const int nz = min(NZ, P.N_z - g * kFwdZ);
+  const float4 *qg = reinterpret_cast<const float4 *>(q) + (size_t)g * P.N_p * P.N_r * (kFwdZ / 4);
+  float *ob = P.obj + ((size_t)f * P.N_z + g * kFwdZ) * Nxy;
+  const int pix = (blockIdx.x - fg * runs) * 256 + (int)threadIdx.x;
+  if (pix < Nxy) {
+    const int row = pix / P.N_x, col = pix - row * P.N_x;
+    double acc[NZ];
+#pragma unroll
+    for (int i = 0; i < NZ; i++) acc[i] = 0.0;
+    const bool in = P.mask[pix] && nv > 0;
+    if (in) {
       const double x = P.x0 + ((double)col + 0.5) * P.delta_xy;
       const double y = P.y0 + ((double)row + 0.5) * P.delta_xy;
-      double acc = 0.0;
+#pragma unroll 2
       for (int k = 0; k < nv; k++) {
         const int v = P.view_idx[vb + k];
-        const double u = (x * P.cosv[v] - y * P.sinv[v] - P.R0) / P.delta_r - 0.5;
-        const double j = floor(u);
-        const double t = u - j;
+        const double u = fma(fma(x, P.cosv[v], -(y * P.sinv[v])), P.u_inv, -P.u_r0) - 0.5;
+        const double j = floor(u), t = u - j;
         const int j0 = (int)j;
-        const float *qv = q + ((size_t)z * P.N_p + v) * P.N_r;
-        const double q0 = (j0 >= 0 && j0 < P.N_r) ? (double)qv[j0] : 0.0;
-        const double q1 = (j0 + 1 >= 0 && j0 + 1 < P.N_r) ? (double)qv[j0 + 1] : 0.0;
-        acc += (1.0 - t) * q0 + t * q1;
+        const float4 *qv = qg + (size_t)v * P.N_r * (kFwdZ / 4);
+        if (j0 >= 0 && j0 + 1 < P.N_r) {
+          const float4 *a = qv + j0 * (kFwdZ / 4), *b = a + kFwdZ / 4;
+#pragma unroll
+          for (int i = 0; i < NZ / 4; i++) {
+            const float4 qa = a[i], qb = b[i];
+            acc[4 * i] = fma(t, (double)qb.x, fma(1.0 - t, (double)qa.x, acc[4 * i]));
+            acc[4 * i + 1] = fma(t, (double)qb.y, fma(1.0 - t, (double)qa.y, acc[4 * i + 1]));
+            acc[4 * i + 2] = fma(t, (double)qb.z, fma(1.0 - t, (double)qa.z, acc[4 * i + 2]));
+            acc[4 * i + 3] = fma(t, (double)qb.w, fma(1.0 - t, (double)qa.w, acc[4 * i + 3]));
+          }
+        } else if (j0 == -1 || j0 == P.N_r - 1) {
+          // one of the two bins is off the detector
+          const float *a = reinterpret_cast<const float *>(qv + max(j0, 0) * (kFwdZ / 4));
+          const double w = j0 < 0 ? t : 1.0 - t;
+#pragma unroll
+          for (int i = 0; i < NZ; i++) acc[i] = fma(w, (double)a[i], acc[i]);
+        }
       }
-      out = (float)(acc * kPi / nv);
     }
-    P.obj[i] = out;
+#pragma unroll
+    for (int i = 0; i < NZ; i++)
+      if (i < nz) ob[(size_t)i * Nxy + pix] = in ? (float)(acc[i] * kPi / nv) : 0.0f;
   }
 }
+template __global__ void k_fbp_back<4>(KP, const float *);
+template __global__ void k_fbp_back<8>(KP, const float *);
 
 // ---------------------------------------------------------------------------
 // Voxel update: one workgroup per cell of one colour, voxels in sequence.
