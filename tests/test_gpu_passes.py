@@ -87,3 +87,23 @@ def test_prior_cost_keeps_infinities_and_nan():
     st.set_object(x)
     assert np.isnan(st.cost()[2])
     st.close()
+
+
+@pytest.mark.parametrize("N,nz,shift,mxy,mz", [(15, 1, 0.0, 1, 1), (18, 5, 1.25, 1, 1),
+                                               (20, 4, -4.0, 2, 2), (24, 12, 0.0, 1, 1),
+                                               (24, 8, 3.0, 4, 4)])
+def test_forward_projection_bitwise_at_the_edges(N, nz, shift, mxy, mz):
+    """Bit for bit the oracle's forward projection, as
+    test_forward_projection_bitwise asserts on a centred scan."""
+    from oracle import pyorc
+    print(f"forward N={N} nz={nz} shift={shift} mult={mxy},{mz}", flush=True)
+    scan = scan_of(N, nz, shift, n_views=34)
+    st = tb.Stage(scan, mult_xy=mxy, mult_z=mz)
+    o = pyorc.Problem(scan, mult_xy=mxy, mult_z=mz)
+    x = np.random.default_rng(6).random(st.obj_shape).astype(np.float32)
+    st.set_object(x)
+    o.obj()[...] = x
+    got = st.forward_project()
+    st.close()
+    np.testing.assert_array_equal(got, o.forward_project())
+    assert np.abs(got).max() > 0

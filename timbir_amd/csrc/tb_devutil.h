@@ -39,30 +39,6 @@ __device__ __forceinline__ void for_acol(const KP &P, const float *__restrict__ 
   }
 }
 
-// Value of bin `j` of the column above, or 0 when j is outside it.
-__device__ __forceinline__ double acol_bin(const KP &P, const float *__restrict__ H, double c,
-                                           double s, int row, int col, int j) {
-#pragma clang fp contract(off)
-  double x = P.x0 + ((double)col + 0.5) * P.delta_xy;
-  double y = P.y0 + ((double)row + 0.5) * P.delta_xy;
-  double r = x * c - y * s;
-  double rmin = r - P.delta_xy, rmax = r + P.delta_xy;
-  if (rmax < P.R0 || rmin > P.RMax) return 0.0;
-  int lo = (int)floor((rmin - P.R0) / P.delta_r);
-  int hi = (int)floor((rmax - P.R0) / P.delta_r);
-  if (hi >= P.N_r) hi = P.N_r - 1;
-  if (lo < 0) lo = 0;
-  if (j < lo || j > hi) return 0.0;
-  double centre = P.R0 + ((double)j + 0.5) * P.delta_r;
-  double dist = fabs(r - centre);
-  int bin = (int)floor(dist / P.OffsetR);
-  if (bin < 0 || bin >= kRespBins) return 0.0;
-  double w1 = dist - bin * P.OffsetR;
-  double w2 = P.OffsetR - w1;
-  double f1 = (w2 * (double)H[bin] + w1 * (double)H[bin + 1]) / P.OffsetR;
-  return f1 > 0 ? f1 : 0.0;
-}
-
 // ProjSelect b = |e sqrt(w)| < T evaluated as the reference does, in double
 // (XT_VoxUpdate.c:108-111); the float test decides all but a thin band.
 __device__ __forceinline__ bool selected(const KP &P, float e, float w) {

@@ -121,13 +121,30 @@ __global__ void k_upsample(const float *__restrict__ in, float *__restrict__ out
 // the result is bit-identical to the reference's.  The A entry depends only
 // on (view, pixel, bin): each is evaluated once and applied to the group's
 // slices, read as one 32-byte record from the slice-interleaved copy that
-// k_fwd_interleave writes.  Each thread visits only the rows and columns
-// whose centres project into reach of its bin, so the threads of a view do
-// similar work at every angle.  Every detector row of a slice receives the
+// k_fwd_interleave writes.  Every detector row of a slice receives the
 // same value.  mode 0: out = A x; mode 1: e = y - A x - d.  Blocks are
 // numbered view-major inside each XCD's share (block b runs on XCD b mod
 // 8), so one XCD's L2 holds the objects of few frames.
+//
+// Bound: FP64 arithmetic.  A column is nonzero at bin j only where the pixel's
+// centre projects within 64 OffsetR = delta_xy / sqrt(2) + delta_r / 2 of the
+// bin's centre, and there calcAMatrixColumnforAngle's other limits (first and
+// last bin, the detector's ends) hold by 0.29 delta_xy, so a thread visits
+// only the columns of a row inside that reach (widened by 1e-6 of a pixel) and
+// evaluates neither those limits nor their two divisions.  The two divisions
+// by OffsetR that remain take fwd_div.  Before, with a candidate span a third
+// wider plus two cells, two divisions per row and four per candidate, 384 x
+// 384 x 12 slices x 6 frames and 720 views took 6.5 ms, in this form 2.3.
 // ---------------------------------------------------------------------------
+
+// a / b correctly rounded, y = 1 / b correctly rounded: two residual steps
+// make the quotient faithful and then exact (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", 1990)
+__device__ __forceinline__ double fwd_div(double a, double b, double y) {
+  double q = a * y;
+  q = fma(fma(-b, q, a), y, q);
+  return fma(fma(-b, q, a), y, q);
+}
 
 // objt[f][g][row][col][q] = obj[f][g * kFwdZ + q][row][col], zero past N_z
 __global__ void k_fwd_interleave(KP P, float4 *__restrict__ objt) {
@@ -163,10 +180,70 @@ __device__ __forceinline__ void fwd_span(double lo, double hi, double g, double 
   k1 = min(n - 1, (int)ceil(kb) + 1);
 }
 
+template <int NZ>
+__device__ __forceinline__ void forward_bin(const KP &P, const float *s_H, const float4 *ob, int v,
+                                            int r, float (&out)[kFwdZ]) {
+#pragma clang fp contract(off)
+  const double c = P.cosv[v], s = P.sinv[v];
+  const double OR = P.OffsetR, yOR = 1.0 / OR;
+  const double centre = P.R0 + ((double)r + 0.5) * P.delta_r;
+  const double reach = kRespBins * OR + 1e-6 * P.delta_xy;
+  float acc[NZ];
+#pragma unroll
+  for (int q = 0; q < NZ; q++) acc[q] = 0.0f;
+  int y_first = 0, y_last = P.N_y - 1;
+  if (fabs(s) > 1e-6) {
+    // y s in (x c - centre - reach, x c - centre + reach) for some column
+    const double xa = (P.x0 + 0.5 * P.delta_xy) * c;
+    const double xb = (P.x0 + (P.N_x - 0.5) * P.delta_xy) * c;
+    fwd_span(fmin(xa, xb) - centre - reach, fmax(xa, xb) - centre + reach, s, P.y0, P.delta_xy,
+             P.N_y, y_first, y_last);
+  }
+  // columns of a row: |k - ((centre + y s) ic - k_off)| < hw
+  const bool wide = fabs(c) > 1e-6;
+  const double ic = wide ? 1.0 / (c * P.delta_xy) : 0.0;
+  const double k_off = P.x0 / P.delta_xy + 0.5;
+  const double hw = reach * fabs(ic) + 1e-6;
+  const double k_max = (double)P.N_x;
+  for (int row = y_first; row <= y_last; row++) {
+    const double y = P.y0 + ((double)row + 0.5) * P.delta_xy;
+    const double ys = y * s;
+    int k0 = 0, k1 = P.N_x - 1;
+    if (wide) {
+      const double kc = fma(centre + ys, ic, -k_off);
+      k0 = (int)fmin(fmax(ceil(kc - hw), 0.0), k_max);
+      k1 = (int)fmin(fmax(floor(kc + hw), -1.0), k_max - 1.0);
+    }
+    for (int col = k0; col <= k1; col++) {
+      const float4 *px = ob + ((size_t)row * P.N_x + col) * (kFwdZ / 4);
+      float pv[NZ];
+#pragma unroll
+      for (int q = 0; q < NZ / 4; q++) {
+        const float4 p = px[q];
+        pv[4 * q] = p.x, pv[4 * q + 1] = p.y, pv[4 * q + 2] = p.z, pv[4 * q + 3] = p.w;
+      }
+      // calcAMatrixColumnforAngle's value (XT_AMatrix.c:50-110)
+      const double x = P.x0 + ((double)col + 0.5) * P.delta_xy;
+      const double dist = fabs((x * c - ys) - centre);
+      const int bin = (int)fwd_div(dist, OR, yOR);
+      if (bin < kRespBins) {
+        const double w1 = dist - bin * OR;
+        const double w2 = OR - w1;
+        const double a = fwd_div(w2 * (double)s_H[bin] + w1 * (double)s_H[bin + 1], OR, yOR);
+        if (a > 0.0) {
+#pragma unroll
+          for (int q = 0; q < NZ; q++) acc[q] = (float)((double)acc[q] + (double)pv[q] * a);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NZ; q++) out[q] = acc[q];
+}
+
 __global__ __launch_bounds__(kFwdT) void k_forward(KP P, const int *__restrict__ view_frame,
                                                    const float4 *__restrict__ objt,
                                                    float *__restrict__ out, int mode) {
-#pragma clang fp contract(off)
   __shared__ float s_H[kHrStride];
   const int ntile = (P.N_r + kFwdT - 1) / kFwdT;
   const int nb = ntile * P.N_p;
@@ -187,35 +264,9 @@ __global__ __launch_bounds__(kFwdT) void k_forward(KP P, const int *__restrict__
     __syncthreads();
   }
   if (f >= 0 && r < P.N_r) {
-    const double c = P.cosv[v], s = P.sinv[v];
-    const float4 *ob = objt + (size_t)(f * ngroups + g) * P.N_x * P.N_y * 2;
-    // voxels whose projected centre x c - y s lies in [lo, hi) can cover bin r
-    const double lo = P.R0 + r * P.delta_r - P.delta_xy - 1e-9;
-    const double hi = P.R0 + (r + 1) * P.delta_r + P.delta_xy + 1e-9;
-    int y_first = 0, y_last = P.N_y - 1;
-    if (fabs(s) > 1e-6) {
-      // y s in (x c - hi, x c - lo] for some column centre x
-      const double xa = (P.x0 + 0.5 * P.delta_xy) * c;
-      const double xb = (P.x0 + (P.N_x - 0.5) * P.delta_xy) * c;
-      fwd_span(fmin(xa, xb) - hi, fmax(xa, xb) - lo, s, P.y0, P.delta_xy, P.N_y, y_first,
-               y_last);
-    }
-    for (int row = y_first; row <= y_last; row++) {
-      const double y = P.y0 + ((double)row + 0.5) * P.delta_xy;
-      int k0 = 0, k1 = P.N_x - 1;
-      // x c in [lo + y s, hi + y s)
-      if (fabs(c) > 1e-6) fwd_span(lo + y * s, hi + y * s, c, P.x0, P.delta_xy, P.N_x, k0, k1);
-      for (int col = k0; col <= k1; col++) {
-        const float4 *px = ob + ((size_t)row * P.N_x + col) * 2;
-        const float4 p0 = px[0], p1 = px[1];
-        const double a = acol_bin(P, s_H, c, s, row, col, r);
-        if (a != 0.0) {
-          const float pv[kFwdZ] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
-#pragma unroll
-          for (int q = 0; q < kFwdZ; q++) acc[q] = (float)((double)acc[q] + (double)pv[q] * a);
-        }
-      }
-    }
+    const float4 *ob = objt + (size_t)(f * ngroups + g) * P.N_x * P.N_y * (kFwdZ / 4);
+    if (nz > 4) forward_bin<kFwdZ>(P, s_H, ob, v, r, acc);
+    else forward_bin<4>(P, s_H, ob, v, r, acc);
   }
   if (r >= P.N_r) return;
 #pragma unroll
