@@ -1,0 +1,79 @@
+"""The learned initialiser's kernels at the sizes where their tiles end: the
+staged convolution (strips of 64 x 1 and 32 x 2 voxels, rows and columns past
+the volume, every channel split), the convolution of an upsampled and
+concatenated input, the weight gradient (tiles, runs of planes, more units than
+slices), and the elementwise kernels' scalar forms (channels and addresses that
+16-byte accesses do not allow)."""
+import ctypes as C
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import unet_ref as U
+from timbir_amd.devmem import DevArray
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+from test_gpu_unet import bf, dev, empty, host, log, ptr  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def L():
+    from timbir_amd import learned
+    return learned.nn_lib()
+
+
+def at(t, elems, size):
+    """The address `elems` elements of `size` bytes into t."""
+    return C.c_void_p(t.addr + elems * size)
+
+
+@pytest.mark.parametrize("shape,cin,cout", [
+    ((1, 1, 1, 1), 32, 32), ((1, 2, 9, 65), 32, 32), ((1, 3, 8, 64), 32, 96), ((2, 1, 5, 63), 64, 64),
+    ((1, 2, 7, 33), 64, 32), ((1, 3, 4, 31), 96, 32), ((1, 2, 9, 40), 96, 64), ((1, 2, 5, 64), 128, 64),
+    ((1, 2, 3, 20), 128, 128), ((1, 2, 10, 34), 192, 64), ((1, 1, 4, 66), 192, 192),
+    ((1, 2, 3, 17), 160, 32)])   # 160: the kernel without LDS
+def test_conv3d_tiles(L, shape, cin, cout):
+    """fp32 output within 5e-5 of the largest value of the float64 result of
+    the same bf16 operands (up to 27 x 192 fp32 products summed), as
+    test_conv3d_matches_oracle; with bias and ReLU, and stored at an address
+    that is not 16-byte aligned."""
+    log(f"conv tile {shape} {cin}->{cout}")
+    rng = np.random.default_rng(cin * 7 + cout)
+    x = U.bf16(rng.standard_normal(shape + (cin,)).astype(np.float32))
+    w = U.bf16((rng.standard_normal((27, cout, cin)) / np.sqrt(27 * cin)).astype(np.float32))
+    b = rng.standard_normal(cout).astype(np.float32)
+    xt, wt, bt, y = bf(x), bf(w), dev(b), empty((int(np.prod(shape)) * cout + 4,))
+    ref = np.maximum(U.conv3d(x.astype(np.float64), w.astype(np.float64), b), 0)
+    for off in (0, 1):
+        assert L.tb_nn_conv3d(ptr(xt), ptr(wt), ptr(bt), at(y, off, 4), *shape, cin, cout, 1, 1,
+                              None) == 0
+        got = host(y)[off:off + ref.size].reshape(ref.shape)
+        assert np.abs(got - ref).max() <= 5e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("shape,ca,cb,cout", [((1, 2, 2, 2), 64, 32, 32), ((2, 4, 10, 66), 64, 32, 32),
+                                              ((1, 2, 8, 34), 64, 32, 64), ((1, 4, 6, 62), 128, 64, 64),
+                                              ((1, 2, 18, 32), 128, 64, 96)])
+def test_conv3d_up2cat_is_the_two_calls(L, shape, ca, cb, cout):
+    """Bit for bit the upsampling and concatenation followed by the
+    convolution; other channel counts are refused."""
+    log(f"conv up2cat {shape} {ca}+{cb}->{cout}")
+    rng = np.random.default_rng(ca + cout)
+    n, d, h, w_ = shape
+    a = bf(rng.standard_normal((n, d // 2, h // 2, w_ // 2, ca)))
+    b = bf(rng.standard_normal(shape + (cb,)))
+    w = bf(rng.standard_normal((27, cout, ca + cb)) / 30)
+    bias = dev(rng.standard_normal(cout))
+    cat, y1, y2 = (empty(shape + (c,), "bf16") for c in (ca + cb, cout, cout))
+    assert L.tb_nn_up2_concat(ptr(a), ptr(b), ptr(cat), *shape, ca, cb, None) == 0
+    assert L.tb_nn_conv3d(ptr(cat), ptr(w), ptr(bias), ptr(y1), *shape, ca + cb, cout, 1, 0, None) == 0
+    assert L.tb_nn_conv3d_up2cat(ptr(a), ptr(b), ptr(w), ptr(bias), ptr(y2), *shape, ca, cb, cout, 1,
+                                 None) == 0
+    assert np.abs(host(y1)).max() > 0
+    np.testing.assert_array_equal(host(y1), host(y2))
+    assert L.tb_nn_conv3d_up2cat(ptr(a), ptr(b), ptr(w), ptr(bias), ptr(y2), *shape, 32, 32, cout, 1,
+                                 None) == -1

@@ -32,7 +32,7 @@ EXPORTS = [
     "tb_autotune", "tb_autotune_entries", "tb_autotune_put", "tb_autotune_clear",
     # learned initialiser kernels (tb_unet.hip)
     "tb_nn_last_error", "tb_dev_malloc", "tb_dev_free", "tb_dev_copy", "tb_dev_zero",
-    "tb_dev_synchronize", "tb_nn_conv3d", "tb_nn_conv3d_flip", "tb_nn_conv3d_wgrad",
+    "tb_dev_synchronize", "tb_nn_conv3d", "tb_nn_conv3d_up2cat", "tb_nn_conv3d_flip", "tb_nn_conv3d_wgrad",
     "tb_nn_channel_sum", "tb_nn_relu_bwd", "tb_nn_avgpool2", "tb_nn_up2_concat",
     "tb_nn_up2_concat_bwd", "tb_nn_add", "tb_nn_make_input", "tb_nn_frame_mean", "tb_nn_head", "tb_nn_head_bwd",
     "tb_nn_mse", "tb_nn_sum_parts", "tb_nn_adam", "tb_nn_to_bf16",

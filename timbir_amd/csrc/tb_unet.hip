@@ -124,6 +124,191 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
   }
 }
 
+// The same convolution with the input staged in LDS.  The input's channels are
+// 32 CA of a tensor at half size, nearest x2 upsampled (`ina`, CA may be 0),
+// then 32 CB of one at full size (`in`): the concatenation of a U-Net's skip
+// connection need not exist in memory.  Tile: 64 SP voxels per wave as strips
+// of WT x (64 / WT), 4 waves side by side in h, 16 NB output channels.  One
+// input plane (dz) at a time is staged with its halo, in the order of the taps,
+// and each of its values serves 9 taps from LDS; without it every tap read
+// every value through the L1 (192 B a cycle wanted, 64 there).
+//   Weights are the A operand (M = output channel; row m of fragment b is
+// channel (m / 4) 4 NB + 4 b + m % 4, so a lane ends with 4 NB consecutive
+// channels of a voxel and stores them whole), activations the B operand (N =
+// voxel).  Fragment a holds the voxels x = 4 q + a, so the three x taps of four
+// fragments are six reads instead of twelve, and four of the half-size tensor
+// (a voxel's parent is x / 2); LDS keeps x modulo 4 (parents modulo 2) apart,
+// which makes each read one contiguous KB.
+//   The sums run over (tap, channel chunk) as in k_conv3d_fwd, one MFMA each:
+// the bits are the same.  2 x 16 x 256 x 256 voxels, before and now: 32 -> 32
+// channels 0.38 and 0.18 ms (650 TFLOP/s); 64 + 32 -> 32 with its
+// concatenation 1.6 and 0.46 ms (750 TFLOP/s).
+template <int CA, int CB, int SP, int WT>
+struct ConvTile {
+  static constexpr int RPS = 64 / WT, HT = 4 * SP * RPS;
+  static constexpr int HR = HT + 2, QW = WT / 4 + 1;  // full size: s[CB][HR][4][QW][32]
+  static constexpr int HC = HT / 2 + 2;               // half size: s[CA][HC][2][QW][32]
+  static constexpr int kFull = CB * HR * 4 * QW * 32, kHalf = CA * HC * 2 * QW * 32;
+  static constexpr size_t kBytes = (size_t)(kFull + kHalf) * sizeof(bf16);
+};
+
+template <int CA, int CB, int NB, int SP, int WT>
+__global__ __launch_bounds__(256) void k_conv3d_tile(
+    const bf16 *__restrict__ ina, const bf16 *__restrict__ in, const bf16 *__restrict__ w,
+    const float *__restrict__ bias, void *__restrict__ out, int N, int D, int H, int W, int Cout,
+    int relu, int out_f32) {
+  using T = ConvTile<CA, CB, SP, WT>;
+  constexpr int C = CA + CB, Cin = 32 * C, RPS = T::RPS, HT = T::HT, HR = T::HR, HC = T::HC,
+                QW = T::QW;
+  constexpr bool HOLD = C <= 3;  // a row's fragments of every chunk fit the registers
+  extern __shared__ bf16 s_in[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane & 15, kq = lane >> 4;
+  const int WB = (W + WT - 1) / WT, HB = (H + HT - 1) / HT, CT = Cout / (16 * NB);
+  // neighbouring tiles on one XCD (block b runs on XCD b mod 8): they share halos
+  unsigned g = blockIdx.x;
+  if ((gridDim.x & 7) == 0) g = (g & 7) * (gridDim.x >> 3) + (g >> 3);
+  const int ct = g % CT; g /= CT;
+  const int w0 = (int)(g % WB) * WT; g /= WB;
+  const int h0 = (int)(g % HB) * HT; g /= HB;
+  const int d = g % D, n = g / D;
+  const int co0 = ct * 16 * NB;
+  const int xq = row % (WT / 4), yr = row / (WT / 4);
+  f32x4 acc[SP][4][NB];
+#pragma unroll
+  for (int s = 0; s < SP; s++)
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+      for (int b = 0; b < NB; b++) acc[s][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16 *wl = w + (size_t)(co0 + (row >> 2) * 4 * NB + (row & 3)) * Cin + kq * 8;
+  int held = -1;  // the half-size plane in LDS
+  for (int dz = 0; dz < 3; dz++) {
+    const int zz = d + dz - 1;
+    if (zz < 0 || zz >= D) continue;
+    __syncthreads();
+    if constexpr (CB > 0) {
+      const bf16 *plane = in + ((size_t)n * D + zz) * H * W * (32 * CB);
+#pragma unroll 4
+      for (int i = threadIdx.x; i < HR * (WT + 2) * 4 * CB; i += 256) {
+        const int part = i % (4 * CB), vox = i / (4 * CB), xi = vox % (WT + 2), y = vox / (WT + 2);
+        const int yy = h0 + y - 1, xx = w0 + xi - 1;
+        bf16x8 v = zero8();
+        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
+          v = *reinterpret_cast<const bf16x8 *>(plane + ((size_t)yy * W + xx) * (32 * CB) + part * 8);
+        *reinterpret_cast<bf16x8 *>(
+            s_in + ((((part >> 2) * HR + y) * 4 + (xi & 3)) * QW + (xi >> 2)) * 32 + (part & 3) * 8) =
+            v;
+      }
+    }
+    if constexpr (CA > 0) {
+      const int H2 = H / 2, W2 = W / 2;
+      if (held != (zz >> 1)) {
+        held = zz >> 1;
+        const bf16 *plane = ina + ((size_t)n * (D / 2) + held) * H2 * W2 * (32 * CA);
+#pragma unroll 4
+        for (int i = threadIdx.x; i < HC * (WT / 2 + 2) * 4 * CA; i += 256) {
+          const int part = i % (4 * CA), vox = i / (4 * CA);
+          const int xi = vox % (WT / 2 + 2), y = vox / (WT / 2 + 2);
+          const int yy = h0 / 2 + y - 1, xx = w0 / 2 + xi - 1;
+          bf16x8 v = zero8();
+          if (yy >= 0 && yy < H2 && xx >= 0 && xx < W2)
+            v = *reinterpret_cast<const bf16x8 *>(plane + ((size_t)yy * W2 + xx) * (32 * CA) +
+                                                  part * 8);
+          *reinterpret_cast<bf16x8 *>(s_in + T::kFull +
+                                      ((((part >> 2) * HC + y) * 2 + (xi & 1)) * QW + (xi >> 1)) * 32 +
+                                      (part & 3) * 8) = v;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int dy = 0; dy < 3; dy++) {
+      const bf16 *wt = wl + (size_t)(dz * 9 + dy * 3) * Cout * Cin;
+      // voxels 4 q + t - 1 of chunk c, t = 0 .. 5; of the half-size tensor
+      // their parents 2 q + u - 1, u = (t + 1) / 2
+      auto frag = [&](int s, int c, int t) -> bf16x8 {
+        const int y = (wave * SP + s) * RPS + yr + dy;
+        const bf16 *p;
+        if (c < CA) {
+          const int u = (t + 1) >> 1;
+          p = s_in + T::kFull + (((c * HC + ((y + 1) >> 1)) * 2 + (u & 1)) * QW + xq + (u >> 1)) * 32;
+        } else {
+          p = s_in + ((((c - CA) * HR + y) * 4 + (t & 3)) * QW + xq + (t >> 2)) * 32;
+        }
+        return *reinterpret_cast<const bf16x8 *>(p + kq * 8);
+      };
+      bf16x8 fr[SP][HOLD ? C : 1][6];
+      if constexpr (HOLD) {
+#pragma unroll
+        for (int s = 0; s < SP; s++)
+#pragma unroll
+          for (int c = 0; c < C; c++)
+#pragma unroll
+            for (int t = 0; t < 6; t++)
+              fr[s][c][t] = c < CA && t > 0 && (t & 1) == 0 ? fr[s][c][t - 1] : frag(s, c, t);
+      }
+#pragma unroll
+      for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+        for (int c = 0; c < C; c++) {
+          bf16x8 wv[NB];
+#pragma unroll
+          for (int b = 0; b < NB; b++)
+            wv[b] = *reinterpret_cast<const bf16x8 *>(wt + (size_t)dx * Cout * Cin +
+                                                      (size_t)b * 4 * Cin + c * 32);
+#pragma unroll
+          for (int s = 0; s < SP; s++) {
+            bf16x8 x[4];
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+              x[a] = HOLD ? fr[s][HOLD ? c : 0][a + dx]
+                     : c < CA && a > 0 && ((a + dx) & 1) == 0 ? x[a - 1]
+                                                              : frag(s, c, a + dx);
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+              for (int b = 0; b < NB; b++) acc[s][a][b] = mfma(wv[b], x[a], acc[s][a][b]);
+          }
+        }
+    }
+  }
+  // lane: channels co .. co + 4 NB - 1 of voxel x = w0 + 4 xq + a
+  const int co = co0 + kq * 4 * NB;
+  float bb[4 * NB];
+#pragma unroll
+  for (int k = 0; k < 4 * NB; k++) bb[k] = bias ? bias[co + k] : 0.f;
+#pragma unroll
+  for (int s = 0; s < SP; s++) {
+    const int h = h0 + (wave * SP + s) * RPS + yr;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      const int x = w0 + 4 * xq + a;
+      if (h >= H || x >= W) continue;
+      const size_t o = ((((size_t)n * D + d) * H + h) * W + x) * Cout + co;
+#pragma unroll
+      for (int b = 0; b < NB; b += 2) {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          v[k] = acc[s][a][b + k / 4][k % 4] + bb[4 * b + k];
+          if (relu) v[k] = fmaxf(v[k], 0.f);
+        }
+        if (out_f32) {
+          float4 *p = reinterpret_cast<float4 *>(static_cast<float *>(out) + o + 4 * b);
+          p[0] = make_float4(v[0], v[1], v[2], v[3]);
+          p[1] = make_float4(v[4], v[5], v[6], v[7]);
+        } else {
+          bf16x8 q;
+#pragma unroll
+          for (int k = 0; k < 8; k++) q[k] = (bf16)v[k];
+          *reinterpret_cast<bf16x8 *>(static_cast<bf16 *>(out) + o + 4 * b) = q;
+        }
+      }
+    }
+  }
+}
+
 // wt[t][ci][co] = w[26 - t][co][ci]: the weights of the gradient with respect
 // to the input, which is the forward convolution of the output gradient with
 // the spatially flipped, transposed kernel
@@ -528,12 +713,60 @@ extern "C" int tb_dev_synchronize(void) {
   return 0;
 }
 
+// The staged kernel's launch.  Output channels: 96 at once, else 64, else 32.
+// Strips of 64 x 1 voxels, or 32 x 2 where that leaves fewer lanes without a
+// voxel (and for 128 + 64 input channels, whose tile of 64 leaves one workgroup
+// per CU).  Two strips per wave for 32 output channels of 32 inputs, where the
+// weights' share of the L1 would otherwise bound.
+template <int CA, int CB, int NB, int SP, int WT>
+static int conv_tile(const void *a, const void *in, const void *w, const float *bias, void *out,
+                     int n, int d, int h, int wd, int cout, int relu, int out_f32, hipStream_t s) {
+  using T = ConvTile<CA, CB, SP, WT>;
+  auto fn = k_conv3d_tile<CA, CB, NB, SP, WT>;
+  const long long blocks = (long long)n * d * ((h + T::HT - 1) / T::HT) * ((wd + WT - 1) / WT) *
+                           (cout / (16 * NB));
+  if (blocks > 0x7fffffffLL) return nn_fail("tb_nn_conv3d: volume too large");
+  if (T::kBytes > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::kBytes);
+    if (e != hipSuccess) return nn_fail("tb_nn_conv3d", e);
+  }
+  hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), T::kBytes, s,
+                     static_cast<const bf16 *>(a), static_cast<const bf16 *>(in),
+                     static_cast<const bf16 *>(w), bias, out, n, d, h, wd, cout, relu, out_f32);
+  NNCHK("tb_nn_conv3d");
+  return 0;
+}
+
+using conv_fn = int (*)(const void *, const void *, const void *, const float *, void *, int, int,
+                        int, int, int, int, int, hipStream_t);
+template <int CA, int CB, int NB, int SP>
+static conv_fn conv_pick(int wd) {
+  const int a64 = (wd + 63) / 64 * 64, a32 = (wd + 31) / 32 * 32;
+  return a32 < a64 || CA == 4 ? conv_tile<CA, CB, NB, SP, 32> : conv_tile<CA, CB, NB, SP, 64>;
+}
+template <int CA, int CB>
+static conv_fn conv_pick(int cout, int wd) {
+  if (cout % 96 == 0) return conv_pick<CA, CB, 6, 1>(wd);
+  if (cout % 64 == 0) return conv_pick<CA, CB, 4, 1>(wd);
+  return conv_pick<CA, CB, 2, CA == 0 && CB == 1 ? 2 : 1>(wd);
+}
+
 extern "C" int tb_nn_conv3d(const void *in, const void *w, const float *bias, void *out,
                             int32_t n, int32_t d, int32_t h, int32_t wd, int32_t cin,
                             int32_t cout, int32_t relu, int32_t out_f32, void *stream) {
   if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || cin % 32 || cout % 32 || cin <= 0 || cout <= 0)
     return nn_fail("tb_nn_conv3d: sizes must be positive, channels multiples of 32");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  conv_fn fn = cin == 32    ? conv_pick<0, 1>(cout, wd)
+               : cin == 64  ? conv_pick<0, 2>(cout, wd)
+               : cin == 96  ? conv_pick<0, 3>(cout, wd)
+               : cin == 128 ? conv_pick<0, 4>(cout, wd)
+               : cin == 192 ? conv_pick<0, 6>(cout, wd)
+                            : nullptr;
+  // the staged kernel stores 16 bytes at a time
+  if (fn && reinterpret_cast<uintptr_t>(out) % 16 == 0)
+    return fn(nullptr, in, w, bias, out, n, d, h, wd, cout, relu, out_f32, s);
   const int MB = 4, NB = 2;
   const long long waves = (long long)n * d * h * ((wd + 16 * MB - 1) / (16 * MB)) * (cout / (16 * NB));
   const long long blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
@@ -543,6 +776,21 @@ extern "C" int tb_nn_conv3d(const void *in, const void *w, const float *bias, vo
                      d, h, wd, cin, cout, relu, out_f32);
   NNCHK("tb_nn_conv3d");
   return 0;
+}
+
+extern "C" int tb_nn_conv3d_up2cat(const void *a, const void *b, const void *w, const float *bias,
+                                   void *out, int32_t n, int32_t d, int32_t h, int32_t wd,
+                                   int32_t ca, int32_t cb, int32_t cout, int32_t relu,
+                                   void *stream) {
+  if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || d % 2 || h % 2 || wd % 2 || cout <= 0 || cout % 32)
+    return nn_fail("tb_nn_conv3d_up2cat: sizes must be positive and even, channels multiples of 32");
+  conv_fn fn = ca == 64 && cb == 32    ? conv_pick<2, 1>(cout, wd)
+               : ca == 128 && cb == 64 ? conv_pick<4, 2>(cout, wd)
+                                       : nullptr;
+  if (!fn) return nn_fail("tb_nn_conv3d_up2cat: 64 + 32 or 128 + 64 input channels");
+  if (reinterpret_cast<uintptr_t>(out) % 16)
+    return nn_fail("tb_nn_conv3d_up2cat: the output must be 16-byte aligned");
+  return fn(a, b, w, bias, out, n, d, h, wd, cout, relu, 0, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tb_nn_conv3d_flip(const void *w, void *wt, int32_t cin, int32_t cout,

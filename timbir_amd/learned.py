@@ -52,6 +52,7 @@ def nn_lib():
     vp, i32, i64, f32 = C.c_void_p, C.c_int32, C.c_int64, C.c_float
     sig = {
         "tb_nn_conv3d": [vp, vp, vp, vp] + [i32] * 8 + [vp],
+        "tb_nn_conv3d_up2cat": [vp] * 5 + [i32] * 8 + [vp],
         "tb_nn_conv3d_flip": [vp, vp, i32, i32, vp],
         "tb_nn_conv3d_wgrad": [vp, vp, vp, vp] + [i32] * 7 + [vp],
         "tb_nn_channel_sum": [vp, vp, vp, i32, i64, i32, vp],
@@ -160,6 +161,16 @@ class UNet:
                 ta, _ = acts[a]
                 tb_, shp = acts[b]
                 ca, cb = ta.shape[-1], tb_.shape[-1]
+                if not keep:
+                    # nothing else reads the concatenation: it stays unwritten
+                    y = DevArray(shp + (cout,), "bf16")
+                    _ok(L.tb_nn_conv3d_up2cat(_p(ta), _p(tb_), _p(self.wbf[name]),
+                                              _p(self.master[(name, "b")]), _p(y), *shp, ca, cb,
+                                              cout, 1, s))
+                    acts[name] = (y, shp)
+                    for k in [k for k in acts if k not in _LIVE[name]]:
+                        del acts[k]
+                    continue
                 xin = DevArray(shp + (ca + cb,), "bf16")
                 _ok(L.tb_nn_up2_concat(_p(ta), _p(tb_), _p(xin), *shp, ca, cb, s))
                 acts[src] = (xin, shp)
