@@ -77,3 +77,89 @@ def test_conv3d_up2cat_is_the_two_calls(L, shape, ca, cb, cout):
     np.testing.assert_array_equal(host(y1), host(y2))
     assert L.tb_nn_conv3d_up2cat(ptr(a), ptr(b), ptr(w), ptr(bias), ptr(y2), *shape, 32, 32, cout, 1,
                                  None) == -1
+
+
+@pytest.mark.parametrize("c,off", [(32, 0), (32, 1), (96, 0), (5, 0)])
+def test_elementwise_forms_agree(L, c, off):
+    """Pooling, upsampling, their backward passes, ReLU and the sum of two
+    gradients in numpy on the same bf16 values, bit for bit; channel sums
+    within 1e-5 of the sum of magnitudes (fp32 sums of a few hundred)."""
+    log(f"elementwise c={c} offset {off}")
+    rng = np.random.default_rng(c)
+    shape = (2, 2, 4, 6)
+    n, d, h, w = shape
+    cell = (n, d // 2, h // 2, w // 2)
+    x = U.bf16(rng.standard_normal(shape + (c,)).astype(np.float32))
+    a = U.bf16(rng.standard_normal(cell + (c,)).astype(np.float32))
+
+    def put(v):
+        return bf(np.concatenate([np.zeros(off, np.float32), np.asarray(v, np.float32).ravel()]))
+
+    def get(t, shp):
+        return host(t)[off:].reshape(shp)
+
+    def new(shp):
+        return empty((int(np.prod(shp)) + off,), "bf16")
+
+    def p(t):
+        return at(t, off, 2)
+
+    X, A = put(x), put(a)
+    o = new(cell + (c,))
+    assert L.tb_nn_avgpool2(p(X), p(o), *shape, c, 0, None) == 0
+    s = np.zeros(cell + (c,), np.float32)
+    for k in range(8):
+        s = s + x[:, k >> 2::2, (k >> 1 & 1)::2, (k & 1)::2]
+    np.testing.assert_array_equal(get(o, cell + (c,)), U.bf16(s * np.float32(0.125)))
+    o = new(shape + (c,))
+    assert L.tb_nn_avgpool2(p(A), p(o), *shape, c, 1, None) == 0
+    np.testing.assert_array_equal(get(o, shape + (c,)), U.bf16(U.up2(a) * np.float32(0.125)))
+    o = new(shape + (2 * c,))
+    assert L.tb_nn_up2_concat(p(A), p(X), p(o), *shape, c, c, None) == 0
+    np.testing.assert_array_equal(get(o, shape + (2 * c,)), np.concatenate([U.up2(a), x], -1))
+    ga, gb = new(cell + (c,)), new(shape + (c,))
+    cat = put(np.concatenate([x, U.up2(a)], -1))
+    assert L.tb_nn_up2_concat_bwd(p(cat), p(ga), p(gb), *shape, c, c, None) == 0
+    np.testing.assert_array_equal(get(ga, cell + (c,)), U.bf16(s))
+    np.testing.assert_array_equal(get(gb, shape + (c,)), U.up2(a))
+    y = put(-x)
+    assert L.tb_nn_relu_bwd(p(X), p(y), x.size, None) == 0
+    np.testing.assert_array_equal(get(y, x.shape), np.where(x > 0, -x, 0))
+    z = put(U.up2(a))
+    assert L.tb_nn_add(p(z), p(X), x.size, None) == 0
+    np.testing.assert_array_equal(get(z, x.shape), U.bf16(U.up2(a) + x))
+    for slices in (1, 7):
+        out, part = empty((c,)), empty((slices * c,))
+        nv = x.size // c
+        assert L.tb_nn_channel_sum(p(X), ptr(out), ptr(part), slices, nv, c, None) == 0
+        ref = x.reshape(nv, c).astype(np.float64)
+        assert (np.abs(host(out) - ref.sum(0)) <= 1e-5 * np.abs(ref).sum(0)).all()
+
+
+@pytest.mark.parametrize("c", [32, 64, 12])
+def test_head_backward_and_network_input(L, c):
+    """The head's gradients against numpy (the bf16 gradient bit for bit,
+    the sums within 1e-5 of the sum of magnitudes), and the network input's
+    channels for a mean shared by all samples."""
+    log(f"head c={c}")
+    rng = np.random.default_rng(c)
+    nv, slices, scale = 333, 5, 50.0
+    h = U.bf16(rng.standard_normal((nv, c)).astype(np.float32))
+    w, g = (rng.standard_normal(k).astype(np.float32) for k in (c, nv))
+    ht, wt, gt = bf(h), dev(w), dev(g)
+    gh, part, hb = empty((nv, c), "bf16"), empty((slices, c + 1)), empty((c + 1,))
+    assert L.tb_nn_head_bwd(ptr(ht), ptr(wt), ptr(gt), ptr(gh), ptr(part), slices, nv, c, scale,
+                            None) == 0
+    assert L.tb_nn_sum_parts(ptr(part), ptr(hb), c + 1, slices, None) == 0
+    gs = (g * np.float32(1 / np.float32(scale))).astype(np.float32)
+    np.testing.assert_array_equal(host(gh), U.bf16(gs[:, None] * w[None]))
+    terms = np.concatenate([h, np.ones((nv, 1))], 1).astype(np.float64) * gs[:, None]
+    assert (np.abs(host(hb) - terms.sum(0)) <= 1e-5 * np.abs(terms).sum(0)).all()
+    per, v = 37, rng.standard_normal(3 * 37).astype(np.float32)
+    m = rng.standard_normal(per).astype(np.float32)
+    x = empty((v.size, 32), "bf16")
+    assert L.tb_nn_make_input(ptr(dev(v)), ptr(dev(m)), ptr(x), v.size, per, scale, None) == 0
+    want = np.zeros((v.size, 32), np.float32)
+    want[:, 0] = U.bf16(v * np.float32(scale))
+    want[:, 1] = U.bf16(np.tile(m, 3) * np.float32(scale))
+    np.testing.assert_array_equal(host(x), want)

@@ -395,130 +395,238 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_wgrad(
         dst[(size_t)(co0 + 16 * a + 4 * kq + j) * Cin + ci0 + 16 * b + row] = acc[a][b][j];
 }
 
-// out[i] = sum_s part[s][i], s in order
-__global__ void k_sum_parts(const float *__restrict__ part, float *__restrict__ out, size_t n,
-                            int S) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
+// out[i] = sum_s part[s][i]: 16 runs of slices side by side, each in order,
+// then the runs in order.  Block: 64 entries.  (One thread per entry walked the
+// slices one load at a time: 68 us on average over a training step's sums, 15
+// in this form.)
+constexpr int kSumRuns = 16;
+__global__ __launch_bounds__(64 * kSumRuns) void k_sum_parts(const float *__restrict__ part,
+                                                             float *__restrict__ out, size_t n,
+                                                             int S) {
+  __shared__ float sh[kSumRuns][64];
+  const int col = threadIdx.x & 63, run = threadIdx.x >> 6;
+  const int per = (S + kSumRuns - 1) / kSumRuns;
+  const int s0 = min(run * per, S), s1 = min(s0 + per, S);
+  for (size_t i0 = blockIdx.x * (size_t)64; i0 < n; i0 += (size_t)gridDim.x * 64) {
+    const size_t i = i0 + col;
     float acc = 0.f;
-    for (int s = 0; s < S; s++) acc += part[(size_t)s * n + i];
-    out[i] = acc;
+    if (i < n) {
+#pragma unroll 8
+      for (int s = s0; s < s1; s++) acc += part[(size_t)s * n + i];
+    }
+    __syncthreads();
+    sh[run][col] = acc;
+    __syncthreads();
+    if (run == 0 && i < n) {
+#pragma unroll
+      for (int r = 1; r < kSumRuns; r++) acc += sh[r][col];
+      out[i] = acc;
+    }
   }
 }
 
-// part[s][c] = sum over the voxels of slice s of g[v][c] (bias gradient)
-__global__ void k_channel_sum(const bf16 *__restrict__ g, float *__restrict__ part,
-                              long long nvox, int C, int S) {
-  const int s = blockIdx.x;
+// The elementwise kernels below move 8 channels (16 bytes) per thread; those
+// over voxels take one row (n, z, y) per block, so that an index costs no
+// 64-bit division.  With one channel per thread the network input took 156 us,
+// the head 147, the pooling 36 on average for 2 x 16 x 256 x 256 voxels; now
+// 35, 23 and 17.
+// V: 8, or 1 where the channels or an address do not allow 16-byte accesses.
+template <int V>
+__device__ __forceinline__ void ldv(const bf16 *p, float (&o)[V]) {
+  if constexpr (V == 8) {
+    const bf16x8 v = *reinterpret_cast<const bf16x8 *>(p);
+#pragma unroll
+    for (int k = 0; k < 8; k++) o[k] = (float)v[k];
+  } else {
+    o[0] = (float)p[0];
+  }
+}
+template <int V>
+__device__ __forceinline__ void stv(bf16 *p, const float (&o)[V]) {
+  if constexpr (V == 8) {
+    bf16x8 v;
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = (bf16)o[k];
+    *reinterpret_cast<bf16x8 *>(p) = v;
+  } else {
+    p[0] = (bf16)o[0];
+  }
+}
+
+struct Row {
+  int n, z, y;
+};
+__device__ __forceinline__ Row row_of(unsigned b, int D, int H) {
+  Row r;
+  const unsigned q = b / (unsigned)H;
+  r.y = (int)(b - q * (unsigned)H);
+  r.n = (int)(q / (unsigned)D);
+  r.z = (int)(q - (unsigned)r.n * (unsigned)D);
+  return r;
+}
+
+// A block's per-channel sums, combined over its threads: thread t holds V
+// channels of group t % nc in acc, the threads past a whole number of groups
+// nothing
+template <int V, int BS>
+__device__ __forceinline__ void block_channel_sum(const float (&acc)[V], int nc, float *sh,
+                                                  float *out) {
+  const int per = BS / nc * nc;
+#pragma unroll
+  for (int k = 0; k < V; k++) {
+    __syncthreads();
+    sh[threadIdx.x] = acc[k];
+    __syncthreads();
+    if ((int)threadIdx.x < nc) {
+      float s = 0.f;
+      for (int t = threadIdx.x; t < per; t += nc) s += sh[t];
+      out[threadIdx.x * V + k] = s;
+    }
+  }
+}
+
+// part[s][c] = sum over the voxels of slice s of g[v][c] (bias gradient): the
+// block's threads hold channel groups and step over the slice's voxels side by
+// side (one thread per channel, all voxels in turn: 163 us on average over the
+// layers of a training step on 4 x 8 x 128 x 128 voxels, 18 in this form)
+template <int V>
+__global__ __launch_bounds__(256) void k_channel_sum(const bf16 *__restrict__ g,
+                                                     float *__restrict__ part, long long nvox,
+                                                     int C, int S) {
+  __shared__ float sh[256];
+  const int s = blockIdx.x, CG = C / V;
   const long long v0 = nvox * s / S, v1 = nvox * (s + 1) / S;
-  for (int c = threadIdx.x; c < C; c += blockDim.x) {
-    float acc = 0.f;
-    for (long long v = v0; v < v1; v++) acc += (float)g[(size_t)v * C + c];
-    part[(size_t)s * C + c] = acc;
+  for (int c0 = 0; c0 < CG; c0 += 256) {
+    const int nc = min(256, CG - c0), vs = 256 / nc;
+    const int c = (int)threadIdx.x % nc, dv = (int)threadIdx.x / nc;
+    float acc[V] = {};
+    if (dv < vs) {
+#pragma unroll 4
+      for (long long v = v0 + dv; v < v1; v += vs) {
+        float x[V];
+        ldv<V>(g + (size_t)v * C + (c0 + c) * V, x);
+#pragma unroll
+        for (int k = 0; k < V; k++) acc[k] += x[k];
+      }
+    }
+    block_channel_sum<V, 256>(acc, nc, sh, part + (size_t)s * C + c0 * V);
   }
 }
 
 // g[i] = y[i] > 0 ? g[i] : 0 (ReLU backward through the stored output)
-__global__ void k_relu_bwd(const bf16 *__restrict__ y, bf16 *__restrict__ g, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
+__global__ void k_relu_bwd(const bf16 *__restrict__ y, bf16 *__restrict__ g, size_t n, int vec) {
+  const size_t n8 = vec ? n / 8 : 0;
+  const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = tid; i < n8; i += step) {
+    const bf16x8 a = reinterpret_cast<const bf16x8 *>(y)[i];
+    bf16x8 v = reinterpret_cast<bf16x8 *>(g)[i];
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = (float)a[k] > 0.f ? v[k] : (bf16)0.f;
+    reinterpret_cast<bf16x8 *>(g)[i] = v;
+  }
+  for (size_t i = n8 * 8 + tid; i < n; i += step)
     if (!((float)y[i] > 0.f)) g[i] = (bf16)0.f;
 }
 
-// 2x2x2 average pooling, forward and backward
-__global__ void k_avgpool2(const bf16 *__restrict__ in, bf16 *__restrict__ out, int N, int D,
-                           int H, int W, int C) {
-  const int Do = D / 2, Ho = H / 2, Wo = W / 2;
-  const size_t n = (size_t)N * Do * Ho * Wo * C;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    size_t q = i;
-    const int c = (int)(q % C); q /= C;
-    const int x = (int)(q % Wo); q /= Wo;
-    const int y = (int)(q % Ho); q /= Ho;
-    const int z = (int)(q % Do);
-    const int nn = (int)(q / Do);
-    float s = 0.f;
+// 2x2x2 average pooling, forward and backward (block: one output row)
+template <int V>
+__global__ __launch_bounds__(256) void k_avgpool2(const bf16 *__restrict__ in,
+                                                  bf16 *__restrict__ out, int D, int H, int W,
+                                                  int C) {
+  const Row r = row_of(blockIdx.x, D / 2, H / 2);
+  const int CG = C / V, items = W / 2 * CG;
+  const bf16 *src = in + (((size_t)r.n * D + 2 * r.z) * H + 2 * r.y) * (size_t)W * C;
+  bf16 *dst = out + (size_t)blockIdx.x * (W / 2) * C;
+  for (int i = threadIdx.x; i < items; i += 256) {
+    const int x = i / CG, c = (i - x * CG) * V;
+    float s[V] = {};
+#pragma unroll
     for (int k = 0; k < 8; k++) {
-      const size_t u = (((size_t)nn * D + 2 * z + (k >> 2)) * H + 2 * y + ((k >> 1) & 1)) * W +
-                       2 * x + (k & 1);
-      s += (float)in[u * C + c];
+      float v[V];
+      ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + 2 * x + (k & 1)) * C + c, v);
+#pragma unroll
+      for (int q = 0; q < V; q++) s[q] += v[q];
     }
-    out[i] = (bf16)(s * 0.125f);
+#pragma unroll
+    for (int q = 0; q < V; q++) s[q] *= 0.125f;
+    stv<V>(dst + (size_t)x * C + c, s);
   }
 }
 
-__global__ void k_avgpool2_bwd(const bf16 *__restrict__ gout, bf16 *__restrict__ gin, int N,
-                               int D, int H, int W, int C) {
-  const size_t n = (size_t)N * D * H * W * C;
-  const int Do = D / 2, Ho = H / 2, Wo = W / 2;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    size_t q = i;
-    const int c = (int)(q % C); q /= C;
-    const int x = (int)(q % W); q /= W;
-    const int y = (int)(q % H); q /= H;
-    const int z = (int)(q % D);
-    const int nn = (int)(q / D);
-    const size_t p = (((size_t)nn * Do + z / 2) * Ho + y / 2) * Wo + x / 2;
-    gin[i] = (bf16)((float)gout[p * C + c] * 0.125f);
+template <int V>
+__global__ __launch_bounds__(256) void k_avgpool2_bwd(const bf16 *__restrict__ gout,
+                                                      bf16 *__restrict__ gin, int D, int H, int W,
+                                                      int C) {
+  const Row r = row_of(blockIdx.x, D, H);
+  const int CG = C / V, items = W * CG;
+  const bf16 *src = gout + (((size_t)r.n * (D / 2) + r.z / 2) * (H / 2) + r.y / 2) * (size_t)(W / 2) * C;
+  bf16 *dst = gin + (size_t)blockIdx.x * W * C;
+  for (int i = threadIdx.x; i < items; i += 256) {
+    const int x = i / CG, c = (i - x * CG) * V;
+    float v[V];
+    ldv<V>(src + (size_t)(x / 2) * C + c, v);
+#pragma unroll
+    for (int q = 0; q < V; q++) v[q] *= 0.125f;
+    stv<V>(dst + (size_t)x * C + c, v);
   }
 }
 
 // out[v][0:Ca] = a[parent(v)][:] (nearest x2 upsampling of the coarse
 // features), out[v][Ca:Ca+Cb] = b[v][:] (the skip connection)
-__global__ void k_up2_concat(const bf16 *__restrict__ a, const bf16 *__restrict__ b,
-                             bf16 *__restrict__ out, int N, int D, int H, int W, int Ca, int Cb) {
-  const int C = Ca + Cb;
-  const size_t n = (size_t)N * D * H * W * C;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    size_t q = i;
-    const int c = (int)(q % C); q /= C;
-    const size_t v = q;
-    const int x = (int)(q % W); q /= W;
-    const int y = (int)(q % H); q /= H;
-    const int z = (int)(q % D);
-    const int nn = (int)(q / D);
-    if (c < Ca) {
-      const size_t p = (((size_t)nn * (D / 2) + z / 2) * (H / 2) + y / 2) * (W / 2) + x / 2;
-      out[i] = a[p * Ca + c];
-    } else {
-      out[i] = b[v * Cb + (c - Ca)];
-    }
+template <int V>
+__global__ __launch_bounds__(256) void k_up2_concat(const bf16 *__restrict__ a,
+                                                    const bf16 *__restrict__ b,
+                                                    bf16 *__restrict__ out, int D, int H, int W,
+                                                    int Ca, int Cb) {
+  const Row r = row_of(blockIdx.x, D, H);
+  const int C = Ca + Cb, CG = C / V, items = W * CG;
+  const bf16 *ra = a + (((size_t)r.n * (D / 2) + r.z / 2) * (H / 2) + r.y / 2) * (size_t)(W / 2) * Ca;
+  const bf16 *rb = b + (size_t)blockIdx.x * W * Cb;
+  bf16 *dst = out + (size_t)blockIdx.x * W * C;
+  for (int i = threadIdx.x; i < items; i += 256) {
+    const int x = i / CG, c = (i - x * CG) * V;
+    const bf16 *p = c < Ca ? ra + (size_t)(x / 2) * Ca + c : rb + (size_t)x * Cb + (c - Ca);
+    if constexpr (V == 8)
+      *reinterpret_cast<bf16x8 *>(dst + (size_t)x * C + c) = *reinterpret_cast<const bf16x8 *>(p);
+    else
+      dst[(size_t)x * C + c] = *p;
   }
 }
 
 // backward of k_up2_concat: ga[p][c] = sum over the 8 children of g[v][c],
-// gb[v][c] = g[v][Ca + c]
-__global__ void k_up2_concat_bwd(const bf16 *__restrict__ g, bf16 *__restrict__ ga,
-                                 bf16 *__restrict__ gb, int N, int D, int H, int W, int Ca,
-                                 int Cb) {
-  const int C = Ca + Cb;
-  const int Dc = D / 2, Hc = H / 2, Wc = W / 2;
-  const size_t na = (size_t)N * Dc * Hc * Wc * Ca;
-  const size_t nb = (size_t)N * D * H * W * Cb;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < na + nb;
-       i += (size_t)gridDim.x * blockDim.x) {
-    if (i < na) {
-      size_t q = i;
-      const int c = (int)(q % Ca); q /= Ca;
-      const int x = (int)(q % Wc); q /= Wc;
-      const int y = (int)(q % Hc); q /= Hc;
-      const int z = (int)(q % Dc);
-      const int nn = (int)(q / Dc);
-      float s = 0.f;
-      for (int k = 0; k < 8; k++) {
-        const size_t u = (((size_t)nn * D + 2 * z + (k >> 2)) * H + 2 * y + ((k >> 1) & 1)) * W +
-                         2 * x + (k & 1);
-        s += (float)g[u * C + c];
-      }
-      ga[i] = (bf16)s;
-    } else {
-      const size_t j = i - na;
-      const int c = (int)(j % Cb);
-      const size_t v = j / Cb;
-      gb[j] = g[v * C + Ca + c];
+// gb[v][c] = g[v][Ca + c]; block: one coarse row and the four full-size rows
+// of its children
+template <int V>
+__global__ __launch_bounds__(256) void k_up2_concat_bwd(const bf16 *__restrict__ g,
+                                                        bf16 *__restrict__ ga,
+                                                        bf16 *__restrict__ gb, int D, int H, int W,
+                                                        int Ca, int Cb) {
+  const Row r = row_of(blockIdx.x, D / 2, H / 2);
+  const int C = Ca + Cb, AG = Ca / V, BG = Cb / V;
+  const size_t row0 = ((size_t)r.n * D + 2 * r.z) * H + 2 * r.y;
+  const bf16 *src = g + row0 * W * C;
+  for (int i = threadIdx.x; i < W / 2 * AG; i += 256) {
+    const int x = i / AG, c = (i - x * AG) * V;
+    float s[V] = {};
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      float v[V];
+      ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + 2 * x + (k & 1)) * C + c, v);
+#pragma unroll
+      for (int q = 0; q < V; q++) s[q] += v[q];
+    }
+    stv<V>(ga + ((size_t)blockIdx.x * (W / 2) + x) * Ca + c, s);
+  }
+  for (int k = 0; k < 4; k++) {
+    const size_t row = row0 + (size_t)(k >> 1) * H + (k & 1);
+    for (int i = threadIdx.x; i < W * BG; i += 256) {
+      const int x = i / BG, c = (i - x * BG) * V;
+      if constexpr (V == 8)
+        *reinterpret_cast<bf16x8 *>(gb + (row * W + x) * Cb + c) =
+            *reinterpret_cast<const bf16x8 *>(g + (row * W + x) * C + Ca + c);
+      else
+        gb[(row * W + x) * Cb + c] = g[(row * W + x) * C + Ca + c];
     }
   }
 }
@@ -527,16 +635,24 @@ __global__ void k_up2_concat_bwd(const bf16 *__restrict__ g, bf16 *__restrict__ 
 // fbp[v], channels 2..31 zero; the volumes are fp32 [N][D][H][W] (one
 // sample per frame) and mean is [D][H][W] (shared by all samples)
 __global__ void k_make_input(const float *__restrict__ fbp, const float *__restrict__ mean,
-                             bf16 *__restrict__ x, long long nvox, long long per, float scale) {
-  const size_t n = (size_t)nvox * 32;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+                             bf16 *__restrict__ x, long long nvox, long long per, float scale,
+                             int vec) {
+  const bool small = nvox <= 0x7fffffffLL && per <= 0x7fffffffLL;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < (size_t)nvox * 4;
        i += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % 32);
-    const size_t v = i / 32;
-    float val = 0.f;
-    if (c == 0) val = scale * fbp[v];
-    else if (c == 1 && mean) val = scale * mean[v % per];
-    x[i] = (bf16)val;
+    const size_t v = i >> 2;
+    bf16x8 o = zero8();
+    if ((i & 3) == 0) {
+      o[0] = (bf16)(scale * fbp[v]);
+      if (mean) o[1] = (bf16)(scale * mean[small ? (uint32_t)v % (uint32_t)per : v % (size_t)per]);
+    }
+    bf16 *p = x + v * 32 + (i & 3) * 8;
+    if (vec) {
+      *reinterpret_cast<bf16x8 *>(p) = o;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; k++) p[k] = o[k];
+    }
   }
 }
 
@@ -556,11 +672,23 @@ __global__ void k_frame_mean(const float *__restrict__ x, float *__restrict__ me
 // convolution to one channel, a residual on the filtered back-projection)
 __global__ void k_head_fwd(const bf16 *__restrict__ h, const float *__restrict__ w,
                            const float *__restrict__ b, const float *__restrict__ fbp,
-                           float *__restrict__ out, long long nvox, int C, float inv_scale) {
+                           float *__restrict__ out, long long nvox, int C, float inv_scale,
+                           int vec) {
   for (size_t v = blockIdx.x * (size_t)blockDim.x + threadIdx.x; v < (size_t)nvox;
        v += (size_t)gridDim.x * blockDim.x) {
     float s = b[0];
-    for (int c = 0; c < C; c++) s += w[c] * (float)h[v * C + c];
+    if (vec) {
+      for (int c = 0; c < C; c += 32) {
+        bf16x8 x[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          x[k] = *reinterpret_cast<const bf16x8 *>(h + v * C + c + 8 * k);
+#pragma unroll
+        for (int k = 0; k < 32; k++) s += w[c + k] * (float)x[k / 8][k % 8];
+      }
+    } else {
+      for (int c = 0; c < C; c++) s += w[c] * (float)h[v * C + c];
+    }
     out[v] = fbp[v] + s * inv_scale;
   }
 }
@@ -588,26 +716,49 @@ __global__ void k_mse(const float *__restrict__ out, const float *__restrict__ t
 
 // head backward: gh[v][c] = gout[v] w[c] / scale (bf16); the head's weight
 // and bias gradients per slice of voxels: part[s][c] = sum gout[v] h[v][c] /
-// scale (c < C), part[s][C] = sum gout[v] / scale
-__global__ void k_head_bwd(const bf16 *__restrict__ h, const float *__restrict__ w,
-                           const float *__restrict__ gout, bf16 *__restrict__ gh,
-                           float *__restrict__ part, long long nvox, int C, int S,
-                           float inv_scale) {
-  const size_t n = (size_t)nvox * C;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % C);
-    gh[i] = (bf16)(gout[i / C] * inv_scale * w[c]);
-  }
-  // weight gradient partials: block b < S takes slice b
-  if ((int)blockIdx.x < S) {
-    const int s = blockIdx.x;
-    const long long v0 = nvox * s / S, v1 = nvox * (s + 1) / S;
-    for (int c = threadIdx.x; c <= C; c += blockDim.x) {
-      float acc = 0.f;
-      for (long long v = v0; v < v1; v++)
-        acc += gout[v] * inv_scale * (c < C ? (float)h[(size_t)v * C + c] : 1.f);
-      part[(size_t)s * (C + 1) + c] = acc;
+// scale (c < C), part[s][C] = sum gout[v] / scale.  One pass, block = slice:
+// the weight sums, once a thread per channel walking the slice's voxels, were
+// the whole of its 417 us for 4 x 8 x 128 x 128 voxels; now 55.
+template <int V>
+__global__ __launch_bounds__(512) void k_head_bwd(const bf16 *__restrict__ h,
+                                                  const float *__restrict__ w,
+                                                  const float *__restrict__ gout,
+                                                  bf16 *__restrict__ gh, float *__restrict__ part,
+                                                  long long nvox, int C, int S, float inv_scale) {
+  __shared__ float sh[512];
+  const int s = blockIdx.x, CG = C / V;
+  const long long v0 = nvox * s / S, v1 = nvox * (s + 1) / S;
+  for (int c0 = 0; c0 < CG; c0 += 512) {
+    const int nc = min(512, CG - c0), vs = 512 / nc;
+    const int cg = (int)threadIdx.x % nc, dv = (int)threadIdx.x / nc, c = (c0 + cg) * V;
+    float acc[V] = {}, wc[V], gs = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; k++) wc[k] = w[c + k];
+    if (dv < vs) {
+#pragma unroll 4
+      for (long long v = v0 + dv; v < v1; v += vs) {
+        const float g = gout[v] * inv_scale;
+        float x[V], o[V];
+        ldv<V>(h + (size_t)v * C + c, x);
+#pragma unroll
+        for (int k = 0; k < V; k++) {
+          o[k] = g * wc[k];
+          acc[k] += g * x[k];
+        }
+        stv<V>(gh + (size_t)v * C + c, o);
+        gs += g;
+      }
+    }
+    block_channel_sum<V, 512>(acc, nc, sh, part + (size_t)s * (C + 1) + c0 * V);
+    if (c0 == 0) {
+      __syncthreads();
+      sh[threadIdx.x] = gs;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        float t = 0.f;
+        for (int k = 0; k < vs; k++) t += sh[k * nc];
+        part[(size_t)s * (C + 1) + C] = t;
+      }
     }
   }
 }
@@ -632,10 +783,18 @@ __global__ void k_adam(float *__restrict__ p, const float *__restrict__ gr, floa
 
 // a[i] = a[i] + b[i] (bf16, the sum rounded once): gradients reaching one
 // activation from two consumers
-__global__ void k_add_bf16(bf16 *__restrict__ a, const bf16 *__restrict__ b, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    a[i] = (bf16)((float)a[i] + (float)b[i]);
+__global__ void k_add_bf16(bf16 *__restrict__ a, const bf16 *__restrict__ b, size_t n, int vec) {
+  const size_t n8 = vec ? n / 8 : 0;
+  const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = tid; i < n8; i += step) {
+    bf16x8 x = reinterpret_cast<bf16x8 *>(a)[i];
+    const bf16x8 y = reinterpret_cast<const bf16x8 *>(b)[i];
+#pragma unroll
+    for (int k = 0; k < 8; k++) x[k] = (bf16)((float)x[k] + (float)y[k]);
+    reinterpret_cast<bf16x8 *>(a)[i] = x;
+  }
+  for (size_t i = n8 * 8 + tid; i < n; i += step) a[i] = (bf16)((float)a[i] + (float)b[i]);
 }
 
 __global__ void k_to_bf16(const float *__restrict__ a, bf16 *__restrict__ b, size_t n) {
@@ -674,6 +833,8 @@ static int grid1d(size_t n) {
   if (g > 65535 * 8) g = 65535 * 8;
   return (int)g;
 }
+
+static bool al16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 extern "C" const char *tb_nn_last_error(void) { return g_nn_err.c_str(); }
 
@@ -802,6 +963,11 @@ extern "C" int tb_nn_conv3d_flip(const void *w, void *wt, int32_t cin, int32_t c
   return 0;
 }
 
+static void sum_parts(const float *part, float *out, size_t n, int slices, hipStream_t s) {
+  const unsigned blocks = (unsigned)std::min<size_t>(std::max<size_t>((n + 63) / 64, 1), 65536);
+  hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(64 * kSumRuns), 0, s, part, out, n, slices);
+}
+
 extern "C" int tb_nn_conv3d_wgrad(const void *in, const void *gout, float *gw, float *part,
                                   int32_t slices, int32_t n, int32_t d, int32_t h, int32_t wd,
                                   int32_t cin, int32_t cout, void *stream) {
@@ -814,7 +980,7 @@ extern "C" int tb_nn_conv3d_wgrad(const void *in, const void *gout, float *gw, f
                      0, s, static_cast<const bf16 *>(in), static_cast<const bf16 *>(gout), part,
                      n, d, h, wd, cin, cout, slices);
   const size_t nw = (size_t)kTaps * cin * cout;
-  hipLaunchKernelGGL(k_sum_parts, dim3(grid1d(nw)), dim3(256), 0, s, part, gw, nw, slices);
+  sum_parts(part, gw, nw, slices, s);
   NNCHK("tb_nn_conv3d_wgrad");
   return 0;
 }
@@ -822,18 +988,27 @@ extern "C" int tb_nn_conv3d_wgrad(const void *in, const void *gout, float *gw, f
 extern "C" int tb_nn_channel_sum(const void *g, float *out, float *part, int32_t slices,
                                  int64_t nvox, int32_t c, void *stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_channel_sum, dim3(slices), dim3(64), 0, s, static_cast<const bf16 *>(g),
-                     part, (long long)nvox, c, slices);
-  hipLaunchKernelGGL(k_sum_parts, dim3(grid1d(c)), dim3(256), 0, s, part, out, (size_t)c, slices);
+  auto fn = c % 8 == 0 && al16(g) ? k_channel_sum<8> : k_channel_sum<1>;
+  hipLaunchKernelGGL(fn, dim3(slices), dim3(256), 0, s, static_cast<const bf16 *>(g), part,
+                     (long long)nvox, c, slices);
+  sum_parts(part, out, (size_t)c, slices, s);
   NNCHK("tb_nn_channel_sum");
   return 0;
 }
 
 extern "C" int tb_nn_relu_bwd(const void *y, void *g, int64_t count, void *stream) {
-  hipLaunchKernelGGL(k_relu_bwd, dim3(grid1d(count)), dim3(256), 0,
+  hipLaunchKernelGGL(k_relu_bwd, dim3(grid1d((count + 7) / 8)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), static_cast<const bf16 *>(y),
-                     static_cast<bf16 *>(g), (size_t)count);
+                     static_cast<bf16 *>(g), (size_t)count, al16(y) && al16(g));
   NNCHK("tb_nn_relu_bwd");
+  return 0;
+}
+
+// blocks of the row kernels: one per row of an n x d x h volume
+static int row_blocks(long long n, long long d, long long h, unsigned *out) {
+  const long long r = n * d * h;
+  if (r > 0x7fffffffLL) return nn_fail("volume too large");
+  *out = r > 0 ? (unsigned)r : 0u;
   return 0;
 }
 
@@ -841,48 +1016,60 @@ extern "C" int tb_nn_avgpool2(const void *in, void *out, int32_t n, int32_t d, i
                               int32_t wd, int32_t c, int32_t backward, void *stream) {
   if (d % 2 || h % 2 || wd % 2) return nn_fail("tb_nn_avgpool2: odd size");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (backward)
-    hipLaunchKernelGGL(k_avgpool2_bwd, dim3(grid1d((size_t)n * d * h * wd * c)), dim3(256), 0, s,
-                       static_cast<const bf16 *>(in), static_cast<bf16 *>(out), n, d, h, wd, c);
-  else
-    hipLaunchKernelGGL(k_avgpool2, dim3(grid1d((size_t)n * d * h * wd * c / 8)), dim3(256), 0, s,
-                       static_cast<const bf16 *>(in), static_cast<bf16 *>(out), n, d, h, wd, c);
+  const bool vec = c % 8 == 0 && al16(in) && al16(out);
+  const int k = backward ? 1 : 2;
+  unsigned rows = 0;
+  if (row_blocks(n, d / k, h / k, &rows)) return -1;
+  if (!rows) return 0;
+  auto fn = backward ? (vec ? k_avgpool2_bwd<8> : k_avgpool2_bwd<1>)
+                     : (vec ? k_avgpool2<8> : k_avgpool2<1>);
+  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, s, static_cast<const bf16 *>(in),
+                     static_cast<bf16 *>(out), d, h, wd, c);
   NNCHK("tb_nn_avgpool2");
   return 0;
 }
 
 extern "C" int tb_nn_up2_concat(const void *a, const void *b, void *out, int32_t n, int32_t d,
                                 int32_t h, int32_t wd, int32_t ca, int32_t cb, void *stream) {
-  hipLaunchKernelGGL(k_up2_concat, dim3(grid1d((size_t)n * d * h * wd * (ca + cb))), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const bf16 *>(a),
-                     static_cast<const bf16 *>(b), static_cast<bf16 *>(out), n, d, h, wd, ca, cb);
+  unsigned rows = 0;
+  if (row_blocks(n, d, h, &rows)) return -1;
+  if (!rows) return 0;
+  auto fn = ca % 8 == 0 && cb % 8 == 0 && al16(a) && al16(b) && al16(out) ? k_up2_concat<8>
+                                                                          : k_up2_concat<1>;
+  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const bf16 *>(a), static_cast<const bf16 *>(b),
+                     static_cast<bf16 *>(out), d, h, wd, ca, cb);
   NNCHK("tb_nn_up2_concat");
   return 0;
 }
 
 extern "C" int tb_nn_up2_concat_bwd(const void *g, void *ga, void *gb, int32_t n, int32_t d,
                                     int32_t h, int32_t wd, int32_t ca, int32_t cb, void *stream) {
-  const size_t tot = (size_t)n * (d / 2) * (h / 2) * (wd / 2) * ca + (size_t)n * d * h * wd * cb;
-  hipLaunchKernelGGL(k_up2_concat_bwd, dim3(grid1d(tot)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const bf16 *>(g),
-                     static_cast<bf16 *>(ga), static_cast<bf16 *>(gb), n, d, h, wd, ca, cb);
+  unsigned rows = 0;
+  if (row_blocks(n, d / 2, h / 2, &rows)) return -1;
+  if (!rows) return 0;
+  auto fn = ca % 8 == 0 && cb % 8 == 0 && al16(g) && al16(ga) && al16(gb) ? k_up2_concat_bwd<8>
+                                                                          : k_up2_concat_bwd<1>;
+  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const bf16 *>(g), static_cast<bf16 *>(ga),
+                     static_cast<bf16 *>(gb), d, h, wd, ca, cb);
   NNCHK("tb_nn_up2_concat_bwd");
   return 0;
 }
 
 extern "C" int tb_nn_add(void *a, const void *b, int64_t count, void *stream) {
-  hipLaunchKernelGGL(k_add_bf16, dim3(grid1d(count)), dim3(256), 0,
+  hipLaunchKernelGGL(k_add_bf16, dim3(grid1d((count + 7) / 8)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), static_cast<bf16 *>(a),
-                     static_cast<const bf16 *>(b), (size_t)count);
+                     static_cast<const bf16 *>(b), (size_t)count, al16(a) && al16(b));
   NNCHK("tb_nn_add");
   return 0;
 }
 
 extern "C" int tb_nn_make_input(const float *fbp, const float *mean, void *x, int64_t nvox,
                                 int64_t per_sample, float scale, void *stream) {
-  hipLaunchKernelGGL(k_make_input, dim3(grid1d((size_t)nvox * 32)), dim3(256), 0,
+  hipLaunchKernelGGL(k_make_input, dim3(grid1d((size_t)nvox * 4)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), fbp, mean, static_cast<bf16 *>(x),
-                     (long long)nvox, (long long)per_sample, scale);
+                     (long long)nvox, (long long)per_sample, scale, al16(x));
   NNCHK("tb_nn_make_input");
   return 0;
 }
@@ -900,7 +1087,7 @@ extern "C" int tb_nn_head(const void *h, const float *w, const float *b, const f
                           float *out, int64_t nvox, int32_t c, float scale, void *stream) {
   hipLaunchKernelGGL(k_head_fwd, dim3(grid1d(nvox)), dim3(256), 0,
                      static_cast<hipStream_t>(stream), static_cast<const bf16 *>(h), w, b, fbp,
-                     out, (long long)nvox, c, 1.f / scale);
+                     out, (long long)nvox, c, 1.f / scale, c % 32 == 0 && al16(h));
   NNCHK("tb_nn_head");
   return 0;
 }
@@ -908,8 +1095,8 @@ extern "C" int tb_nn_head(const void *h, const float *w, const float *b, const f
 extern "C" int tb_nn_head_bwd(const void *h, const float *w, const float *gout, void *gh,
                               float *part, int32_t slices, int64_t nvox, int32_t c, float scale,
                               void *stream) {
-  const int blocks = std::max(grid1d((size_t)nvox * c), (int)slices);
-  hipLaunchKernelGGL(k_head_bwd, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream),
+  auto fn = c % 8 == 0 && al16(h) && al16(gh) ? k_head_bwd<8> : k_head_bwd<1>;
+  hipLaunchKernelGGL(fn, dim3(slices), dim3(512), 0, static_cast<hipStream_t>(stream),
                      static_cast<const bf16 *>(h), w, gout, static_cast<bf16 *>(gh), part,
                      (long long)nvox, c, slices, 1.f / scale);
   NNCHK("tb_nn_head_bwd");
@@ -926,8 +1113,7 @@ extern "C" int tb_nn_mse(const float *out, const float *target, float *gout, dou
 
 extern "C" int tb_nn_sum_parts(const float *part, float *out, int64_t count, int32_t slices,
                                void *stream) {
-  hipLaunchKernelGGL(k_sum_parts, dim3(grid1d(count)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), part, out, (size_t)count, slices);
+  sum_parts(part, out, (size_t)count, slices, static_cast<hipStream_t>(stream));
   NNCHK("tb_nn_sum_parts");
   return 0;
 }
