@@ -79,6 +79,27 @@ def test_conv3d_up2cat_is_the_two_calls(L, shape, ca, cb, cout):
                                  None) == -1
 
 
+@pytest.mark.parametrize("shape,cin,cout,slices", [
+    ((1, 1, 1, 1), 32, 32, 1), ((1, 5, 16, 32), 32, 32, 3), ((2, 3, 17, 33), 32, 64, 256),
+    ((1, 9, 15, 70), 96, 32, 5), ((3, 2, 33, 31), 64, 96, 2)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_conv3d_wgrad_tiles(L, shape, cin, cout, slices, off):
+    """Within 5e-5 of the largest value of the float64 sums, as
+    test_conv3d_matches_oracle; operands at aligned and unaligned addresses."""
+    log(f"wgrad tile {shape} {cin}->{cout} slices {slices} offset {off}")
+    rng = np.random.default_rng(cin + 3 * cout)
+    x = U.bf16(rng.standard_normal(shape + (cin,)).astype(np.float32))
+    g = U.bf16(rng.standard_normal(shape + (cout,)).astype(np.float32))
+    pad = np.zeros(off, np.float32)
+    xt = bf(np.concatenate([pad, x.ravel()]))
+    gt = bf(np.concatenate([pad, g.ravel()]))
+    gw, part = empty((27, cout, cin)), empty((slices * 27 * cin * cout,))
+    assert L.tb_nn_conv3d_wgrad(at(xt, off, 2), at(gt, off, 2), ptr(gw), ptr(part), slices, *shape,
+                                cin, cout, None) == 0
+    ref = U.conv3d_wgrad(x.astype(np.float64), g.astype(np.float64))
+    assert np.abs(host(gw) - ref).max() <= 5e-5 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("c,off", [(32, 0), (32, 1), (96, 0), (5, 0)])
 def test_elementwise_forms_agree(L, c, off):
     """Pooling, upsampling, their backward passes, ReLU and the sum of two
