@@ -102,7 +102,7 @@ __device__ __forceinline__ float qggmrf_b(float d, float sq, float sqp, float c)
 // active.
 template <int CTRL>
 __device__ __forceinline__ int dpp_all(int v) {
-  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, false);
+  return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true);
 }
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -165,6 +165,23 @@ __device__ __forceinline__ void wave_total_df(double &d, float &f) {
   f = swap_sum_f<false>(f);
   d = swap_sum_d<true>(d);
   f = swap_sum_f<true>(f);
+}
+// The same sums, pair by pair, with the total in lane 63 alone: the last two
+// levels take the other rows' sums by row broadcast, one move for a register
+// instead of a copy and a swap.
+__device__ __forceinline__ void wave_last_df(double &d, float &f) {
+  d += dpp_d<0xB1>(d);
+  f += dpp_f<0xB1>(f);
+  d += dpp_d<0x4E>(d);
+  f += dpp_f<0x4E>(f);
+  d += dpp_d<0x141>(d);
+  f += dpp_f<0x141>(f);
+  d += dpp_d<0x140>(d);
+  f += dpp_f<0x140>(f);
+  d += dpp_d<0x142>(d);  // row_bcast15: rows 1 and 3 take rows 0 and 2
+  f += dpp_f<0x142>(f);
+  d += dpp_d<0x143>(d);  // row_bcast31: row 3 takes the lower half's sum
+  f += dpp_f<0x143>(f);
 }
 // Two float sums in plain FP32, level by level as wave_total_df.
 __device__ __forceinline__ void wave_total_ff(float &a, float &b) {
@@ -242,6 +259,20 @@ __device__ __forceinline__ void lo32_total_ff(float &a, float &b) {
   b += dpp_f<0x140>(b);
   a = swap_sum_f<false>(a);
   b = swap_sum_f<false>(b);
+}
+
+// The same two sums over lanes 0..31, in lane 31 alone.
+__device__ __forceinline__ void lo32_last_ff(float &a, float &b) {
+  a += dpp_f<0xB1>(a);
+  b += dpp_f<0xB1>(b);
+  a += dpp_f<0x4E>(a);
+  b += dpp_f<0x4E>(b);
+  a += dpp_f<0x141>(a);
+  b += dpp_f<0x141>(b);
+  a += dpp_f<0x140>(a);
+  b += dpp_f<0x140>(b);
+  a += dpp_f<0x142>(a);
+  b += dpp_f<0x142>(b);
 }
 
 }  // namespace tb

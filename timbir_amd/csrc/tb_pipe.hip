@@ -120,6 +120,53 @@ __device__ __forceinline__ bool huber_sel(const KP &P, float e, float w) {
   return (q - P.T2h) + (corr - P.T2l) < 0.0f;
 }
 
+// Generalized-Huber weights (XT_VoxUpdate.c:66-80) of N entries of a lane:
+// w inside the threshold, T delta sqrt(w) / |e| outside.  The rounded e^2 w
+// decides wherever it is off T^2 by more than its own error (2^-22 of it;
+// the band is four times that, and 2^-20 for what underflow loses), and
+// huber_sel inside the band.  The outer weight is evaluated only when some
+// lane of the wave needs it.
+struct HuberBand {
+  float lo, hi;
+};
+__device__ __forceinline__ HuberBand huber_band(const KP &P) {
+  const float d = fmaf(P.T2h, 0x1p-20f, 0x1p-20f);
+  HuberBand B;
+  B.lo = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(P.T2h - d)));
+  B.hi = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(P.T2h + d)));
+  return B;
+}
+template <int N>
+__device__ __forceinline__ void huber_weights(const KP &P, const HuberBand &B,
+                                              const float (&e)[N], const float (&w)[N],
+                                              float (&cw)[N]) {
+  float q[N];
+  unsigned long long in = ~0ull;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    q[k] = e[k] * e[k] * w[k];
+    cw[k] = w[k];
+    in &= __builtin_amdgcn_ballot_w64(q[k] < B.lo);
+  }
+  if (__builtin_expect(in != ~0ull, 0)) {
+    bool sel[N], edge = false;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      sel[k] = q[k] < B.lo;
+      edge |= !(sel[k] | (q[k] > B.hi));
+    }
+    if (__builtin_amdgcn_ballot_w64(edge) != 0ull) {
+#pragma unroll
+      for (int k = 0; k < N; k++) sel[k] = huber_sel(P, e[k], w[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const float out = P.Td * __builtin_amdgcn_sqrtf(w[k]) * __builtin_amdgcn_rcpf(fabsf(e[k]));
+      cw[k] = sel[k] ? w[k] : out;
+    }
+  }
+}
+
 constexpr int kNoPix = 0x7fffffff;  // empty slot (never equals a packed pixel)
 
 // One wavefront per cell, lane = view (VPL views per lane).  The workgroup
@@ -432,6 +479,15 @@ __global__ __launch_bounds__(64) void k_icd_lds(KP P, const int2 *__restrict__ c
 // partial sums in LDS and meets the others at one barrier; then every wave
 // evaluates the same closed-form step from the same sums in the same order,
 // so all waves hold the identical dx.
+//
+// What bounds it: one voxel after another, each a chain of about 100
+// instructions of the theta wave and as many of the prior wave, issued by one
+// wavefront per SIMD at 4 to 5 cycles each, around two LDS round trips and a
+// barrier.  So the instructions count: no copies between groups (the ring),
+// the lane's own A value and w0 loaded rather than picked from a record, row
+// broadcasts in the last levels of the sums, one rounded product for the
+// Huber test.  256 x 256, 64 views a frame, 128 cells: 525 ns a voxel before,
+// 420 after (11.08 and 8.84 ms a pass of one chunk in each colour).
 // ---------------------------------------------------------------------------
 struct StepIn {
   double t1[2][16];  // per theta wave, double-buffered by voxel parity
@@ -445,9 +501,10 @@ struct StepIn {
 // waves, theta2 in FP32.  TF 1: both in FP32 with compensated (TwoSum)
 // accumulation over lanes; the waves' compensated totals s + c are exact in
 // FP64 and added there.  TF 2: both in plain FP32 throughout.
-template <int MAXTH, int TF = 0>
+// between() is run between the reads of the published values and their use.
+template <int MAXTH, int TF = 0, class F>
 __device__ __forceinline__ float solve_step(const KP &P, const StepIn &S, int par, int nth,
-                                            float *V_out, bool *skip_out) {
+                                            float *V_out, bool *skip_out, F between) {
 #pragma clang fp contract(off)
   // every slot is read at once (one LDS latency) and added as a fixed
   // pairwise tree over the MAXTH slots; slots of absent waves hold zero
@@ -459,6 +516,9 @@ __device__ __forceinline__ float solve_step(const KP &P, const StepIn &S, int pa
     a1[w] = (T1T)S.t1[par][w];
     a2[w] = S.t2[par][w];
   }
+  const float pb = S.pr[par][0], pbx = S.pr[par][1], V = S.pr[par][2];
+  const bool skip = S.pr[par][3] != 0.0f;
+  between();
 #pragma unroll
   for (int m = MAXTH; m > 1; m = (m + 1) / 2) {
     const int h = (m + 1) / 2;
@@ -471,14 +531,17 @@ __device__ __forceinline__ float solve_step(const KP &P, const StepIn &S, int pa
   const double T1 = (double)a1[0];
   const float T2 = a2[0];
   (void)nth;
-  const float pb = S.pr[par][0], pbx = S.pr[par][1], V = S.pr[par][2];
-  const bool skip = S.pr[par][3] != 0.0f;
   const float th1 = (float)T1;
   const float num = P.alpha * (pbx - th1);
   const float step = num * __builtin_amdgcn_rcpf(pb + T2);
   *V_out = V;
   *skip_out = skip;
   return skip ? V : V + step;
+}
+template <int MAXTH, int TF = 0>
+__device__ __forceinline__ float solve_step(const KP &P, const StepIn &S, int par, int nth,
+                                            float *V_out, bool *skip_out) {
+  return solve_step<MAXTH, TF>(P, S, par, nth, V_out, skip_out, [] {});
 }
 
 // A-matrix column of a voxel in one view (calcAMatrixColumnforAngle,
@@ -572,14 +635,25 @@ template __global__ void k_build_columns<9>(KP);
 template __global__ void k_build_columns<17>(KP);
 
 // The prior wave of the multi-wavefront kernels: the object side of the
-// voxel sequence (neighbour prefetch one group ahead with in-flight patching,
-// the qGGMRF prior surrogate of XT_ICD_update.c:134-183, zero-skip,
+// voxel sequence (neighbour prefetch with in-flight patching, the qGGMRF
+// prior surrogate of XT_ICD_update.c:134-183, zero-skip,
 // XT_VoxUpdate.c:236-259, the object and update-map stores), meeting the
 // theta waves at one barrier per voxel.
+//
+// RING (the LDS kernel, whose theta waves load little): the neighbours of
+// voxel n + G are loaded right after voxel n's value is stored, into the
+// registers voxel n has just left, so the G voxels of the unrolled loop are
+// the ring, nothing is copied and no wait covers more than the load it needs.
+// Otherwise (e and w in global memory) the next group's neighbours are loaded
+// together at the start of a group: a gather per voxel between the theta
+// waves' loads slows those (512 x 512, 128 views a frame: 104 against 92 ms
+// a pass).  A load sees every value stored before it (one wavefront's
+// accesses to one address take effect in issue order); the loads in flight
+// at a store that hold the stored voxel as an in-plane neighbour are patched.
 // PAD: the theta waves run whole groups of G voxels, the last one padded
 // with empty slots; the prior wave meets them at every slot, publishing a
 // skipped step (dx = 0) for an empty one.
-template <int MAXTH, bool PAD = false>
+template <int MAXTH, bool RING, bool PAD = false>
 __device__ __forceinline__ void prior_wave(const KP &P, StepIn &S, const int *list, int n0,
                                            int cnt, int f, int z, int iter, int seq,
                                            int count_mag, int nth, int lane) {
@@ -603,137 +677,160 @@ __device__ __forceinline__ void prior_wave(const KP &P, StepIn &S, const int *li
       nsq = P.sTq, nisqp = 1.0f / P.sTqp, nc = P.c_t;
     }
   }
-  const bool inplane = lane < 27 && ndz == 0 && lane != 13;
-  const int noff = ndy * 65536 + ndx;
+  const bool neighb = lane != 13;
   const int zz = z + ndz, ff = f + ndt;
   const bool zok = nlane && zz >= 0 && zz < P.N_z && ff >= 0 && ff < P.N_time;
   const int zc = min(max(zz, 0), P.N_z - 1), fc = min(max(ff, 0), P.N_time - 1);
-  const int nplane = (fc * P.N_z + zc) * Nxy;
-  const int cbase = cell * Nxy;
+  // the lane's neighbour of packed pixel pix and linear pixel lin: packed
+  // pix + noff, object word lin + nbase.  A lane whose neighbour lies in no
+  // slice or frame of the object has an offset that leaves the image.
+  const unsigned noff = zok ? (unsigned)(ndy * 65536 + ndx) : 0x80000000u;
+  const int nbase = (fc * P.N_z + zc) * Nxy + ndy * P.N_x + ndx;
+  // pix - (packed in-plane neighbour) of this lane; a value no pair of
+  // pixels has in the other lanes
+  const int poff = lane < 27 && ndz == 0 && lane != 13 ? ndy * 65536 + ndx : 0x7f000000;
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  us2 lim;
+  lim[0] = (unsigned short)(P.N_x - 1);
+  lim[1] = (unsigned short)(P.N_y - 1);
   const float two_c = 2.0f * nc;
+  // a voxel's value and map entry are stored by lane 0: the other lanes'
+  // offsets lie past the slice's plane, where buffer stores have no effect
+  const __amdgpu_buffer_rsrc_t objc =
+      __builtin_amdgcn_make_buffer_rsrc(P.obj + (size_t)cell * Nxy, (short)0, Nxy * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t magc =
+      __builtin_amdgcn_make_buffer_rsrc(P.mag + (size_t)cell * Nxy, (short)0, Nxy * 4, 0x00020000);
+  const unsigned voff = lane == 0 ? 0u : 0xffffffffu;
 
-  int apix[G], anid[G], bpix[G], bnid[G];
-  float anb[G], bnb[G], bnv[G];
-  // packed pixels of the pending voxels, one per lane (A in lanes 0..G-1,
-  // B in lanes G..2G-1): one vector test per update finds the rare case of
-  // an in-plane neighbour among them
-  int pend = kNoPix;
-  auto fill = [&](int k, int pix) {
-    bpix[k] = pix;
-    const bool valid = pix != kNoPix;
-    const int yy = valid ? (pix >> 16) : 0, xx = valid ? (pix & 0xffff) : 0;
-    const int jj = yy + ndy, kk = xx + ndx;
-    const bool nok = valid & zok & (jj >= 0) & (jj < P.N_y) & (kk >= 0) & (kk < P.N_x);
-    bnb[k] = P.obj[(unsigned)(nok ? nplane + jj * P.N_x + kk : P.nobj + 64)];
-    bnid[k] = (valid & inplane) ? pix + noff : -2;
-    bnv[k] = __int_as_float(0x7fc00000);
+  // the neighbour value of this lane, or the NaN word: both coordinates of
+  // pix + noff, taken modulo 2^16, are at most N - 1 (saturating u16
+  // differences are zero)
+  auto fetch = [&](int pix, int lin) -> float {
+    const us2 t = __builtin_bit_cast(us2, (unsigned)pix + noff);
+    const us2 over = __builtin_elementwise_sub_sat(t, lim);
+    const bool ok = __builtin_bit_cast(unsigned, over) == 0u;
+    return P.obj[(unsigned)(ok ? nbase + lin : P.nobj + 64)];
   };
-  double vmacc = 0.0;  // lane k: magnitudes of the voxels at group position k
-  unsigned long long nupd = 0, nzero = 0;
-  const int ngroups = (cnt + G - 1) / G;
-  int raw = list[n0 + min(lane, cnt - 1)];
-  wait_vm_all();
-  int pnext[G];
-#pragma unroll
-  for (int k = 0; k < G; k++) pnext[k] = k < cnt ? __builtin_amdgcn_readlane(raw, k) : kNoPix;
+  // lane k: the voxel k places on from the group's first (the last voxel
+  // past the end, which is loaded and not used)
+  auto at = [&](int n) -> int { return list[n0 + min(n + lane, cnt - 1)]; };
+  auto lin_of = [&](int pix) -> int { return (pix >> 16) * P.N_x + (pix & 0xffff); };
+  float anb[G], bnb[G];  // neighbours of this group's voxels (RING: of the
+                         // next G), and of the next group's
+  int pv = at(0), lv = lin_of(pv);
+  int raw = at(G);
 #pragma unroll
   for (int k = 0; k < G; k++) {
-    apix[k] = kNoPix;
-    anid[k] = -2;
-    anb[k] = __int_as_float(0x7fc00000);
+    // issued in the order of the loop, with stores of no lane in place of a
+    // voxel's, so that the loop's first pass waits for no more than the others
+    if (RING) {
+      __builtin_amdgcn_raw_buffer_store_b32(0u, objc, 0xffffffffu, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(0u, magc, 0xffffffffu, 0, 0);
+    }
+    anb[k] = fetch(__builtin_amdgcn_readlane(pv, k), __builtin_amdgcn_readlane(lv, k));
   }
-  for (int g = 0; g <= ngroups; g++) {
+  double vm[G];  // |x| sums of the voxels at each group position
 #pragma unroll
-    for (int k = 0; k < G; k++) fill(k, pnext[k]);
-    raw = list[n0 + min((g + 1) * G + lane, cnt - 1)];
+  for (int k = 0; k < G; k++) vm[k] = 0.0;
+  int nzero = 0;
+  // left by its end alone: a way round from an early exit back to the loop's
+  // head would make every wait in it cover that way's order of the loads too
+  auto sweep = [&] {
+    for (int n = 0;; n += G) {
+      const unsigned pend = (unsigned)pv + 65537u;
+      const int pvn = raw;
+      raw = at(n + 2 * G);
+      if (!RING) {
 #pragma unroll
-    for (int k = 0; k < G; k++) pend = lane == G + k ? bpix[k] : pend;
-    float rx = 0.0f, rm = 0.0f;
-    int ridx = P.nobj + lane;
-    int rsk = -1;  // lane k: voxel k of the group skipped (1), updated (0), absent (-1)
+        for (int k = 0; k < G; k++)
+          bnb[k] = fetch(__builtin_amdgcn_readlane(pv, G + k), __builtin_amdgcn_readlane(lv, G + k));
+      }
+      const int left = cnt - n;
 #pragma unroll
-    for (int s = 0; s < G; s++) {
-      const int pix = apix[s];
-      const int n = (g - 1) * G + s;
-      const int par = n & 1;
-      if (pix == kNoPix) {  // only past the end of the sequence
-        if (PAD && g > 0) {
-          if (lane == 0) {
-            S.pr[par][0] = 1.0f;
-            S.pr[par][1] = 0.0f;
-            S.pr[par][2] = 0.0f;
-            S.pr[par][3] = 1.0f;
+      for (int s = 0; s < G; s++) {
+        const int par = s & 1;
+        if (s >= left) {  // past the end of the sequence
+          if (PAD && s > 0) {
+            for (int t = s; t < G; t++) {
+              if (lane == 0) {
+                S.pr[t & 1][0] = 1.0f;
+                S.pr[t & 1][1] = 0.0f;
+                S.pr[t & 1][2] = 0.0f;
+                S.pr[t & 1][3] = 1.0f;
+              }
+              __syncthreads();
+            }
           }
-          __syncthreads();
+          return;
         }
-        continue;
-      }
-      const float nbv = anb[s];
-      const bool vld = (nbv == nbv) & (lane != 13);
-      const float V = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nbv), 13));
-      const bool anypos = __ballot((lane != 13) & (nbv > 0.0f)) != 0ull;
-      const float dlt = vld ? V - nbv : 0.0f;
-      const float t1 =
-          __builtin_amdgcn_exp2f(0.8f * __builtin_amdgcn_logf(fabsf(dlt))) * nisqp;
-      const float t3 = nc + t1;
-      const float b = fmaf(1.2f, t1, two_c) * __builtin_amdgcn_rcpf(t3 * t3 * nsq);
-      const float gb = (vld ? ng : 0.0f) * b;
-      float pb = gb, pbx = -gb * dlt;
-      lo32_total_ff(pb, pbx);  // neighbour lanes are 0..28
-      const bool skip = (V == 0.0f) && iter > 1 && !anypos;
-      if (lane == 0) {
-        S.pr[par][0] = pb;
-        S.pr[par][1] = pbx;
-        S.pr[par][2] = V;
-        S.pr[par][3] = skip ? 1.0f : 0.0f;
-      }
-      __syncthreads();
-      float Vs;
-      bool sk;
-      const float xn = solve_step<MAXTH>(P, S, par, nth, &Vs, &sk);
-      const float dx = xn - V;
-      // (dy + 1) * 65536 + (dx + 1) with |dy|, |dx| <= 1 for a neighbour
-      const unsigned dd = (unsigned)(pend - pix + 65537);
-      const bool adj = (pend != kNoPix) & (dd != 65537u) & ((dd & 0xffffu) <= 2u) &
-                       (dd <= 131074u);
-      if (__ballot(adj) != 0ull) {
+        const int pix = __builtin_amdgcn_readlane(pv, s), lin = __builtin_amdgcn_readlane(lv, s);
+        const float nbv = anb[s];
+        const bool vld = (nbv == nbv) & neighb;
+        const float V = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(nbv), 13));
+        const float dlt = vld ? V - nbv : 0.0f;
+        const float t1 =
+            __builtin_amdgcn_exp2f(0.8f * __builtin_amdgcn_logf(fabsf(dlt))) * nisqp;
+        const float t3 = nc + t1;
+        const float b = fmaf(1.2f, t1, two_c) * __builtin_amdgcn_rcpf(t3 * t3 * nsq);
+        const float gb = (vld ? ng : 0.0f) * b;
+        float pb = gb, pbx = -gb * dlt;
+        lo32_last_ff(pb, pbx);  // neighbour lanes are 0..28
+        float skip = 0.0f;
+        if (iter > 1 && V == 0.0f) {
+          if (__builtin_amdgcn_ballot_w64(neighb & (nbv > 0.0f)) == 0ull) {
+            skip = 1.0f;
+            nzero++;
+          }
+        }
+        if (lane == 31) {
+          S.pr[par][0] = pb;
+          S.pr[par][1] = pbx;
+          S.pr[par][2] = V;
+          S.pr[par][3] = skip;
+        }
+        __syncthreads();
+        float Vs;
+        bool sk;
+        const float xn = solve_step<MAXTH>(P, S, par, nth, &Vs, &sk);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(xn), objc, voff, lin * 4, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(fabsf(xn - V)), magc, voff, lin * 4, 0);
+        vm[s] += fabs((double)xn);  // a skipped voxel's xn is zero
+        // among the voxels in flight, lanes s + 1 .. (one vector test per
+        // update): (dy + 1) * 65536 + (dx + 1) with |dy|, |dx| <= 1 for a
+        // neighbour; 3 passes too, the patch itself is exact
+        const unsigned near = (unsigned)__builtin_amdgcn_ballot_w64(
+            ((pend - (unsigned)pix) & 0xfffcfffcu) == 0u);
+        if (near & (RING ? 0x7fu << (s + 1) : 0xffffu & (0xfffeu << s))) {
 #pragma unroll
-        for (int o = s + 1; o < G; o++) anb[o] = anid[o] == pix ? xn : anb[o];
-#pragma unroll
-        for (int o = 0; o < G; o++) bnv[o] = bnid[o] == pix ? xn : bnv[o];
+          for (int o = 0; o < G; o++) {
+            if (RING ? o != s : o > s) {
+              const int po = __builtin_amdgcn_readlane(pv, RING && o < s ? G + o : o);
+              anb[o] = pix - po == poff ? xn : anb[o];
+            }
+            if (!RING) bnb[o] = pix - __builtin_amdgcn_readlane(pv, G + o) == poff ? xn : bnb[o];
+          }
+        }
+        if (RING)
+          anb[s] = fetch(__builtin_amdgcn_readlane(pv, G + s), __builtin_amdgcn_readlane(lv, G + s));
       }
-      const int lin = cbase + (pix >> 16) * P.N_x + (pix & 0xffff);
-      rx = lane == s ? xn : rx;
-      rm = lane == s ? (skip ? 0.0f : fabsf(dx)) : rm;
-      ridx = lane == s ? lin : ridx;
-      rsk = lane == s ? (skip ? 1 : 0) : rsk;
+      if (!RING) {
+#pragma unroll
+        for (int k = 0; k < G; k++) anb[k] = bnb[k];
+      }
+      pv = pvn;
+      lv = lin_of(pv);
     }
-    // the group's update counts and |x| sums (updateVoxels_Atten's return
-    // value, XT_VoxUpdate.c:263-281), lane by lane
-    vmacc += (count_mag && rsk == 0) ? fabs((double)rx) : 0.0;
-    nupd += (unsigned long long)__popcll(__ballot(rsk == 0));
-    nzero += (unsigned long long)__popcll(__ballot(rsk == 1));
-    wait_vm_all();
-    P.obj[(unsigned)ridx] = rx;
-    P.mag[(unsigned)ridx] = rm;
+  };
+  sweep();
+  // updateVoxels_Atten's return value (XT_VoxUpdate.c:263-281)
+  double vmacc = 0.0;
 #pragma unroll
-    for (int k = 0; k < G; k++) {
-      apix[k] = bpix[k];
-      anid[k] = bnid[k];
-      anb[k] = bnv[k] == bnv[k] ? bnv[k] : bnb[k];
-    }
-    // B moves to lanes 0..G-1
-    pend = __shfl(pend, (lane + G) & 63);
-    pend = lane < G ? pend : kNoPix;
-#pragma unroll
-    for (int k = 0; k < G; k++)
-      pnext[k] = (g + 1) * G + k < cnt ? __builtin_amdgcn_readlane(raw, k) : kNoPix;
-  }
-  const double voxmag = wave_sum_d(vmacc);
+  for (int k = 0; k < G; k++) vmacc = lane == k ? vm[k] : vmacc;
+  const double voxmag = wave_sum_d(count_mag ? vmacc : 0.0);
   if (lane == 0 && seq != 2) {
     P.cell_voxmag[cell] += voxmag;
-    P.cell_upd[cell] += nupd;
-    P.cell_zero[cell] += nzero;
+    P.cell_upd[cell] += (unsigned long long)(cnt - nzero);
+    P.cell_zero[cell] += (unsigned long long)nzero;
   }
 }
 
@@ -789,212 +886,157 @@ __device__ __forceinline__ void k_icd_mw_body(const KP &P, const int2 cl, int it
   if (wave < nth) {
     // ---------------- theta wave ----------------
     // Lane layer k holds the entry (view q_k, bin w0 + ub, row mm) of the
-    // current voxel; its A value and w0 come from the column table,
-    // prefetched one group of G voxels ahead.  The next voxel's (e, w) is
-    // read before this voxel's e is written and corrected afterwards by
-    // a(this voxel, that bin) * dx: the same fma the lane owning that entry
-    // stores, so no bits change.
+    // current voxel; its A value and w0 come from the column table, loaded
+    // G voxels ahead into the registers of the voxel that has just left (the
+    // unrolled loop is the ring).  The next voxel's (e, w) is read before
+    // this voxel's e is written, while the sums are published, and corrected
+    // afterwards by a(this voxel, that bin) * dx, a from the lane that owns
+    // that entry: the same fma that lane stores, so no bits change.
     const int lq = lane / EPV, ent = lane - lq * EPV;
     const int ub = ent / MZ, mm = ent - ub * MZ;
-    bool active[VPL];
-    int qv[VPL], dummy[VPL];
+    int idle[VPL];            // -1 in a lane without a view, else 0
+    int ebase[VPL], dummy[VPL];
+    unsigned oa[VPL], ow[VPL];  // byte offsets of the A value and w0 in a pixel's records
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
       const int qq = k * VW + lq, q = wave * vpw + qq;
-      active[k] = (lq < VW) & (qq < vpw) & (q < nv);
-      qv[k] = active[k] ? q : 0;
+      const bool active = (lq < VW) & (qq < vpw) & (q < nv);
+      const int qv = active ? q : 0;
+      idle[k] = active ? 0 : -1;
+      ebase[k] = qv * RS + ub * MZ + mm;
       dummy[k] = rows + (wave * VPL + k) * 64 + lane;
+      oa[k] = (unsigned)(qv * REC + ub) * 4u;
+      ow[k] = (unsigned)(qv * REC + NB) * 4u;
     }
-    const float4 *colt = reinterpret_cast<const float4 *>(P.colt);
-    const size_t fbase = (size_t)f * Nxy;
-    struct Rec {
-      float a[NB];
-      int w0;
+    const HuberBand hb = huber_band(P);
+    const char *tab = reinterpret_cast<const char *>(P.colt) +
+                      (size_t)f * Nxy * P.colt_nv * (REC * 4);
+    // address of the records of a packed pixel
+    auto rec_at = [&](int pix) -> unsigned long long {
+      const unsigned lin = (unsigned)((pix >> 16) * P.N_x + (pix & 0xffff));
+      return (unsigned long long)tab +
+             (unsigned long long)lin * (unsigned)(P.colt_nv * (REC * 4));
     };
-    auto load = [&](int pix, int k) -> Rec {
-      const bool valid = pix != kNoPix;
-      const int lin = valid ? (pix >> 16) * P.N_x + (pix & 0xffff) : 0;
-      const size_t r = ((fbase + lin) * P.colt_nv + qv[k]) * (REC / 4);
-      Rec o;
-      const float4 r0 = colt[r];
-      if (REC == 4) {
-        o.a[0] = r0.x;
-        o.a[1] = r0.y;
-        o.a[2] = r0.z;
-        o.w0 = __float_as_int(r0.w);
-      } else {
-        const float4 r1 = colt[r + 1];
-        const float v[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-#pragma unroll
-        for (int t = 0; t < NB; t++) o.a[t] = v[t];
-        o.w0 = __float_as_int(v[NB]);
-      }
-      // no arithmetic on the loaded registers here: any would make the
-      // compiler wait for the load at once; validity is applied at use
-      return o;
-    };
-    auto pick = [&](const Rec &r, int j) -> float {
-      float v = 0.0f;
-#pragma unroll
-      for (int t = 0; t < NB; t++) v = j == t ? r.a[t] : v;
-      return v;
-    };
-    // w0 of a record as this lane uses it: -1 for an empty slot or a lane
-    // without a view
-    auto w0_of = [&](const Rec &r, int pix, int k) -> int {
-      return (active[k] & (pix != kNoPix)) ? r.w0 : -1;
-    };
-    auto entry_at = [&](int w0, int k) -> int {
-      return w0 >= 0 ? qv[k] * RS + (w0 + ub) * MZ + mm : dummy[k];
-    };
-
-    int apix[G], bpix[G];
-    Rec arec[G][VPL], brec[G][VPL];
-    const int ngroups = (cnt + G - 1) / G;
-    int raw = list[n0 + min(lane, cnt - 1)];
-    int pnext[G];
-#pragma unroll
-    for (int j = 0; j < G; j++) pnext[j] = j < cnt ? __builtin_amdgcn_readlane(raw, j) : kNoPix;
-#pragma unroll
-    for (int j = 0; j < G; j++) {
-      apix[j] = kNoPix;
+    float ra[G][VPL];  // A value and w0 of voxels n .. n + G - 1
+    int rw[G][VPL];
+    auto load = [&](unsigned long long at, int j, float (&a)[VPL], int (&w0)[VPL]) {
+      const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)at, j);
+      const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(at >> 32), j);
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<void *>(((unsigned long long)hi << 32) | lo), (short)0,
+          P.colt_nv * (REC * 4), 0x00020000);
 #pragma unroll
       for (int k = 0; k < VPL; k++) {
-        arec[j][k].w0 = -1;
-#pragma unroll
-        for (int t = 0; t < NB; t++) arec[j][k].a[t] = 0.0f;
+        a[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, oa[k], 0, 0));
+        w0[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(r, ow[k], 0, 0);
       }
-    }
-    // current voxel's entries: A value, (e, w) with e already corrected for
-    // the previous voxel's update, LDS slot, window start and record
+    };
+    // current voxel's A value, window start, (e, w) and LDS slot
     float ca[VPL], ce[VPL], cwv[VPL];
     int cat[VPL], cw0[VPL];
-    Rec crec[VPL];
+    auto slot = [&](int j, float (&a)[VPL], int (&w0)[VPL], int (&at)[VPL]) {
+#pragma unroll
+      for (int k = 0; k < VPL; k++) {
+        w0[k] = rw[j][k] | idle[k];
+        at[k] = w0[k] >= 0 ? ebase[k] + w0[k] * MZ : dummy[k];
+        a[k] = w0[k] >= 0 ? ra[j][k] : 0.0f;
+      }
+    };
+    const int lane0 = lq * EPV + mm;  // the lane of the view's first bin
+    const int raw0 = list[n0 + min(lane, cnt - 1)];
+    int raw = list[n0 + min(G + lane, cnt - 1)];  // issued in the order of the loop
+    {
+      const unsigned long long at = rec_at(raw0);
+#pragma unroll
+      for (int j = 0; j < G; j++) {
+        __builtin_amdgcn_sched_barrier(0);
+        load(at, j, ra[j], rw[j]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot(0, ca, cw0, cat);
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
-      ca[k] = 0.0f;
-      ce[k] = 0.0f;
-      cwv[k] = 0.0f;
-      cat[k] = dummy[k];
-      cw0[k] = -1;
-      crec[k] = arec[0][k];
+      const float2 ew = s_ew[cat[k]];
+      ce[k] = ew.x;
+      cwv[k] = ew.y;
     }
-    unsigned nent = 0;  // entries with a > 0 (at most 2 x 65535 x 3 per lane)
-    for (int g = 0; g <= ngroups; g++) {
+    int nent = 0;  // entries with a > 0 (at most 2 x 65535 x 3 per lane)
+    auto sweep = [&] {  // left by its end alone, as prior_wave's
+      for (int n = 0;; n += G) {
+        // the next group's records; past the end the last voxel's, which are
+        // read and not used
+        const unsigned long long at = rec_at(raw);
+        raw = list[n0 + min(n + 2 * G + lane, cnt - 1)];
+        const int left = cnt - n;
 #pragma unroll
-      for (int j = 0; j < G; j++) {
-        bpix[j] = pnext[j];
-#pragma unroll
-        for (int k = 0; k < VPL; k++) brec[j][k] = load(pnext[j], k);
-      }
-      raw = list[n0 + min((g + 1) * G + lane, cnt - 1)];
-#pragma unroll
-      for (int s = 0; s < G; s++) {
-        const int pix = apix[s];
-        if (pix == kNoPix) continue;  // only past the end of the sequence
-        const int n = (g - 1) * G + s;
-        const int par = n & 1;
-        // this voxel's partial sums (XT_VoxUpdate.c:61-92)
-        double t1;
-        float t2;
-        // generalized-Huber weights (XT_VoxUpdate.c:66-80): w inside the
-        // threshold, T delta sqrt(w) / |e| outside; the outer weight is
-        // evaluated only when some lane of the wave needs it
-        float cwk[VPL];
-        bool sel[VPL], allsel = true;
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          sel[k] = huber_sel(P, ce[k], cwv[k]);
-          cwk[k] = cwv[k];
-          allsel &= sel[k];
-        }
-        if (__builtin_expect(__ballot(!allsel) != 0ull, 0)) {
+        for (int s = 0; s < G; s++) {
+          const int par = s & 1;
+          // this voxel's partial sums (XT_VoxUpdate.c:61-92)
+          float cwk[VPL];
+          huber_weights<VPL>(P, hb, ce, cwv, cwk);
+          double t1;
+          float t2;
 #pragma unroll
           for (int k = 0; k < VPL; k++) {
-            const float cw_out =
-                P.Td * __builtin_amdgcn_sqrtf(cwv[k]) * __builtin_amdgcn_rcpf(fabsf(ce[k]));
-            cwk[k] = sel[k] ? cwv[k] : cw_out;
+            const float ac = ca[k] * cwk[k];
+            const double p1 = (double)(-ce[k] * ac);
+            t1 = k == 0 ? p1 : t1 + p1;
+            t2 = k == 0 ? ca[k] * ac : fmaf(ca[k], ac, t2);
           }
-        }
+          wave_last_df(t1, t2);
+          if (lane == 63) {
+            S.t1[par][wave] = t1;
+            S.t2[par][wave] = t2;
+          }
+          float na[VPL], cn[VPL];
+          int nw0[VPL], nat[VPL];
+          float2 ewn[VPL];
+          slot((s + 1) % G, na, nw0, nat);
 #pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          const float cw = cwk[k];
-          const float ac = ca[k] * cw;
-          const double p1 = (double)(-ce[k] * ac);
-          const float p2 = ca[k] * ac;
-          t1 = k == 0 ? p1 : t1 + p1;
-          t2 = k == 0 ? p2 : t2 + p2;
-          nent += ca[k] > 0.0f ? 1u : 0u;
-        }
-        // the next voxel's entries and their (e, w), read before this
-        // voxel's e is written; independent of the sums, so they fill the
-        // reduction's latency
-        const int npix = s + 1 < G ? apix[s + 1] : bpix[0];
-        int nw0[VPL], nat[VPL];
-        float2 ewn[VPL];
-        float cn_prev[VPL], na[VPL];
+          for (int k = 0; k < VPL; k++) {
+            ewn[k] = s_ew[nat[k]];
+            // the next voxel's bin in this voxel's window; a voxel off the
+            // detector has w0 = -1 and A = 0
+            const int d = nw0[k] + (ub - cw0[k]);
+            const float av = __int_as_float(
+                __builtin_amdgcn_ds_bpermute((lane0 + d * MZ) * 4, __float_as_int(ca[k])));
+            cn[k] = (nw0[k] >= 0) & ((unsigned)d < (unsigned)NB) ? av : 0.0f;
+          }
+          __syncthreads();
+          float V;
+          bool skip;
+          const float xn = solve_step<MAXTH>(P, S, par, nth, &V, &skip, [&] {
+            // issued here, in the latency of the sums' read
+            __builtin_amdgcn_sched_barrier(0);
+            load(at, s, ra[s], rw[s]);
 #pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          const Rec &nr = s + 1 < G ? arec[s + 1][k] : brec[0][k];
-          nw0[k] = w0_of(nr, npix, k);
-          nat[k] = entry_at(nw0[k], k);
-          ewn[k] = s_ew[nat[k]];
-          const int d = nw0[k] + ub - cw0[k];  // the next voxel's bin in this voxel's window
-          const float pd = pick(crec[k], d), pu = pick(nr, ub);
-          cn_prev[k] = ((nw0[k] >= 0) & (cw0[k] >= 0)) ? pd : 0.0f;
-          na[k] = nw0[k] >= 0 ? pu : 0.0f;
-          // computed here, not sunk past the barrier onto the critical path
-          asm volatile("" ::"v"(cn_prev[k]), "v"(na[k]), "v"(nat[k]));
-        }
-        wave_total_df(t1, t2);
-        if (lane == 0) {
-          S.t1[par][wave] = t1;
-          S.t2[par][wave] = t2;
-        }
-        __syncthreads();
-        float V;
-        bool skip;
-        const float xn = solve_step<MAXTH>(P, S, par, nth, &V, &skip);
-        const float dx = xn - V;
+            for (int k = 0; k < VPL; k++) {
+              asm volatile("" ::"v"(cn[k]));
+              nent += ca[k] > 0.0f ? 1 : 0;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          });
+          const float dx = xn - V;
 #pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          s_ew[cat[k]].x = fmaf(-ca[k], dx, ce[k]);
-          ce[k] = fmaf(-cn_prev[k], dx, ewn[k].x);
-          cwv[k] = ewn[k].y;
-          crec[k] = s + 1 < G ? arec[s + 1][k] : brec[0][k];
-          cw0[k] = nw0[k];
-          ca[k] = na[k];
-          cat[k] = nat[k];
+          for (int k = 0; k < VPL; k++) {
+            s_ew[cat[k]].x = fmaf(-ca[k], dx, ce[k]);
+            ce[k] = fmaf(-cn[k], dx, ewn[k].x);
+            cwv[k] = ewn[k].y;
+            ca[k] = na[k];
+            cw0[k] = nw0[k];
+            cat[k] = nat[k];
+          }
+          if (s + 1 >= left) return;
         }
       }
-#pragma unroll
-      for (int j = 0; j < G; j++) {
-        apix[j] = bpix[j];
-#pragma unroll
-        for (int k = 0; k < VPL; k++) arec[j][k] = brec[j][k];
-      }
-#pragma unroll
-      for (int j = 0; j < G; j++)
-        pnext[j] = (g + 1) * G + j < cnt ? __builtin_amdgcn_readlane(raw, j) : kNoPix;
-      if (g == 0) {
-        // the first voxel's entries
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          crec[k] = arec[0][k];
-          cw0[k] = w0_of(crec[k], apix[0], k);
-          ca[k] = cw0[k] >= 0 ? pick(crec[k], ub) : 0.0f;
-          cat[k] = entry_at(cw0[k], k);
-          const float2 ew0 = s_ew[cat[k]];
-          ce[k] = ew0.x;
-          cwv[k] = ew0.y;
-        }
-      }
-    }
+    };
+    sweep();
     const double ne = wave_sum_d((double)nent);
     if (lane == 0) S.nent[wave] = (unsigned long long)ne;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, true>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
 
   // e back to global memory; entry count
@@ -1273,7 +1315,7 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
             }
             nent += ca[k] > 0.0f ? MZ : 0;
           }
-          wave_total_df(t1, t2);
+          wave_last_df(t1, t2);
         } else {
           // FP32 sums: compensated (TF 1) or plain (TF 2)
           float s1 = 0.f, c1 = 0.f, s2 = 0.f, c2 = 0.f;
@@ -1306,7 +1348,7 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
             t2 = s2;
           }
         }
-        if (lane == 0) {
+        if (lane == 63) {
           S.t1[par][wave] = t1;
           S.t2[par][wave] = t2;
         }
@@ -1353,7 +1395,7 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, false>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
   __syncthreads();
   if (threadIdx.x == 0 && seq != 2) {
@@ -1609,8 +1651,8 @@ __global__ __launch_bounds__(64 * (MAXTH + 1)) void k_icd_mwd(KP P, const int2 *
           }
           nent += qa[0][k] > 0.0f ? MZ : 0;
         }
-        wave_total_df(t1, t2);
-        if (lane == 0) {
+        wave_last_df(t1, t2);
+        if (lane == 63) {
           S.t1[par][wave] = t1;
           S.t2[par][wave] = t2;
         }
@@ -1665,7 +1707,7 @@ __global__ __launch_bounds__(64 * (MAXTH + 1)) void k_icd_mwd(KP P, const int2 *
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH, true>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, false, true>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
   __syncthreads();
   if (threadIdx.x == 0 && seq != 2) {
@@ -2031,8 +2073,8 @@ __global__ __launch_bounds__(64 * (MAXTH + 1)) void k_icd_bat(KP P, const int2 *
           double p1;
           float p2;
           terms(a[i], v, wv[i], huber_sel(P, v, wv[i]), p1, p2);
-          wave_total_df(p1, p2);
-          if (lane == 0) {
+          wave_last_df(p1, p2);
+          if (lane == 63) {
             S.t1[wave][0] = p1;
             S.f[wave][0] = p2;
           }
@@ -2427,8 +2469,8 @@ __device__ __forceinline__ void k_icd_wide_body(const KP &P, const int2 cl, int 
         }
         nent += a[j] > 0.0f ? R : 0;
       }
-      wave_total_df(t1, t2);
-      if (lane == 0) {
+      wave_last_df(t1, t2);
+      if (lane == 63) {
         S.t1[par][wave] = t1;
         S.t2[par][wave] = t2;
       }
@@ -2454,7 +2496,7 @@ __device__ __forceinline__ void k_icd_wide_body(const KP &P, const int2 cl, int 
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, false>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
   __syncthreads();
   if (threadIdx.x == 0 && seq != 2) {
@@ -2650,8 +2692,8 @@ __global__ __launch_bounds__(64 * (MAXTH + 1)) void k_icd_split(KP P, const int2
         }
         nent += ac[j] > 0.0f ? R : 0;
       }
-      wave_total_df(t1, t2);
-      if (lane == 0) {
+      wave_last_df(t1, t2);
+      if (lane == 63) {
         S.t1[par][wave] = t1;
         S.t2[par][wave] = t2;
       }
@@ -3064,8 +3106,8 @@ __device__ __forceinline__ void k_icd_wpass_body(const KP &P, const int2 cl, int
           nent += a[p] > 0.0f ? R : 0;
         }
       }
-      wave_total_df(t1, t2);
-      if (lane == 0) {
+      wave_last_df(t1, t2);
+      if (lane == 63) {
         S.t1[par][wave] = t1;
         S.t2[par][wave] = t2;
       }
@@ -3093,7 +3135,7 @@ __device__ __forceinline__ void k_icd_wpass_body(const KP &P, const int2 cl, int
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, false>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
   __syncthreads();
   if (threadIdx.x == 0 && seq != 2) {
@@ -3278,8 +3320,8 @@ __device__ __forceinline__ void k_icd_wloop_body(const KP &P, const int2 cl, int
           nent += a[p] > 0.0f ? R : 0;
         }
       }
-      wave_total_df(t1, t2);
-      if (lane == 0) {
+      wave_last_df(t1, t2);
+      if (lane == 63) {
         S.t1[par][wave] = t1;
         S.t2[par][wave] = t2;
       }
@@ -3318,7 +3360,7 @@ __device__ __forceinline__ void k_icd_wloop_body(const KP &P, const int2 cl, int
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
     // ---------------- prior wave ----------------
-    prior_wave<MAXTH>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
+    prior_wave<MAXTH, false>(P, S, list, n0, cnt, f, z, iter, seq, count_mag, nth, lane);
   }
   __syncthreads();
   if (threadIdx.x == 0 && seq != 2) {
