@@ -107,24 +107,27 @@ __device__ __forceinline__ void wait_vm_all() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// Generalized-Huber selection b = |e sqrt(w)| < T (XT_VoxUpdate.c:108-111)
-// decided exactly: e^2 w is carried as q + (error terms) with FMA residuals
-// and compared with T^2 = T2h + T2l, so the outcome is the exact one (the
-// reference's double evaluation differs from it only within 1e-16 of T).
+// Generalized-Huber selection b = |e sqrt(w)| < T (XT_VoxUpdate.c:108-111):
+// e^2 w with the FMA residuals of its two products, against T^2 = T2h + T2l.
+// The product's own residual stands in both terms, so the decision is that of
+// e^2 w within 2^-24 of it (the reference's double evaluation is within
+// 2^-52).  Written out as fused operations: the entries it decides are part
+// of the result's bits, whatever the compiler contracts around it.
 __device__ __forceinline__ bool huber_sel(const KP &P, float e, float w) {
+#pragma clang fp contract(off)
   const float p = e * e;
   const float pe = fmaf(e, e, -p);
   const float q = p * w;
   const float qe = fmaf(p, w, -q);
   const float corr = fmaf(pe, w, qe);
-  return (q - P.T2h) + (corr - P.T2l) < 0.0f;
+  return fmaf(p, w, -P.T2h) + (corr - P.T2l) < 0.0f;
 }
 
 // Generalized-Huber weights (XT_VoxUpdate.c:66-80) of N entries of a lane:
 // w inside the threshold, T delta sqrt(w) / |e| outside.  The rounded e^2 w
-// decides wherever it is off T^2 by more than its own error (2^-22 of it;
-// the band is four times that, and 2^-20 for what underflow loses), and
-// huber_sel inside the band.  The outer weight is evaluated only when some
+// decides wherever it is off T^2 by more than its own error and huber_sel's
+// (2^-22 of it; the band is four times that, and 2^-20 for what underflow
+// loses), and huber_sel inside the band.  The outer weight is evaluated only when some
 // lane of the wave needs it.
 struct HuberBand {
   float lo, hi;
@@ -573,16 +576,32 @@ __device__ __forceinline__ int col_window(const KP &P, double u, int nb, int &lo
   hic = min(lo + 2 * m, P.N_r - 1);
   return on ? min(loc, P.N_r - nb) : -1;
 }
-__device__ __forceinline__ float col_value(const KP &P, const float *H, double u, int j, int loc,
+// The value at bin j in two steps, the response's two samples loaded in the
+// first, so that a caller may let the load's latency pass between them.
+struct ColVal {
+  float h0, h1, fr;
+  bool ok;
+};
+__device__ __forceinline__ ColVal col_load(const KP &P, const float *H, double u, int j, int loc,
                                            int hic) {
 #pragma clang fp contract(off)
+  ColVal c;
   const double t = fabs(u - ((double)j + 0.5)) * P.u_kk;
   const int bin = (int)t;
-  const bool ok = (j >= loc) & (j <= hic) & (bin < kRespBins);
-  const int bb = ok ? bin : 0;
-  const float fr = (float)(t - (double)bin);
-  const float h0 = H[bb], h1 = H[bb + 1];
-  return fmaf(fr, h1 - h0, h0) * (ok ? 1.0f : 0.0f);
+  c.ok = (j >= loc) & (j <= hic) & (bin < kRespBins);
+  const int bb = c.ok ? bin : 0;
+  c.fr = (float)(t - (double)bin);
+  c.h0 = H[bb];
+  c.h1 = H[bb + 1];
+  return c;
+}
+__device__ __forceinline__ float col_lerp(const ColVal &c) {
+#pragma clang fp contract(off)
+  return fmaf(c.fr, c.h1 - c.h0, c.h0) * (c.ok ? 1.0f : 0.0f);
+}
+__device__ __forceinline__ float col_value(const KP &P, const float *H, double u, int j, int loc,
+                                           int hic) {
+  return col_lerp(col_load(P, H, u, j, loc, hic));
 }
 
 // Column table of the multi-wavefront kernel: for every (frame, pixel, view
@@ -1097,12 +1116,21 @@ template __global__ void k_icd_mw_m<5, 2, 2, 3>(const KP *, const int4 *, int, i
 // prior wave is the same.  A lane holds one (view, bin) of the voxel's column
 // with all MZ detector rows of the slice, which are contiguous in the
 // [N_z][N_p][N_r][mz] layout, for VPL views.  Per voxel n a lane:
-//   issues the column-table entry (a, w0) of voxel n + 2 and the (e, w) rows
-//   of voxel n + 1 (addressed by the w0 that arrived during voxel n - 1),
+//   issues the (e, w) rows of voxel n + 1 and the column-table entry (a, w0)
+//   of a voxel RD + 2 places on, into the registers of the entry it has just
+//   taken (or, where A comes from the geometry, the response samples of
+//   voxel n + 3),
 //   reduces voxel n's theta sums, meets the other waves, solves,
-//   waits once for everything it issued, stores voxel n's e, and corrects
-//   voxel n + 1's e, read before that store, by a(voxel n, that bin) * dx:
-//   the same fma the lane owning the bin stores, so no bits change.
+//   stores voxel n's e, and corrects voxel n + 1's e, read before that store,
+//   by a(voxel n, that bin) * dx: the same fma the lane owning the bin
+//   stores, so no bits change.
+// What bounds it: the latency of those rows (L2, or the memory side for
+// large cells) and the theta chain, one after the other for each voxel; no
+// wait is explicit, so each covers its own load and the table's latency is
+// hidden altogether.  Before and after waiting for everything at each
+// voxel, a pass: 192 x 192, 5 bins x 2 rows, 128 views, 32 cells 60.8 and
+// 57.9 ms; twelve 128 x 128 and 192 x 192 problems of 180 views, 24 cells a
+// launch 72.3 and 66.9 ms; 512 x 512, 128 views, 256 cells 90.7 and 88.9 ms.
 // ---------------------------------------------------------------------------
 template <int MZ>
 __device__ __forceinline__ void ld_rows(const float *p, float (&o)[MZ]) {
@@ -1143,6 +1171,8 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
   constexpr int G = 8;             // pixels read per list load
   constexpr int VW = 64 / NB;      // views of one lane layer
   constexpr int REC = col_rec(NB);
+  // records in flight: as many as the registers of the lane's rows leave
+  constexpr int RD = VPL > 1 ? 2 : MZ <= 2 ? 8 : 4;
   __shared__ StepIn S;
   const int f = cl.x, z = cl.y;
   const int cell = f * P.N_z + z;
@@ -1174,160 +1204,180 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
   if (wave < nth) {
     // ---------------- theta wave ----------------
     const int lq = lane / NB, ub = lane - lq * NB;
+    const int lane0 = lq * NB;  // the lane of the view's first bin
     bool act[VPL];
-    int qv[VPL];
+    int idle[VPL];              // -1 in a lane without a view, else 0
     size_t ebase[VPL];
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-      const int qq = k * VW + lq, q = wave * vpw + qq;
-      act[k] = (lq < VW) & (qq < vpw) & (q < nv);
-      qv[k] = act[k] ? q : 0;
-      ebase[k] = sidx(P, z, nv > 0 ? P.view_idx[vb + qv[k]] : 0, ub, 0);
-    }
-    const float *colt = P.colt;
-    const size_t fbase = (size_t)f * Nxy;
-    auto rec_at = [&](int pix, int k) -> size_t {
-      const int lin = pix != kNoPix ? (pix >> 16) * P.N_x + (pix & 0xffff) : 0;
-      return ((fbase + lin) * (size_t)P.colt_nv + qv[k]) * REC;
-    };
-    // The shuffled (HICD) voxels of 3-bin columns, one view per lane, take
-    // their A value and window from the view's geometry in the lane, with
-    // the column table's own arithmetic (the same bits): their records
-    // would be 2 KB reads at random places of the table.  Raster-ordered
-    // lines read the table, and so do lanes of several views, for which the
-    // arithmetic costs more than the reads.
-    const bool calc = NB == 3 && VPL == 1 && seq == 0;
+    unsigned oa[VPL], ow[VPL];  // byte offsets of the A value and w0 in a pixel's records
     double cAu[VPL], cBu[VPL], cCu[VPL];
     const float *cH[VPL];
 #pragma unroll
     for (int k = 0; k < VPL; k++) {
-      const int v = nv > 0 ? P.view_idx[vb + qv[k]] : 0;
+      const int qq = k * VW + lq, q = wave * vpw + qq;
+      act[k] = (lq < VW) & (qq < vpw) & (q < nv);
+      const int qv = act[k] ? q : 0;
+      idle[k] = act[k] ? 0 : -1;
+      const int v = nv > 0 ? P.view_idx[vb + qv] : 0;
+      ebase[k] = sidx(P, z, v, ub, 0);
+      oa[k] = (unsigned)(qv * REC + ub) * 4u;
+      ow[k] = (unsigned)(qv * REC + NB) * 4u;
       col_coef(P, v, cAu[k], cBu[k], cCu[k]);
       cH[k] = P.hr + (size_t)v * kHrStride;
     }
-    auto col_at = [&](int pix, int k, float &a, int &w0) {
-      if (calc) {
-        const int yy = pix != kNoPix ? pix >> 16 : 0, xx = pix != kNoPix ? pix & 0xffff : 0;
-        const double u = col_u(xx, yy, cAu[k], cBu[k], cCu[k]);
-        int loc, hic;
-        w0 = col_window(P, u, NB, loc, hic);
-        a = w0 >= 0 ? col_value(P, cH[k], u, w0 + ub, loc, hic) : 0.0f;
-      } else {
-        const size_t r = rec_at(pix, k);
-        a = colt[r + ub];
-        w0 = __float_as_int(colt[r + NB]);
+    const HuberBand hb = huber_band(P);
+    const char *tab = reinterpret_cast<const char *>(P.colt) +
+                      (size_t)f * Nxy * P.colt_nv * (REC * 4);
+    // address of the records of a packed pixel
+    auto rec_at = [&](int pix) -> unsigned long long {
+      const unsigned lin = (unsigned)((pix >> 16) * P.N_x + (pix & 0xffff));
+      return (unsigned long long)tab +
+             (unsigned long long)lin * (unsigned)(P.colt_nv * (REC * 4));
+    };
+    auto rec_load = [&](unsigned long long at, int j, float (&a)[VPL], int (&w0)[VPL]) {
+      const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)at, j);
+      const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(at >> 32), j);
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<void *>(((unsigned long long)hi << 32) | lo), (short)0,
+          P.colt_nv * (REC * 4), 0x00020000);
+#pragma unroll
+      for (int k = 0; k < VPL; k++) {
+        a[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, oa[k], 0, 0));
+        w0[k] = (int)__builtin_amdgcn_raw_buffer_load_b32(r, ow[k], 0, 0);
       }
     };
-    const int *lst = list + n0;
-    auto pix_at = [&](int raw, int k, int n) -> int {
-      return n < cnt ? __builtin_amdgcn_readlane(raw, k) : kNoPix;
+    auto col_begin = [&](int pix, int k, int &w0) -> ColVal {
+      const double u = col_u(pix & 0xffff, pix >> 16, cAu[k], cBu[k], cCu[k]);
+      int loc, hic;
+      w0 = col_window(P, u, NB, loc, hic);
+      return col_load(P, cH[k], u, max(w0, 0) + ub, loc, hic);
     };
+    // lane k: the voxel k places on from the group's first (the last voxel
+    // past the end, whose loads are not used)
+    auto at_list = [&](int n) -> int { return list[n0 + min(n + lane, cnt - 1)]; };
+    int nent = 0;  // entries with a > 0, of MZ rows each
 
-    // voxel n ("c"): a, w0, (e corrected, w) rows and their address;
-    // voxel n + 1 ("n"): a, w0 arrived, (e, w) rows in flight
-    float ca[VPL], na[VPL], ce[VPL][MZ], cwv[VPL][MZ], ne[VPL][MZ], nwv[VPL][MZ];
-    int cw0[VPL], nw0[VPL];
-    size_t cea[VPL], nea[VPL];
-    int rawc = lst[min(lane, cnt - 1)];
-    int rawn = lst[min(G + lane, cnt - 1)];
-    wait_vm_all();
-    {
-      const int p0 = pix_at(rawc, 0, 0), p1 = pix_at(rawc, 1, 1);
-      float a0[VPL], a1[VPL];
-      int w00[VPL], w01[VPL];
+    // CALC: the A values and windows from the views' geometry, in the lane;
+    // else from the column table's records, RD voxels ahead in a ring
+    auto sweep = [&](auto calc_t) {
+      constexpr bool CALC = decltype(calc_t)::value;
+      // voxel n ("c"): a, w0, the corrected e and w rows and their place;
+      // voxel n + 1 ("n"): a, w0
+      float ca[VPL], na[VPL], ce[VPL * MZ], cwv[VPL * MZ];
+      int cw0[VPL], nw0[VPL];
+      size_t cea[VPL];
+      float ra[RD][VPL];  // records of voxels n + 2 .. n + RD + 1
+      int rw[RD][VPL];
+      ColVal pc[VPL];     // CALC: voxel n + 2's column, its samples in flight
+      int pw[VPL];
+      int pv = at_list(0);
+      int raw = at_list(G);
+      {
+        if constexpr (CALC) {
 #pragma unroll
-      for (int k = 0; k < VPL; k++) {
-        col_at(p0, k, a0[k], w00[k]);
-        col_at(p1, k, a1[k], w01[k]);
-      }
-      wait_vm_all();
+          for (int k = 0; k < VPL; k++) {
+            int w0, w1;
+            const ColVal c0 = col_begin(__builtin_amdgcn_readlane(pv, 0), k, w0);
+            const ColVal c1 = col_begin(__builtin_amdgcn_readlane(pv, 1), k, w1);
+            pc[k] = col_begin(__builtin_amdgcn_readlane(pv, 2), k, pw[k]);
+            cw0[k] = w0 | idle[k];
+            ca[k] = cw0[k] >= 0 ? col_lerp(c0) : 0.0f;
+            nw0[k] = w1 | idle[k];
+            na[k] = nw0[k] >= 0 ? col_lerp(c1) : 0.0f;
+          }
+        } else {
+          const unsigned long long at = rec_at(pv);
+          float a0[VPL], a1[VPL];
+          int w0[VPL], w1[VPL];
+          rec_load(at, 0, a0, w0);
+          rec_load(at, 1, a1, w1);
 #pragma unroll
-      for (int k = 0; k < VPL; k++) {
-        cw0[k] = act[k] ? w00[k] : -1;
-        ca[k] = cw0[k] >= 0 ? a0[k] : 0.0f;
-        const bool v1 = act[k] & (p1 != kNoPix);
-        nw0[k] = v1 ? w01[k] : -1;
-        na[k] = nw0[k] >= 0 ? a1[k] : 0.0f;
-        cea[k] = ebase[k] + (size_t)max(cw0[k], 0) * MZ;
-        ld_rows<MZ>(P.e + cea[k], ce[k]);
-        ld_rows<MZ>(P.w + cea[k], cwv[k]);
-      }
-      wait_vm_all();
-    }
-    int rawnn = rawn;
-    unsigned long long nent = 0;
-    const int ngroups = (cnt + G - 1) / G;
-    for (int g = 0; g < ngroups; g++) {
+          for (int j = 2; j < RD + 2; j++) {
+            __builtin_amdgcn_sched_barrier(0);
+            rec_load(at, j, ra[j % RD], rw[j % RD]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < G; s++) {
-        const int n = g * G + s;
-        if (n >= cnt) break;
-        const int par = n & 1;
-        if (s == 0) rawnn = lst[min((g + 2) * G + lane, cnt - 1)];
-        // issue: column entries of voxel n + 2, (e, w) rows of voxel n + 1
-        const int p2 = s + 2 < G ? pix_at(rawc, s + 2, n + 2) : pix_at(rawn, s + 2 - G, n + 2);
-        float a2[VPL];
-        int w2[VPL];
+          for (int k = 0; k < VPL; k++) {
+            cw0[k] = w0[k] | idle[k];
+            ca[k] = cw0[k] >= 0 ? a0[k] : 0.0f;
+            nw0[k] = w1[k] | idle[k];
+            na[k] = nw0[k] >= 0 ? a1[k] : 0.0f;
+          }
+        }
 #pragma unroll
         for (int k = 0; k < VPL; k++) {
-          col_at(p2, k, a2[k], w2[k]);
-          nea[k] = ebase[k] + (size_t)max(nw0[k], 0) * MZ;
-          ld_rows<MZ>(P.e + nea[k], ne[k]);
-          ld_rows<MZ>(P.w + nea[k], nwv[k]);
+          cea[k] = ebase[k] + (size_t)max(cw0[k], 0) * MZ;
+          float t[MZ];
+          ld_rows<MZ>(P.e + cea[k], t);
+#pragma unroll
+          for (int m = 0; m < MZ; m++) ce[k * MZ + m] = t[m];
+          ld_rows<MZ>(P.w + cea[k], t);
+#pragma unroll
+          for (int m = 0; m < MZ; m++) cwv[k * MZ + m] = t[m];
         }
-        // voxel n's theta sums (XT_VoxUpdate.c:61-92)
-        // generalized-Huber weights (XT_VoxUpdate.c:66-80); the outer
-        // weight only when some lane of the wave needs it
-        float cwk[VPL][MZ];
-        bool sel[VPL][MZ], allsel = true;
+      }
+      for (int n = 0;; n += G) {  // left by its end alone, as prior_wave's
+        unsigned long long at = 0;
+        if constexpr (!CALC) at = rec_at(pv);
+        const int pvn = raw;
+        raw = at_list(n + 2 * G);
+        const int left = cnt - n;
 #pragma unroll
-        for (int k = 0; k < VPL; k++)
-#pragma unroll
-          for (int m = 0; m < MZ; m++) {
-            sel[k][m] = huber_sel(P, ce[k][m], cwv[k][m]);
-            cwk[k][m] = cwv[k][m];
-            allsel &= sel[k][m];
-          }
-        if (__builtin_expect(__ballot(!allsel) != 0ull, 0)) {
-#pragma unroll
-          for (int k = 0; k < VPL; k++)
-#pragma unroll
-            for (int m = 0; m < MZ; m++) {
-              const float cw_out = P.Td * __builtin_amdgcn_sqrtf(cwv[k][m]) *
-                                   __builtin_amdgcn_rcpf(fabsf(ce[k][m]));
-              cwk[k][m] = sel[k][m] ? cwv[k][m] : cw_out;
-            }
-        }
-        double t1;
-        float t2;
-        if constexpr (TF == 0) {
+        for (int s = 0; s < G; s++) {
+          const int par = s & 1;
+          // issue: the (e, w) rows of voxel n + 1, then the record of voxel
+          // n + RD + 2 or the samples of voxel n + 3
+          float ne[VPL][MZ], nwv[VPL][MZ], na2[VPL];
+          size_t nea[VPL];
+          int nw2[VPL];
 #pragma unroll
           for (int k = 0; k < VPL; k++) {
-#pragma unroll
-            for (int m = 0; m < MZ; m++) {
-              const float e = ce[k][m];
-              const float cw = cwk[k][m];
-              const float ac = ca[k] * cw;
-              const double p1 = (double)(-e * ac);
-              const float p2 = ca[k] * ac;
-              t1 = (k == 0 && m == 0) ? p1 : t1 + p1;
-              t2 = (k == 0 && m == 0) ? p2 : t2 + p2;
-            }
-            nent += ca[k] > 0.0f ? MZ : 0;
+            nea[k] = ebase[k] + (size_t)max(nw0[k], 0) * MZ;
+            ld_rows<MZ>(P.e + nea[k], ne[k]);
+            ld_rows<MZ>(P.w + nea[k], nwv[k]);
           }
-          wave_last_df(t1, t2);
-        } else {
-          // FP32 sums: compensated (TF 1) or plain (TF 2)
-          float s1 = 0.f, c1 = 0.f, s2 = 0.f, c2 = 0.f;
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (CALC) {
 #pragma unroll
-          for (int k = 0; k < VPL; k++) {
+            for (int k = 0; k < VPL; k++) {
+              nw2[k] = pw[k] | idle[k];
+              na2[k] = nw2[k] >= 0 ? col_lerp(pc[k]) : 0.0f;
+              pc[k] = col_begin(__builtin_amdgcn_readlane(pv, s + 3), k, pw[k]);
+            }
+          } else {
 #pragma unroll
-            for (int m = 0; m < MZ; m++) {
-              const float e = ce[k][m];
-              const float cw = cwk[k][m];
-              const float ac = ca[k] * cw;
-              const float p1 = -e * ac;
-              const float p2 = ca[k] * ac;
+            for (int k = 0; k < VPL; k++) {
+              nw2[k] = rw[(s + 2) % RD][k] | idle[k];
+              na2[k] = nw2[k] >= 0 ? ra[(s + 2) % RD][k] : 0.0f;
+            }
+            rec_load(at, RD + s + 2, ra[(s + 2) % RD], rw[(s + 2) % RD]);
+          }
+          // voxel n's theta sums (XT_VoxUpdate.c:61-92)
+          float cwk[VPL * MZ];
+          huber_weights<VPL * MZ>(P, hb, ce, cwv, cwk);
+          double t1;
+          float t2;
+          if constexpr (TF == 0) {
+#pragma unroll
+            for (int i = 0; i < VPL * MZ; i++) {
+              const float a = ca[i / MZ], ac = a * cwk[i];
+              const double p1 = (double)(-ce[i] * ac);
+              t1 = i == 0 ? p1 : t1 + p1;
+              // theta2 fused in a fixed order (a part of the result's bits):
+              // of a lane's first two rows the second is rounded first
+              if (i == 0) t2 = a * ac;
+              else if (i == 1 && VPL == 1) t2 = fmaf(a, a * cwk[0], a * ac);
+              else t2 = fmaf(a, ac, t2);
+            }
+            wave_last_df(t1, t2);
+          } else {
+            // FP32 sums: compensated (TF 1) or plain (TF 2)
+            float s1 = 0.f, c1 = 0.f, s2 = 0.f, c2 = 0.f;
+#pragma unroll
+            for (int i = 0; i < VPL * MZ; i++) {
+              const float a = ca[i / MZ], ac = a * cwk[i];
+              const float p1 = -ce[i] * ac;
+              const float p2 = a * ac;
               if constexpr (TF == 1) {
                 cadd(s1, c1, p1);
                 cadd(s2, c2, p2);
@@ -1336,61 +1386,72 @@ __device__ __forceinline__ void k_icd_mwg_body(const KP &P, const int2 cl, int i
                 s2 += p2;
               }
             }
-            nent += ca[k] > 0.0f ? MZ : 0;
+            if constexpr (TF == 1) {
+              wave_total_cc(s1, c1, s2, c2);
+              t1 = (double)s1 + (double)c1;
+              t2 = s2 + c2;
+            } else {
+              wave_total_ff(s1, s2);
+              t1 = (double)s1;
+              t2 = s2;
+            }
           }
-          if constexpr (TF == 1) {
-            wave_total_cc(s1, c1, s2, c2);
-            t1 = (double)s1 + (double)c1;
-            t2 = s2 + c2;
-          } else {
-            wave_total_ff(s1, s2);
-            t1 = (double)s1;
-            t2 = s2;
+          if (lane == 63) {
+            S.t1[par][wave] = t1;
+            S.t2[par][wave] = t2;
           }
-        }
-        if (lane == 63) {
-          S.t1[par][wave] = t1;
-          S.t2[par][wave] = t2;
-        }
-        // a of this voxel at the bin each lane holds for voxel n + 1
-        float cn[VPL];
+          // a of this voxel at the bin each lane holds for voxel n + 1
+          float cn[VPL];
 #pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          const int d = nw0[k] + ub - cw0[k];
-          const bool ov = (nw0[k] >= 0) & (cw0[k] >= 0) & (d >= 0) & (d < NB);
-          const float av = __shfl(ca[k], lq * NB + (ov ? d : 0));
-          cn[k] = ov ? av : 0.0f;
-        }
-        __syncthreads();
-        float V;
-        bool skip;
-        const float xn = solve_step<MAXTH, TF>(P, S, par, nth, &V, &skip);
-        const float dx = xn - V;
-        wait_vm_all();
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-          if (ca[k] != 0.0f) {
-            float o[MZ];
-#pragma unroll
-            for (int m = 0; m < MZ; m++) o[m] = fmaf(-ca[k], dx, ce[k][m]);
-            st_rows<MZ>(P.e + cea[k], o);
+          for (int k = 0; k < VPL; k++) {
+            const int d = nw0[k] + (ub - cw0[k]);
+            const float av = __int_as_float(
+                __builtin_amdgcn_ds_bpermute((lane0 + d) * 4, __float_as_int(ca[k])));
+            cn[k] = (nw0[k] >= 0) & ((unsigned)d < (unsigned)NB) ? av : 0.0f;
+            nent += ca[k] > 0.0f ? 1 : 0;
           }
+          __syncthreads();
+          float V;
+          bool skip;
+          const float xn = solve_step<MAXTH, TF>(P, S, par, nth, &V, &skip);
+          const float dx = xn - V;
 #pragma unroll
-          for (int m = 0; m < MZ; m++) {
-            ce[k][m] = fmaf(-cn[k], dx, ne[k][m]);
-            cwv[k][m] = nwv[k][m];
+          for (int k = 0; k < VPL; k++) {
+            if (ca[k] != 0.0f) {
+              float o[MZ];
+#pragma unroll
+              for (int m = 0; m < MZ; m++) o[m] = fmaf(-ca[k], dx, ce[k * MZ + m]);
+              st_rows<MZ>(P.e + cea[k], o);
+            }
+#pragma unroll
+            for (int m = 0; m < MZ; m++) {
+              ce[k * MZ + m] = fmaf(-cn[k], dx, ne[k][m]);
+              cwv[k * MZ + m] = nwv[k][m];
+            }
+            ca[k] = na[k];
+            cw0[k] = nw0[k];
+            cea[k] = nea[k];
+            nw0[k] = nw2[k];
+            na[k] = na2[k];
           }
-          ca[k] = na[k];
-          cw0[k] = nw0[k];
-          cea[k] = nea[k];
-          const bool v2 = act[k] & (p2 != kNoPix);
-          nw0[k] = v2 ? w2[k] : -1;
-          na[k] = nw0[k] >= 0 ? a2[k] : 0.0f;
+          if constexpr (VPL > 1) {
+            // the rows of one voxel in flight, not two: more do not fit the
+            // registers
+#pragma unroll
+            for (int i = 0; i < VPL * MZ; i++) asm volatile("" : "+v"(ce[i]), "+v"(cwv[i]));
+          }
+          if (s + 1 >= left) return;
         }
+        pv = pvn;
       }
-      rawc = rawn;
-      rawn = rawnn;
+    };
+    if constexpr (NB == 3 && VPL == 1) {
+      if (seq == 0) sweep(std::true_type{});
+      else sweep(std::false_type{});
+    } else {
+      sweep(std::false_type{});
     }
+    nent *= MZ;
     const double nsum = wave_sum_d((double)nent);
     if (lane == 0) S.nent[wave] = (unsigned long long)nsum;
   } else {
