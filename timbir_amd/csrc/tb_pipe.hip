@@ -509,30 +509,61 @@ template <int MAXTH, int TF = 0, class F>
 __device__ __forceinline__ float solve_step(const KP &P, const StepIn &S, int par, int nth,
                                             float *V_out, bool *skip_out, F between) {
 #pragma clang fp contract(off)
-  // every slot is read at once (one LDS latency) and added as a fixed
-  // pairwise tree over the MAXTH slots; slots of absent waves hold zero
   using T1T = typename std::conditional<TF == 2, float, double>::type;
-  T1T a1[MAXTH];
-  float a2[MAXTH];
-#pragma unroll
-  for (int w = 0; w < MAXTH; w++) {
-    a1[w] = (T1T)S.t1[par][w];
-    a2[w] = S.t2[par][w];
-  }
-  const float pb = S.pr[par][0], pbx = S.pr[par][1], V = S.pr[par][2];
-  const bool skip = S.pr[par][3] != 0.0f;
-  between();
-#pragma unroll
-  for (int m = MAXTH; m > 1; m = (m + 1) / 2) {
-    const int h = (m + 1) / 2;
-#pragma unroll
-    for (int w = 0; w + h < m; w++) {
-      a1[w] = a1[w] + a1[w + h];
-      a2[w] = a2[w] + a2[w + h];
+  // the slots are added as a fixed pairwise tree over MAXTH; slots of absent
+  // waves hold zero
+  double T1;
+  float T2, pb, pbx, V;
+  bool skip;
+  if constexpr ((MAXTH == 8 || MAXTH == 15) && TF != 2) {
+    // A slot in each lane and the tree by rotations within the rows of 16
+    // lanes, whose sums repeat every 8, 4, 2 lanes: every lane ends with the
+    // same pairs' total.  Read whole by every lane, the slots are 12 reads of
+    // 16 bytes a lane in each of 10 or more waves and 28 sums in place of 2
+    // reads and 16 instructions (a pass, before and after: twelve problems of
+    // 180 views 66.9 and 62.3 ms, the 192 x 192 coarse stage 57.9 and 55.5).
+    const int sl = threadIdx.x & (MAXTH == 8 ? 7 : 15);
+    double a1 = S.t1[par][sl];
+    float a2 = S.t2[par][sl];
+    pb = S.pr[par][0], pbx = S.pr[par][1], V = S.pr[par][2];
+    skip = S.pr[par][3] != 0.0f;
+    between();
+    if constexpr (MAXTH == 15) {
+      a1 = a1 + dpp_d<0x128>(a1);  // row_ror:8
+      a2 = a2 + dpp_f<0x128>(a2);
     }
+    a1 = a1 + dpp_d<0x124>(a1);
+    a2 = a2 + dpp_f<0x124>(a2);
+    a1 = a1 + dpp_d<0x122>(a1);
+    a2 = a2 + dpp_f<0x122>(a2);
+    a1 = a1 + dpp_d<0x121>(a1);
+    a2 = a2 + dpp_f<0x121>(a2);
+    T1 = a1;
+    T2 = a2;
+  } else {
+    // every slot is read at once (one LDS latency)
+    T1T a1[MAXTH];
+    float a2[MAXTH];
+#pragma unroll
+    for (int w = 0; w < MAXTH; w++) {
+      a1[w] = (T1T)S.t1[par][w];
+      a2[w] = S.t2[par][w];
+    }
+    pb = S.pr[par][0], pbx = S.pr[par][1], V = S.pr[par][2];
+    skip = S.pr[par][3] != 0.0f;
+    between();
+#pragma unroll
+    for (int m = MAXTH; m > 1; m = (m + 1) / 2) {
+      const int h = (m + 1) / 2;
+#pragma unroll
+      for (int w = 0; w + h < m; w++) {
+        a1[w] = a1[w] + a1[w + h];
+        a2[w] = a2[w] + a2[w + h];
+      }
+    }
+    T1 = (double)a1[0];
+    T2 = a2[0];
   }
-  const double T1 = (double)a1[0];
-  const float T2 = a2[0];
   (void)nth;
   const float th1 = (float)T1;
   const float num = P.alpha * (pbx - th1);
