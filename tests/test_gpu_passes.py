@@ -107,3 +107,40 @@ def test_forward_projection_bitwise_at_the_edges(N, nz, shift, mxy, mz):
     st.close()
     np.testing.assert_array_equal(got, o.forward_project())
     assert np.abs(got).max() > 0
+
+
+@pytest.mark.parametrize("kind", ["ties", "wide"])
+@pytest.mark.parametrize("N", [3, 8, 16, 90, 91, 128, 129, 181, 182, 200])
+def test_line_selection_at_its_register_limits(N, kind):
+    """NHICD line lists of cells of 9 to 40000 pixels (a cell's pixels in 8,
+    16 or 32 registers a lane up to 90, 128 and 181 pixels a side, read again
+    beyond; ragged last steps) hold the order statistic of the filtered map: the
+    (N^2 - want)-th smallest is the threshold and the lines above it follow in
+    raster order, as the oracle's lists, entry for entry."""
+    from oracle import pyorc
+    print(f"line selection N={N} {kind}", flush=True)
+    s = datagen.tiny(N=N, nz=2, n_frames=1, n_views=4)
+    o = pyorc.Problem(s, opt=pyorc.options(schedule=pyorc.SCHED_COLOUR))
+    g = tb.Stage(s)
+    rng = np.random.default_rng(N)
+    mag = rng.random(o.obj_shape).astype(np.float32)
+    if kind == "ties":
+        mag = np.floor(mag * 2).astype(np.float32)
+        mag[..., : N // 2, :] = 0.0
+    else:
+        mag = np.exp(-60.0 * mag).astype(np.float32)
+    o.mag()[...] = mag
+    g.set_magmap(mag)
+    o.L.orc_set_select_counts(o.h, o.info["U"])
+    o.vsc_select()
+    g.vsc_select()
+    for z in range(o.info["N_z"]):
+        xo, yo = o.nhicd_list(0, z)
+        xg, yg = g.nhicd_list(0, z)
+        np.testing.assert_array_equal(xg, xo)
+        np.testing.assert_array_equal(yg, yo)
+    # the selection clears the map at selected pixels outside the mask (the
+    # oracle does when it reaches them) and nowhere else
+    changed = g.magmap() != mag
+    assert not changed[..., o.mask() == 1].any() and not g.magmap()[changed].any()
+    g.close()

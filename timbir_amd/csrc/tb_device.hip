@@ -70,6 +70,7 @@ __global__ void k_cost_data(KP, double *);
 __global__ void k_cost_prior(KP, double, double, double, double, double, double, const double *,
                              double, double *);
 __global__ void k_vsc_filter(KP, float *);
+template <int R>
 __global__ void k_vsc_select(KP, const float *, int);
 __global__ void k_mag_sum(KP, double *);
 __global__ void k_fill_f64(double *, size_t, double);
@@ -1552,8 +1553,14 @@ static int vsc_async(tb_stage *st) {
   hipLaunchKernelGGL(k_vsc_filter, dim3((st->N_x + 15) / 16, (st->N_y + 15) / 16, st->N_time * st->N_z),
                      dim3(256), 0, st->stream, P, st->filt);
   // NHICDSelectNum = floor(UpdateSelectNum / NHICD_Iterations), XT_NHICD.c:182
-  hipLaunchKernelGGL(k_vsc_select, dim3(st->N_time * st->N_z), dim3(1024), 0, st->stream, P,
-                     st->filt, st->U / kNhicdK);
+  // the cell's pixels in the registers of its 16 waves where they fit
+  const int nxy = st->N_x * st->N_y;
+  const auto select = nxy <= 8 * 1024    ? k_vsc_select<8>
+                      : nxy <= 16 * 1024 ? k_vsc_select<16>
+                      : nxy <= 32 * 1024 ? k_vsc_select<32>
+                                         : k_vsc_select<0>;
+  hipLaunchKernelGGL(select, dim3(st->N_time * st->N_z), dim3(1024), 0, st->stream, P, st->filt,
+                     st->U / kNhicdK);
   HIPCHK(hipGetLastError());
   return 0;
 }

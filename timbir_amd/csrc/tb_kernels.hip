@@ -961,49 +961,90 @@ __global__ __launch_bounds__(256) void k_vsc_filter(KP P, float *__restrict__ fi
 // patterns order like the values), and the lines above it are listed in
 // raster order.  The reference finds the same order statistic with a
 // randomized quickselect (XT_NHICD.c:63-128).
-constexpr int kVscThreads = 1024;
+//
+// What bounds it: latency, one workgroup a cell.  Each wave owns a contiguous
+// range of the pixels and walks it 64 at a time in the order of the list; R
+// of these steps are held in registers with their mask bits for all six
+// walks (R = 8, 16 and 32 up to 8192, 16384 and 32768 pixels: a cell is then
+// read once), larger cells are read again, eight steps in flight.  The
+// histogram has a copy per lane of 16, since most values share a bucket.  A
+// launch of four cells of 128 x 128 or 192 x 192 pixels took 47 us and takes
+// 16 and 38; 128 cells of 512 x 512 with their filter 0.76 and 0.48 ms.
+constexpr int kVscThreads = 1024, kVscRep = 16;
+template <int R>
 __global__ __launch_bounds__(kVscThreads) void k_vsc_select(KP P, const float *__restrict__ filt,
                                                             int want) {
-  constexpr int NW = kVscThreads / 64;
+  constexpr int NW = kVscThreads / 64, U = R ? R : 8;
   const int cell = blockIdx.x;
   const int Nxy = P.N_x * P.N_y;
   const uint32_t *vals = reinterpret_cast<const uint32_t *>(filt + (size_t)cell * Nxy);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __shared__ uint32_t hist[256];
+  __shared__ uint32_t hist[256 * kVscRep], total[256];
   __shared__ uint32_t s_prefix, s_k;
   __shared__ int s_cnt[2][NW];
   if (threadIdx.x == 0) {
     s_prefix = 0;
     s_k = (uint32_t)(Nxy - want);  // 1-based rank of the threshold
   }
-  __syncthreads();
+  const int per = (Nxy + NW - 1) / NW;
+  const int w0 = min(wid * per, Nxy), w1 = min(w0 + per, Nxy);
+  uint32_t b[U], m = 0;  // values and mask bits of U steps
+  const int last = max(w1 - 1, 0);
+  auto load = [&](int i0, bool with_mask) {
+    uint8_t mk[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = min(i0 + 64 * u + lane, last);
+      b[u] = vals[i];
+      mk[u] = with_mask ? P.mask[i] : 0;
+    }
+    m = 0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      b[u] |= (uint32_t)((last - (i0 + 64 * u + lane)) >> 31);  // all ones past the range
+      m |= (uint32_t)(mk[u] == 1) << u;
+    }
+  };
+  // fn(pixel, value, mask bit) over the wave's range, step by step, in every
+  // lane of the wave.  A lane past the range holds all ones: above every value in the ranking, so that no rank counts it,
+  // and a NaN, above no threshold.
+  auto walk = [&](bool with_mask, auto fn) {
+    for (int i0 = w0; R ? i0 == w0 : i0 < w1; i0 += 64 * U) {
+      if (!R) load(i0, with_mask);
+#pragma unroll
+      for (int u = 0; u < U; u++) fn(i0 + 64 * u + lane, b[u], (m >> u) & 1u);
+    }
+  };
+  if (R) load(w0, true);
   uint32_t thresh_bits = 0xffffffffu;  // want <= 0: nothing above
   if (want > 0) {
     for (int pass = 0; pass < 4; pass++) {
       const int shift = 24 - 8 * pass;
       const uint32_t hmask = pass == 0 ? 0u : (0xffffffffu << (32 - 8 * pass));
-      if (threadIdx.x < 256) hist[threadIdx.x] = 0;
+      for (int t = threadIdx.x; t < 256 * kVscRep; t += kVscThreads) hist[t] = 0;
       __syncthreads();
       const uint32_t pre = s_prefix;
-      // eight independent loads in flight per thread
-      for (int i0 = threadIdx.x; i0 < Nxy; i0 += 8 * kVscThreads) {
-        uint32_t b[8];
+      walk(false, [&](int i, uint32_t v, uint32_t) {
+        if ((v & hmask) == pre)
+          atomicAdd(&hist[((v >> shift) & 0xff) * kVscRep + (lane & (kVscRep - 1))], 1u);
+      });
+      __syncthreads();
+      {
+        // four threads a bucket add its copies
+        const uint32_t *h = &hist[threadIdx.x * (kVscRep / 4)];
+        uint32_t c = 0;
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = i0 + u * kVscThreads;
-          b[u] = i < Nxy ? vals[i] : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-          if ((i0 + u * kVscThreads < Nxy) && (b[u] & hmask) == pre)
-            atomicAdd(&hist[(b[u] >> shift) & 0xff], 1u);
+        for (int t = 0; t < kVscRep / 4; t++) c += h[t];
+        c += __shfl_xor(c, 1);
+        c += __shfl_xor(c, 2);
+        if ((threadIdx.x & 3) == 0) total[threadIdx.x >> 2] = c;
       }
       __syncthreads();
       if (wid == 0) {
         // inclusive scan of the 256 counts, 4 per lane, then the first
         // bucket whose running count reaches k
-        const uint32_t c0 = hist[4 * lane], c1 = hist[4 * lane + 1], c2 = hist[4 * lane + 2],
-                       c3 = hist[4 * lane + 3];
+        const uint32_t c0 = total[4 * lane], c1 = total[4 * lane + 1], c2 = total[4 * lane + 2],
+                       c3 = total[4 * lane + 3];
         const uint32_t own = c0 + c1 + c2 + c3;
         uint32_t incl = own;
 #pragma unroll
@@ -1033,19 +1074,15 @@ __global__ __launch_bounds__(kVscThreads) void k_vsc_select(KP P, const float *_
     thresh_bits = s_prefix;
   }
   const float thresh = __uint_as_float(thresh_bits);
-  // compaction in raster order: wave w owns the contiguous range
-  // [w * per, (w + 1) * per) and walks it 64 pixels at a time (coalesced,
-  // ballot offsets); one block-wide prefix of the wave counts in between
-  const int per = (Nxy + NW - 1) / NW;
-  const int w0 = min(wid * per, Nxy), w1 = min(w0 + per, Nxy);
+  // compaction in raster order: the waves' counts, then a walk with ballot
+  // offsets
   int nsel = 0, nin = 0;
   if (want > 0)
-    for (int i = w0 + lane; i - lane < w1; i += 64) {
-      const bool f = i < w1 && __uint_as_float(vals[i]) > thresh;
-      const bool in = f && P.mask[i] == 1;
+    walk(true, [&](int i, uint32_t v, uint32_t mk) {
+      const bool f = __uint_as_float(v) > thresh;
       nsel += __popcll(__ballot(f));
-      nin += __popcll(__ballot(in));
-    }
+      nin += __popcll(__ballot(f && mk));
+    });
   if (lane == 0) {
     s_cnt[0][wid] = nsel;
     s_cnt[1][wid] = nin;
@@ -1061,10 +1098,12 @@ __global__ __launch_bounds__(kVscThreads) void k_vsc_select(KP P, const float *_
     ti += s_cnt[1][w];
   }
   const unsigned long long below = (1ull << lane) - 1ull;
+  float thr = thresh;
+  asm volatile("" : "+v"(thr), "+v"(m));  // the ballots are taken again, not kept
   if (want > 0)
-    for (int i = w0 + lane; i - lane < w1; i += 64) {
-      const bool f = i < w1 && __uint_as_float(vals[i]) > thresh;
-      const bool in = f && P.mask[i] == 1;
+    walk(true, [&](int i, uint32_t v, uint32_t mk) {
+      const bool f = __uint_as_float(v) > thr;
+      const bool in = f && mk;
       const unsigned long long bf = __ballot(f), bi = __ballot(in);
       if (f) {
         const int pos = ps + __popcll(bf & below);
@@ -1080,12 +1119,16 @@ __global__ __launch_bounds__(kVscThreads) void k_vsc_select(KP P, const float *_
       if (f && !in) P.mag[(size_t)cell * Nxy + i] = 0.0f;
       ps += __popcll(bf);
       pi += __popcll(bi);
-    }
+    });
   if (threadIdx.x == 0) {
     P.nh_count[cell] = min(ts, P.nh_cap);
     P.nh_ord_count[cell] = min(ti, P.nh_cap);
   }
 }
+template __global__ void k_vsc_select<8>(KP, const float *, int);
+template __global__ void k_vsc_select<16>(KP, const float *, int);
+template __global__ void k_vsc_select<32>(KP, const float *, int);
+template __global__ void k_vsc_select<0>(KP, const float *, int);
 
 // sum of the magnitude map over masked pixels (convergence numerator,
 // XT_ICD_update.c:1068-1072)
