@@ -962,7 +962,7 @@ extern "C" int tb_variance_update(tb_stage *st) {
 static int ensure_order(tb_stage *st, int iter) {
   if (st->ord_iter == iter) return 0;
   KP P = st->kp();
-  hipLaunchKernelGGL(k_build_order, dim3(st->N_time * st->N_z), dim3(256), 0, st->stream, P, iter);
+  hipLaunchKernelGGL(k_build_order, dim3(st->N_time * st->N_z), dim3(1024), 0, st->stream, P, iter);
   HIPCHK(hipGetLastError());
   st->ord_iter = iter;
   return 0;
