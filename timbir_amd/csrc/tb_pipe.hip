@@ -132,8 +132,8 @@ __device__ __forceinline__ bool huber_sel(const KP &P, float e, float w) {
 // w inside the threshold, T delta sqrt(w) / |e| outside.  The rounded e^2 w
 // decides wherever it is off T^2 by more than its own error and huber_sel's
 // (2^-22 of it; the band is four times that, and 2^-20 for what underflow
-// loses), and huber_sel inside the band.  The outer weight is evaluated only when some
-// lane of the wave needs it.
+// loses), and huber_sel inside the band.  The outer weight is evaluated only
+// when some lane of the wave needs it.
 struct HuberBand {
   float lo, hi;
 };
