@@ -184,3 +184,26 @@ def test_head_backward_and_network_input(L, c):
     want[:, 0] = U.bf16(v * np.float32(scale))
     want[:, 1] = U.bf16(np.tile(m, 3) * np.float32(scale))
     np.testing.assert_array_equal(host(x), want)
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 5, 7), (1, 1, 4, 6), (2, 4, 1, 3), (1, 2, 3, 1), (3, 5, 2, 2)])
+@pytest.mark.parametrize("c,off", [(32, 0), (32, 1), (5, 0)])
+def test_up2_concat_backward_of_odd_sizes(L, shape, c, off):
+    """The skip connection's gradient at every voxel and the coarse one at the
+    parents that odd sizes leave (their halves rounded down), bit for bit."""
+    log(f"up2 concat backward {shape} c={c} offset {off}")
+    rng = np.random.default_rng(c + shape[3])
+    n, d, h, w = shape
+    g = U.bf16(rng.standard_normal(shape + (2 * c,)).astype(np.float32))
+    G = bf(np.concatenate([np.zeros(off, np.float32), g.ravel()]))
+    cell = (n, d // 2, h // 2, w // 2, c)
+    ga = bf(np.full(max(int(np.prod(cell)), 1) + off, 7.0))
+    gb = bf(np.full(g.size // 2 + off, 7.0))
+    assert L.tb_nn_up2_concat_bwd(at(G, off, 2), at(ga, off, 2), at(gb, off, 2), *shape, c, c,
+                                  None) == 0
+    np.testing.assert_array_equal(host(gb)[off:].reshape(shape + (c,)), g[..., c:])
+    s = np.zeros(cell, np.float32)
+    e = g[:, :d // 2 * 2, :h // 2 * 2, :w // 2 * 2, :c]
+    for k in range(8):
+        s = s + e[:, k >> 2::2, (k >> 1 & 1)::2, (k & 1)::2]
+    np.testing.assert_array_equal(host(ga)[off:off + s.size].reshape(cell), U.bf16(s))

@@ -569,6 +569,35 @@ __device__ __forceinline__ Row row_of(unsigned b, int D, int H) {
   return r;
 }
 
+// Division of a flat index by one of the sizes behind it.  32 bits, for indices
+// below 2^31: one high product with the divisor's reciprocal rounded up (with
+// 2^s < d <= 2^(s+1), m d exceeds 2^(32+s) by less than d, so the error stays
+// below one step of the quotient); else the plain 64-bit division.
+template <class Ix>
+struct Div {
+  Ix d;
+  __device__ __forceinline__ Ix operator()(Ix n) const { return n / d; }
+};
+template <>
+struct Div<uint32_t> {
+  uint32_t d, m, s;
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
+    return m ? __umulhi(n, m) >> s : n;
+  }
+};
+template <class Ix>
+static Div<Ix> make_div(long long d) {
+  Div<Ix> r{};
+  r.d = (Ix)std::max<long long>(d, 1);
+  if constexpr (sizeof(Ix) == 4) {
+    if (r.d > 1) {
+      r.s = 31 - __builtin_clz(r.d - 1);
+      r.m = (uint32_t)(((1ull << (32 + r.s)) + r.d - 1) / r.d);
+    }
+  }
+  return r;
+}
+
 // A block's per-channel sums, combined over its threads: thread t holds V
 // channels of group t % nc in acc, the threads past a whole number of groups
 // nothing
@@ -699,38 +728,40 @@ __global__ __launch_bounds__(256) void k_up2_concat(const bf16 *__restrict__ a,
 }
 
 // backward of k_up2_concat: ga[p][c] = sum over the 8 children of g[v][c],
-// gb[v][c] = g[v][Ca + c]; block: one coarse row and the four full-size rows
-// of its children
-template <int V>
+// gb[v][c] = g[v][Ca + c]; the na groups of V channels of ga, then those of gb.
+// Each output has an item of its own, so every row of gb is written, also the
+// last ones of an odd size, which no parent covers.
+template <int V, class Ix>
 __global__ __launch_bounds__(256) void k_up2_concat_bwd(const bf16 *__restrict__ g,
                                                         bf16 *__restrict__ ga,
                                                         bf16 *__restrict__ gb, int D, int H, int W,
-                                                        int Ca, int Cb) {
-  const Row r = row_of(blockIdx.x, D / 2, H / 2);
-  const int C = Ca + Cb, AG = Ca / V, BG = Cb / V;
-  const size_t row0 = ((size_t)r.n * D + 2 * r.z) * H + 2 * r.y;
-  const bf16 *src = g + row0 * W * C;
-  for (int i = threadIdx.x; i < W / 2 * AG; i += 256) {
-    const int x = i / AG, c = (i - x * AG) * V;
-    float s[V] = {};
+                                                        int Ca, int Cb, Ix na, Ix total,
+                                                        Div<Ix> ag, Div<Ix> bg, Div<Ix> wc,
+                                                        Div<Ix> hc, Div<Ix> dc) {
+  const int C = Ca + Cb;
+  for (Ix j = blockIdx.x * (Ix)blockDim.x + threadIdx.x; j < total;
+       j += (Ix)gridDim.x * blockDim.x) {
+    if (j < na) {
+      const Ix p = ag(j), q = wc(p), r = hc(q), n = dc(r);
+      const int c = (int)(j - p * ag.d) * V, x = (int)(p - q * wc.d), y = (int)(q - r * hc.d),
+                z = (int)(r - n * dc.d);
+      const bf16 *src = g + ((((size_t)n * D + 2 * z) * H + 2 * y) * W + 2 * x) * C + c;
+      float s[V] = {};
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      float v[V];
-      ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + 2 * x + (k & 1)) * C + c, v);
+      for (int k = 0; k < 8; k++) {
+        float v[V];
+        ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + (k & 1)) * C, v);
 #pragma unroll
-      for (int q = 0; q < V; q++) s[q] += v[q];
-    }
-    stv<V>(ga + ((size_t)blockIdx.x * (W / 2) + x) * Ca + c, s);
-  }
-  for (int k = 0; k < 4; k++) {
-    const size_t row = row0 + (size_t)(k >> 1) * H + (k & 1);
-    for (int i = threadIdx.x; i < W * BG; i += 256) {
-      const int x = i / BG, c = (i - x * BG) * V;
+        for (int u = 0; u < V; u++) s[u] += v[u];
+      }
+      stv<V>(ga + (size_t)j * V, s);
+    } else {
+      const Ix i = j - na, v = bg(i);
+      const bf16 *src = g + (size_t)v * C + Ca + (size_t)(i - v * bg.d) * V;
       if constexpr (V == 8)
-        *reinterpret_cast<bf16x8 *>(gb + (row * W + x) * Cb + c) =
-            *reinterpret_cast<const bf16x8 *>(g + (row * W + x) * C + Ca + c);
+        *reinterpret_cast<bf16x8 *>(gb + (size_t)i * 8) = *reinterpret_cast<const bf16x8 *>(src);
       else
-        gb[(row * W + x) * Cb + c] = g[(row * W + x) * C + Ca + c];
+        gb[i] = *src;
     }
   }
 }
@@ -1167,16 +1198,26 @@ extern "C" int tb_nn_up2_concat(const void *a, const void *b, void *out, int32_t
   return 0;
 }
 
+// index type and channels a thread, by the items' number and the operands
+template <int V, class Ix>
+static void up2_concat_bwd(const void *g, void *ga, void *gb, int n, int d, int h, int wd, int ca,
+                           int cb, hipStream_t s) {
+  const size_t na = (size_t)n * (d / 2) * (h / 2) * (wd / 2) * (ca / V);
+  const size_t total = na + (size_t)n * d * h * wd * (cb / V);
+  hipLaunchKernelGGL((k_up2_concat_bwd<V, Ix>), dim3(grid1d(total)), dim3(256), 0, s,
+                     static_cast<const bf16 *>(g), static_cast<bf16 *>(ga),
+                     static_cast<bf16 *>(gb), d, h, wd, ca, cb, (Ix)na, (Ix)total,
+                     make_div<Ix>(ca / V), make_div<Ix>(cb / V), make_div<Ix>(wd / 2),
+                     make_div<Ix>(h / 2), make_div<Ix>(d / 2));
+}
+
 extern "C" int tb_nn_up2_concat_bwd(const void *g, void *ga, void *gb, int32_t n, int32_t d,
                                     int32_t h, int32_t wd, int32_t ca, int32_t cb, void *stream) {
-  unsigned rows = 0;
-  if (row_blocks(n, d / 2, h / 2, &rows)) return -1;
-  if (!rows) return 0;
-  auto fn = ca % 8 == 0 && cb % 8 == 0 && al16(g) && al16(ga) && al16(gb) ? k_up2_concat_bwd<8>
-                                                                          : k_up2_concat_bwd<1>;
-  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const bf16 *>(g), static_cast<bf16 *>(ga),
-                     static_cast<bf16 *>(gb), d, h, wd, ca, cb);
+  const bool vec = ca % 8 == 0 && cb % 8 == 0 && al16(g) && al16(ga) && al16(gb);
+  const bool small = (size_t)n * d * h * wd * ((size_t)ca + cb) < 0x7fffffffu;
+  auto fn = vec ? (small ? up2_concat_bwd<8, uint32_t> : up2_concat_bwd<8, uint64_t>)
+                : (small ? up2_concat_bwd<1, uint32_t> : up2_concat_bwd<1, uint64_t>);
+  fn(g, ga, gb, n, d, h, wd, ca, cb, static_cast<hipStream_t>(stream));
   NNCHK("tb_nn_up2_concat_bwd");
   return 0;
 }
