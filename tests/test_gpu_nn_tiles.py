@@ -207,3 +207,53 @@ def test_up2_concat_backward_of_odd_sizes(L, shape, c, off):
     for k in range(8):
         s = s + e[:, k >> 2::2, (k >> 1 & 1)::2, (k & 1)::2]
     np.testing.assert_array_equal(host(ga)[off:off + s.size].reshape(cell), U.bf16(s))
+
+
+@pytest.mark.parametrize("shape,cin,cout", [((1, 3, 5, 20), 32, 32), ((2, 2, 9, 66), 32, 32),
+                                            ((1, 2, 8, 33), 64, 64), ((1, 2, 4, 64), 96, 96),
+                                            ((1, 2, 1, 40), 128, 64), ((1, 2, 17, 31), 192, 64)])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_conv3d_leaves_out_taps_outside_the_volume(L, shape, cin, cout, value):
+    """A weight that is infinite or NaN reaches only the voxels whose rows of
+    that tap lie inside the volume: the staged convolution (and the one of a
+    concatenation) gives the unstaged one's values, finite in the first and
+    last rows where that is."""
+    log(f"conv non-finite weight {shape} {cin}->{cout} {value}")
+    rng = np.random.default_rng(cin + shape[2])
+    n, d, h, w_ = shape
+    x = bf(rng.standard_normal(shape + (cin,)))
+    for dy in (0, 2):
+        w = (rng.standard_normal((27, cout, cin)) / 30).astype(np.float32)
+        w[dy * 3::9, 5, 7] = value
+        wt, y = bf(w), empty((int(np.prod(shape)) * cout + 4,))
+        got = []
+        for off in (0, 1):
+            assert L.tb_nn_conv3d(ptr(x), ptr(wt), None, at(y, off, 4), *shape, cin, cout, 0, 1,
+                                  None) == 0
+            got.append(host(y)[off:off + n * d * h * w_ * cout].reshape(shape + (cout,)))
+        edge = got[1][:, :, 0 if dy == 0 else h - 1, :, 5]
+        assert np.isfinite(edge).all()
+        assert h == 1 or not np.isfinite(got[1][..., 5]).all()
+        np.testing.assert_array_equal(got[0], got[1])
+
+
+def test_conv3d_up2cat_leaves_out_taps_outside_the_volume(L):
+    log("conv up2cat non-finite weight")
+    rng = np.random.default_rng(3)
+    for shape, ca, cb in (((1, 2, 6, 34), 64, 32), ((1, 4, 10, 66), 64, 32), ((1, 2, 6, 30), 128, 64)):
+        n, d, h, w_ = shape
+        a = bf(rng.standard_normal((n, d // 2, h // 2, w_ // 2, ca)))
+        b = bf(rng.standard_normal(shape + (cb,)))
+        w = (rng.standard_normal((27, 32, ca + cb)) / 30).astype(np.float32)
+        w[0::9, 5, 7] = np.inf
+        w[6::9, 9, ca + 3] = np.nan
+        wt, bias, size = bf(w), dev(rng.standard_normal(32)), int(np.prod(shape)) * 32
+        cat, y1, y2 = empty(shape + (ca + cb,), "bf16"), empty((size + 4,), "bf16"), empty((size,), "bf16")
+        assert L.tb_nn_up2_concat(ptr(a), ptr(b), ptr(cat), *shape, ca, cb, None) == 0
+        assert L.tb_nn_conv3d(ptr(cat), ptr(wt), ptr(bias), at(y1, 1, 2), *shape, ca + cb, 32, 1, 0,
+                              None) == 0
+        assert L.tb_nn_conv3d_up2cat(ptr(a), ptr(b), ptr(wt), ptr(bias), ptr(y2), *shape, ca, cb, 32,
+                                     1, None) == 0
+        want = host(y1)[1:size + 1].reshape(shape + (32,))
+        assert np.isfinite(want[:, :, 0, :, 5]).all() and np.isfinite(want[:, :, -1, :, 9]).all()
+        np.testing.assert_array_equal(host(y2).reshape(shape + (32,)), want)

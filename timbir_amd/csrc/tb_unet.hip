@@ -53,27 +53,19 @@ __device__ __forceinline__ bf16x8 zero8() {
 // 16 MB voxels of one (n, d, h) row and 16 NB output channels; its K loop runs
 // over the 27 taps and the input channels in chunks of 32.  Taps whose
 // (d, h) neighbour row lies outside the volume are skipped (uniform over the
-// wave); voxels whose x neighbour lies outside read zeros.
+// wave); voxels whose x neighbour lies outside read zeros.  CAT: the first Ca
+// input channels are those of `ina`, of half the size, nearest x2 upsampled.
 // ---------------------------------------------------------------------------
-template <int MB, int NB>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
-    const bf16 *__restrict__ in, const bf16 *__restrict__ w, const float *__restrict__ bias,
-    void *__restrict__ out, int N, int D, int H, int W, int Cin, int Cout, int relu,
-    int out_f32) {
+template <int MB, int NB, bool CAT>
+__device__ __forceinline__ void conv_strip(const bf16 *__restrict__ ina, int Ca,
+                                           const bf16 *__restrict__ in,
+                                           const bf16 *__restrict__ w,
+                                           const float *__restrict__ bias, void *__restrict__ out,
+                                           int D, int H, int W, int Cin, int Cout, int relu,
+                                           int out_f32, int n, int d, int h, int w0, int co0) {
   const int lane = threadIdx.x & 63;
-  const long long g = (long long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-  const int WT = (W + 16 * MB - 1) / (16 * MB);
-  const int CT = Cout / (16 * NB);
-  const long long total = (long long)N * D * H * WT * CT;
-  if (g >= total) return;
-  long long r = g;
-  const int ct = (int)(r % CT); r /= CT;
-  const int wt = (int)(r % WT); r /= WT;
-  const int h = (int)(r % H); r /= H;
-  const int d = (int)(r % D);
-  const int n = (int)(r / D);
   const int row = lane & 15, kq = lane >> 4;
-  const int w0 = wt * 16 * MB, co0 = ct * 16 * NB;
+  const int Cb = CAT ? Cin - Ca : Cin;  // channels of `in`
   f32x4 acc[MB][NB];
 #pragma unroll
   for (int a = 0; a < MB; a++)
@@ -83,15 +75,27 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
   for (int tap = 0; tap < kTaps; tap++) {
     const int zz = d + tap / 9 - 1, yy = h + (tap / 3) % 3 - 1, dx = tap % 3 - 1;
     if (zz < 0 || zz >= D || yy < 0 || yy >= H) continue;
-    const bf16 *inrow = in + (((size_t)n * D + zz) * H + yy) * (size_t)W * Cin;
+    const bf16 *inrow = in + (((size_t)n * D + zz) * H + yy) * (size_t)W * Cb;
     const bf16 *wt_tap = w + (size_t)tap * Cout * Cin;
     for (int c = 0; c < nchunk; c++) {
+      const bf16 *src = inrow + c * 32;
+      int ch = Cb, sh = 0;
+      if constexpr (CAT) {
+        if (c * 32 < Ca) {
+          src = ina + (((size_t)n * (D / 2) + zz / 2) * (H / 2) + yy / 2) * (size_t)(W / 2) * Ca +
+                c * 32;
+          ch = Ca;
+          sh = 1;
+        } else {
+          src -= Ca;
+        }
+      }
       bf16x8 av[MB], bv[NB];
 #pragma unroll
       for (int a = 0; a < MB; a++) {
         const int xx = w0 + 16 * a + row + dx;
         av[a] = (xx >= 0 && xx < W)
-                    ? *reinterpret_cast<const bf16x8 *>(inrow + (size_t)xx * Cin + c * 32 + kq * 8)
+                    ? *reinterpret_cast<const bf16x8 *>(src + (size_t)(xx >> sh) * ch + kq * 8)
                     : zero8();
       }
 #pragma unroll
@@ -124,6 +128,26 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
   }
 }
 
+template <int MB, int NB>
+__global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
+    const bf16 *__restrict__ in, const bf16 *__restrict__ w, const float *__restrict__ bias,
+    void *__restrict__ out, int N, int D, int H, int W, int Cin, int Cout, int relu,
+    int out_f32) {
+  const long long g = (long long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  const int WT = (W + 16 * MB - 1) / (16 * MB);
+  const int CT = Cout / (16 * NB);
+  const long long total = (long long)N * D * H * WT * CT;
+  if (g >= total) return;
+  long long r = g;
+  const int ct = (int)(r % CT); r /= CT;
+  const int wt = (int)(r % WT); r /= WT;
+  const int h = (int)(r % H); r /= H;
+  const int d = (int)(r % D);
+  const int n = (int)(r / D);
+  conv_strip<MB, NB, false>(nullptr, 0, in, w, bias, out, D, H, W, Cin, Cout, relu, out_f32, n, d,
+                            h, wt * 16 * MB, ct * 16 * NB);
+}
+
 // The same convolution with the input staged in LDS.  The input's channels are
 // 32 CA of a tensor at half size, nearest x2 upsampled (`ina`, CA may be 0),
 // then 32 CB of one at full size (`in`): the concatenation of a U-Net's skip
@@ -140,7 +164,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
 // (a voxel's parent is x / 2); LDS keeps x modulo 4 (parents modulo 2) apart,
 // which makes each read one contiguous KB.
 //   The sums run over (tap, channel chunk) as in k_conv3d_fwd, one MFMA each:
-// the bits are the same.  2 x 16 x 256 x 256 voxels, before and now: 32 -> 32
+// the bits are the same.  Rows above and below the volume are zeros in LDS; a
+// weight that is infinite or NaN makes those NaN, so a wave that finds such a
+// sum in the volume's first or last row takes conv_strip for its strips, which
+// leaves those taps out.  2 x 16 x 256 x 256 voxels, before and now: 32 -> 32
 // channels 0.38 and 0.18 ms (650 TFLOP/s); 64 + 32 -> 32 with its
 // concatenation 1.6 and 0.46 ms (750 TFLOP/s).
 template <int CA, int CB, int SP, int WT>
@@ -271,6 +298,32 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
               for (int b = 0; b < NB; b++) acc[s][a][b] = mfma(wv[b], x[a], acc[s][a][b]);
           }
         }
+    }
+  }
+  const int hw = h0 + wave * SP * RPS;  // the wave's first row
+  if (hw == 0 || hw + SP * RPS >= H) {
+    bool bad = false;
+#pragma unroll
+    for (int s = 0; s < SP; s++) {
+      const int h = hw + s * RPS + yr;
+#pragma unroll
+      for (int a = 0; a < 4; a++) {
+        const bool in_edge = (h == 0 || h == H - 1) && w0 + 4 * xq + a < W;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int k = 0; k < 4; k++) bad |= in_edge & !(fabsf(acc[s][a][b][k]) < INFINITY);
+      }
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0ull, 0)) {
+#pragma unroll 1
+      for (int i = 0; i < SP * RPS * (WT / 16) * NB; i++) {
+        const int h = hw + i / (WT / 16 * NB), x = w0 + i / NB % (WT / 16) * 16;
+        if (h < H && x < W)
+          conv_strip<1, 1, (CA > 0)>(ina, 32 * CA, in, w, bias, out, D, H, W, Cin, Cout, relu,
+                                     out_f32, n, d, h, x, co0 + i % NB * 16);
+      }
+      return;
     }
   }
   // lane: channels co .. co + 4 NB - 1 of voxel x = w0 + 4 xq + a
