@@ -114,10 +114,14 @@ __device__ __forceinline__ void wait_vm_all() {
 
 // Generalized-Huber selection b = |e sqrt(w)| < T (XT_VoxUpdate.c:108-111):
 // e^2 w with the FMA residuals of its two products, against T^2 = T2h + T2l.
-// The product's own residual stands in both terms, so the decision is that of
-// e^2 w within 2^-24 of it (the reference's double evaluation is within
-// 2^-52).  Written out as fused operations: the entries it decides are part
-// of the result's bits, whatever the compiler contracts around it.
+// Not exact: the second product's residual stands in the fused difference and
+// in corr, so it counts twice, and an entry whose e^2 w is within 2^-24 of T^2
+// may take the wrong side (the reference's double evaluation is within 2^-52).
+// (q - T2h) + (corr - T2l) would be exact; it takes another side for a few
+// entries in 1e9, which moves the object of a 192 x 192 coarse stage by 2.5e-5
+// (relative, one iteration), so it is a change of results and not made here.
+// Written out as fused operations so that every kernel decides alike, whatever
+// the compiler contracts around it.
 __device__ __forceinline__ bool huber_sel(const KP &P, float e, float w) {
 #pragma clang fp contract(off)
   const float p = e * e;
