@@ -257,3 +257,22 @@ def test_conv3d_up2cat_leaves_out_taps_outside_the_volume(L):
         want = host(y1)[1:size + 1].reshape(shape + (32,))
         assert np.isfinite(want[:, :, 0, :, 5]).all() and np.isfinite(want[:, :, -1, :, 9]).all()
         np.testing.assert_array_equal(host(y2).reshape(shape + (32,)), want)
+
+
+def test_head_backward_without_slices_or_channels(L):
+    """No slices: the activation gradient alone.  No channels: the bias
+    gradient alone, its sums within 1e-5 of the sum of magnitudes."""
+    log("head backward, slices 0 and c 0")
+    rng = np.random.default_rng(5)
+    for nv, c in ((700, 32), (333, 12)):
+        h = U.bf16(rng.standard_normal((nv, c)).astype(np.float32))
+        w, g = (rng.standard_normal(k).astype(np.float32) for k in (c, nv))
+        ht, wt, gt = bf(h), dev(w), dev(g)
+        gh, part = empty((nv, c), "bf16"), dev(np.full(4, 3.0))
+        assert L.tb_nn_head_bwd(ptr(ht), ptr(wt), ptr(gt), ptr(gh), ptr(part), 0, nv, c, 4.0,
+                                None) == 0
+        np.testing.assert_array_equal(host(gh), U.bf16((g * np.float32(0.25))[:, None] * w[None]))
+        np.testing.assert_array_equal(host(part), np.full(4, 3.0))
+        part = empty((5, 1))
+        assert L.tb_nn_head_bwd(None, None, ptr(gt), None, ptr(part), 5, nv, 0, 4.0, None) == 0
+        assert abs(host(part).sum() - g.astype(np.float64).sum() / 4) <= 1e-5 * np.abs(g).sum() / 4
