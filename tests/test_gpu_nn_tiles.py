@@ -276,3 +276,25 @@ def test_head_backward_without_slices_or_channels(L):
         part = empty((5, 1))
         assert L.tb_nn_head_bwd(None, None, ptr(gt), None, ptr(part), 5, nv, 0, 4.0, None) == 0
         assert abs(host(part).sum() - g.astype(np.float64).sum() / 4) <= 1e-5 * np.abs(g).sum() / 4
+
+
+def test_network_of_other_widths_infers_as_it_trains(monkeypatch):
+    """A network whose concatenations are not the 64 + 32 and 128 + 64 channels
+    of tb_nn_conv3d_up2cat: its inference pass gives the training pass's
+    output, bit for bit."""
+    from timbir_amd import learned
+    log("network of other widths")
+    monkeypatch.setattr(learned, "ARCH", [
+        ("e1a", "x", 32, 32), ("e1", "e1a", 32, 32), ("e2a", "pool:e1", 32, 32), ("e2", "e2a", 32, 32),
+        ("b1", "pool:e2", 32, 96), ("b2", "b1", 96, 96), ("d2a", "cat:b2,e2", 128, 32),
+        ("d2", "d2a", 32, 32), ("d1a", "cat:d2,e1", 64, 32), ("d1", "d1a", 32, 32)])
+    monkeypatch.setattr(learned, "_LIVE", learned._live_sets())
+    p = learned.init_params(3)
+    rng = np.random.default_rng(3)
+    p["head"] = (rng.normal(0, 0.1, 32).astype(np.float32), np.zeros(1, np.float32))
+    net = learned.UNet(p)
+    x = dev(rng.normal(0, 0.01, (2, 4, 8, 12)))
+    a = net.forward(x, keep=True).numpy()
+    b = net.forward(x).numpy()
+    assert np.abs(a - x.numpy()).max() > 0
+    np.testing.assert_array_equal(a, b)

@@ -91,6 +91,9 @@ def _p(t):
 
 
 S0 = None   # the runtime's default stream
+# channels (coarse, skip) that tb_nn_conv3d_up2cat takes; others go through
+# tb_nn_up2_concat and tb_nn_conv3d
+_UP2CAT = ((64, 32), (128, 64))
 
 
 class UNet:
@@ -161,7 +164,7 @@ class UNet:
                 ta, _ = acts[a]
                 tb_, shp = acts[b]
                 ca, cb = ta.shape[-1], tb_.shape[-1]
-                if not keep:
+                if not keep and (ca, cb) in _UP2CAT:
                     # nothing else reads the concatenation: it stays unwritten
                     y = DevArray(shp + (cout,), "bf16")
                     _ok(L.tb_nn_conv3d_up2cat(_p(ta), _p(tb_), _p(self.wbf[name]),
