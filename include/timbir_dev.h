@@ -375,7 +375,8 @@ int tb_nn_conv3d(const void *in, const void *w, const float *bias, void *out, in
                  int32_t out_f32, void *stream);
 /* tb_nn_up2_concat and tb_nn_conv3d in one (bf16 output), the same bits: the
  * input channels are a's ca (half size, nearest x2 upsampled) then b's cb,
- * 64 + 32 or 128 + 64 of them; n x d x h x wd the full size, even. */
+ * 64 + 32 or 128 + 64 of them; n x d x h x wd the full size, even; a, b, w
+ * and out 16-byte aligned. */
 int tb_nn_conv3d_up2cat(const void *a, const void *b, const void *w, const float *bias, void *out,
                         int32_t n, int32_t d, int32_t h, int32_t wd, int32_t ca, int32_t cb,
                         int32_t cout, int32_t relu, void *stream);

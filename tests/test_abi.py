@@ -115,3 +115,15 @@ def test_bench_traffic_comes_from_the_committed_counter_summary():
     t = bench.measured_traffic()
     assert t is not None and t > 1.85e10
     assert os.path.exists(bench.TRAFFIC_PROFILE)
+
+
+@pytest.mark.parametrize("which", ["a", "b", "w", "out"])
+def test_up2cat_refuses_unaligned_operands(which):
+    # each is read or written 16 bytes at a time; refused before any launch
+    # (the addresses are not memory)
+    from timbir_amd import learned
+    L = learned.nn_lib()
+    p = {k: C.c_void_p(0x1000 + (2 if k == which else 0)) for k in ("a", "b", "w", "out")}
+    assert L.tb_nn_conv3d_up2cat(p["a"], p["b"], p["w"], None, p["out"], 1, 2, 2, 2, 64, 32, 32, 1,
+                                 None) == -1
+    assert b"aligned" in L.tb_nn_last_error()

@@ -1143,8 +1143,8 @@ extern "C" int tb_nn_conv3d_up2cat(const void *a, const void *b, const void *w, 
                : ca == 128 && cb == 64 ? conv_pick<4, 2>(cout, wd)
                                        : nullptr;
   if (!fn) return nn_fail("tb_nn_conv3d_up2cat: 64 + 32 or 128 + 64 input channels");
-  if (reinterpret_cast<uintptr_t>(out) % 16)
-    return nn_fail("tb_nn_conv3d_up2cat: the output must be 16-byte aligned");
+  if (!al16(a) || !al16(b) || !al16(w) || !al16(out))
+    return nn_fail("tb_nn_conv3d_up2cat: a, b, w and out must be 16-byte aligned");
   return fn(a, b, w, bias, out, n, d, h, wd, cout, relu, 0, static_cast<hipStream_t>(stream));
 }
 
