@@ -144,3 +144,11 @@ def test_line_selection_at_its_register_limits(N, kind):
     changed = g.magmap() != mag
     assert not changed[..., o.mask() == 1].any() and not g.magmap()[changed].any()
     g.close()
+
+
+@pytest.mark.parametrize("N,nz,shift", [(23, 2, 0.0), (30, 6, -1.5), (21, 7, 4.0), (18, 10, 0.0),
+                                        (25, 15, 2.0), (32, 16, 0.0)])
+def test_fbp_of_a_groups_remainder(N, nz, shift):
+    """The numbers of slices in the last group that test_fbp_groups_and_edges
+    has not, each its own kernel and row stride, to the same bound."""
+    test_fbp_groups_and_edges(N, nz, shift)

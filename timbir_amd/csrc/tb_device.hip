@@ -23,7 +23,7 @@ __global__ void k_to_ref_layout(KP, const float *, float *);
 __global__ void k_fwd_interleave(KP, float4 *);
 __global__ void k_fbp_filter(KP, float *, int);
 template <int NZ>
-__global__ void k_fbp_back(KP, const float *);
+__global__ void k_fbp_back(KP, const float *, int, int);
 __global__ void k_forward(KP, const int *, const float4 *, float *, int);
 __global__ void k_upsample(const float *, float *, int, int, int, int, int);
 template <int NT>
@@ -862,11 +862,20 @@ extern "C" int tb_init_fbp(tb_stage *st) {
   const size_t lds = (taps + (size_t)per * st->N_r) * sizeof(double);
   HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_fbp_filter),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  HIPCHK(dalloc(&q, (size_t)ngroups * kFwdZ * st->N_p * st->N_r));
+  HIPCHK(dalloc(&q, (size_t)st->N_z * st->N_p * st->N_r));
   hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, ngroups), dim3(512), lds, st->stream, P, q, per);
-  const dim3 grid((unsigned)((st->nxy() + 255) / 256 * st->N_time * ngroups));
-  if (st->N_z <= 4) hipLaunchKernelGGL(k_fbp_back<4>, grid, dim3(256), 0, st->stream, P, q);
-  else hipLaunchKernelGGL(k_fbp_back<8>, grid, dim3(256), 0, st->stream, P, q);
+  // the groups of kFwdZ slices, then the remainder's
+  static_assert(kFwdZ == 8, "one kernel for each number of slices");
+  void (*const back[kFwdZ + 1])(KP, const float *, int, int) = {
+      nullptr,       k_fbp_back<1>, k_fbp_back<2>, k_fbp_back<3>, k_fbp_back<4>,
+      k_fbp_back<5>, k_fbp_back<6>, k_fbp_back<7>, k_fbp_back<8>};
+  const size_t runs = (st->nxy() + 255) / 256 * st->N_time;
+  const int full = st->N_z / kFwdZ, rest = st->N_z % kFwdZ;
+  if (full)
+    hipLaunchKernelGGL(back[kFwdZ], dim3((unsigned)(runs * full)), dim3(256), 0, st->stream, P, q,
+                       0, full);
+  if (rest)
+    hipLaunchKernelGGL(back[rest], dim3((unsigned)runs), dim3(256), 0, st->stream, P, q, full, 1);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess) err = hipStreamSynchronize(st->stream);
   (void)hipFree(q);

@@ -299,7 +299,8 @@ __global__ __launch_bounds__(kFwdT) void k_forward(KP P, const int *__restrict__
 // and gives a thread kFbpF outputs of one parity, which share each sample and
 // all but one tap.  The back-projection's geometry (ray, bin, fraction)
 // depends on the pixel and view alone: a thread evaluates it once for NZ
-// slices, whose filtered rows lie side by side in q[group][v][r][kFwdZ].  With
+// slices, whose filtered rows lie side by side in q[group][v][r][NZ] (kFwdZ
+// slices a group, the last one N_z's remainder, so q holds N_z rows a view).  With
 // a division per tap and a thread per voxel the two took 1.34 and 6.62 ms for
 // 512 x 512 x 16 slices x 8 frames and 1024 views, in this form 0.25 and 0.97.
 // ---------------------------------------------------------------------------
@@ -314,10 +315,10 @@ __global__ __launch_bounds__(512) void k_fbp_filter(KP P, float *__restrict__ q,
     s_h[i] = -1.0 / (kPi * kPi) / (n * n);
   }
   const double h = P.delta_r;
-  float *out = q + ((size_t)g * P.N_p + v) * P.N_r * kFwdZ;
   // item: outputs r0, r0 + 2, .. of one parity, from the samples of the other
   const int items = 2 * ((P.N_r + 2 * kFbpF - 1) / (2 * kFbpF));
   const int nz = min(kFwdZ, P.N_z - g * kFwdZ);
+  float *out = q + (size_t)g * kFwdZ * P.N_p * P.N_r + (size_t)v * P.N_r * nz;
   for (int z0 = 0; z0 < nz; z0 += per) {
     const int ns = min(per, nz - z0);
     __syncthreads();
@@ -352,20 +353,34 @@ __global__ __launch_bounds__(512) void k_fbp_filter(KP P, float *__restrict__ q,
       }
 #pragma unroll
       for (int u = 0; u < kFbpF; u++)
-        if (r0 + 2 * u < P.N_r) out[(size_t)(r0 + 2 * u) * kFwdZ + z0 + sl] = (float)(acc[u] / h);
+        if (r0 + 2 * u < P.N_r) out[(size_t)(r0 + 2 * u) * nz + z0 + sl] = (float)(acc[u] / h);
     }
   }
 }
 
-// thread: one pixel of one frame, NZ slices (blocks: frame, group, run of pixels)
+// thread: one pixel of one frame, the NZ slices of a group (blocks: frame, group
+// g0 .. g0 + ngroups - 1, run of pixels)
 template <int NZ>
-__global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q) {
+__device__ __forceinline__ void ld_slices(const float *p, float (&o)[NZ]) {
+  if constexpr (NZ % 4 == 0) {
+#pragma unroll
+    for (int i = 0; i < NZ / 4; i++) {
+      const float4 v = reinterpret_cast<const float4 *>(p)[i];
+      o[4 * i] = v.x, o[4 * i + 1] = v.y, o[4 * i + 2] = v.z, o[4 * i + 3] = v.w;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < NZ; i++) o[i] = p[i];
+  }
+}
+template <int NZ>
+__global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q, int g0,
+                                                  int ngroups) {
   const int Nxy = P.N_x * P.N_y;
-  const int ngroups = (P.N_z + kFwdZ - 1) / kFwdZ;
-  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, f = fg / ngroups, g = fg - f * ngroups;
+  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, f = fg / ngroups,
+            g = g0 + fg - f * ngroups;
   const int vb = P.view_off[f], nv = P.view_off[f + 1] - vb;
-  const int nz = min(NZ, P.N_z - g * kFwdZ);
-  const float4 *qg = reinterpret_cast<const float4 *>(q) + (size_t)g * P.N_p * P.N_r * (kFwdZ / 4);
+  const float *qg = q + (size_t)g * kFwdZ * P.N_p * P.N_r;
   float *ob = P.obj + ((size_t)f * P.N_z + g * kFwdZ) * Nxy;
   const int pix = (blockIdx.x - fg * runs) * 256 + (int)threadIdx.x;
   if (pix < Nxy) {
@@ -383,20 +398,16 @@ __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict_
         const double u = fma(fma(x, P.cosv[v], -(y * P.sinv[v])), P.u_inv, -P.u_r0) - 0.5;
         const double j = floor(u), t = u - j;
         const int j0 = (int)j;
-        const float4 *qv = qg + (size_t)v * P.N_r * (kFwdZ / 4);
-        if (j0 >= 0 && j0 + 1 < P.N_r) {
-          const float4 *a = qv + j0 * (kFwdZ / 4), *b = a + kFwdZ / 4;
+        const float *qv = qg + (size_t)v * P.N_r * NZ;
+        if (j0 >= 0 && j0 < P.N_r - 1) {
+          float a[NZ], b[NZ];
+          ld_slices<NZ>(qv + (size_t)j0 * NZ, a);
+          ld_slices<NZ>(qv + (size_t)j0 * NZ + NZ, b);
 #pragma unroll
-          for (int i = 0; i < NZ / 4; i++) {
-            const float4 qa = a[i], qb = b[i];
-            acc[4 * i] = fma(t, (double)qb.x, fma(1.0 - t, (double)qa.x, acc[4 * i]));
-            acc[4 * i + 1] = fma(t, (double)qb.y, fma(1.0 - t, (double)qa.y, acc[4 * i + 1]));
-            acc[4 * i + 2] = fma(t, (double)qb.z, fma(1.0 - t, (double)qa.z, acc[4 * i + 2]));
-            acc[4 * i + 3] = fma(t, (double)qb.w, fma(1.0 - t, (double)qa.w, acc[4 * i + 3]));
-          }
+          for (int i = 0; i < NZ; i++) acc[i] = fma(t, (double)b[i], fma(1.0 - t, (double)a[i], acc[i]));
         } else if (j0 == -1 || j0 == P.N_r - 1) {
           // one of the two bins is off the detector
-          const float *a = reinterpret_cast<const float *>(qv + max(j0, 0) * (kFwdZ / 4));
+          const float *a = qv + (size_t)max(j0, 0) * NZ;
           const double w = j0 < 0 ? t : 1.0 - t;
 #pragma unroll
           for (int i = 0; i < NZ; i++) acc[i] = fma(w, (double)a[i], acc[i]);
@@ -404,12 +415,17 @@ __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict_
       }
     }
 #pragma unroll
-    for (int i = 0; i < NZ; i++)
-      if (i < nz) ob[(size_t)i * Nxy + pix] = in ? (float)(acc[i] * kPi / nv) : 0.0f;
+    for (int i = 0; i < NZ; i++) ob[(size_t)i * Nxy + pix] = in ? (float)(acc[i] * kPi / nv) : 0.0f;
   }
 }
-template __global__ void k_fbp_back<4>(KP, const float *);
-template __global__ void k_fbp_back<8>(KP, const float *);
+template __global__ void k_fbp_back<1>(KP, const float *, int, int);
+template __global__ void k_fbp_back<2>(KP, const float *, int, int);
+template __global__ void k_fbp_back<3>(KP, const float *, int, int);
+template __global__ void k_fbp_back<4>(KP, const float *, int, int);
+template __global__ void k_fbp_back<5>(KP, const float *, int, int);
+template __global__ void k_fbp_back<6>(KP, const float *, int, int);
+template __global__ void k_fbp_back<7>(KP, const float *, int, int);
+template __global__ void k_fbp_back<8>(KP, const float *, int, int);
 
 // ---------------------------------------------------------------------------
 // Voxel update: one workgroup per cell of one colour, voxels in sequence.
