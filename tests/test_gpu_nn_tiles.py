@@ -298,3 +298,38 @@ def test_network_of_other_widths_infers_as_it_trains(monkeypatch):
     b = net.forward(x).numpy()
     assert np.abs(a - x.numpy()).max() > 0
     np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape,c", [((1, 2, 2, 2), 8), ((3, 2, 2, 2), 40), ((1, 2, 2, 514), 8),
+                                     ((64, 2, 6, 2), 16), ((1, 6, 10, 14), 24), ((1, 2, 258, 4), 3)])
+def test_pooling_and_concatenation_of_narrow_volumes(L, shape, c):
+    """Short rows, few rows, sides and channels of every kind of divisor:
+    pooling, its backward pass and the concatenation, bit for bit."""
+    log(f"pooling {shape} c={c}")
+    rng = np.random.default_rng(c + shape[2])
+    n, d, h, w = shape
+    cell = (n, d // 2, h // 2, w // 2, c)
+    x = U.bf16(rng.standard_normal(shape + (c,)).astype(np.float32))
+    a = U.bf16(rng.standard_normal(cell).astype(np.float32))
+    X, A, o, p, q = bf(x), bf(a), empty(cell, "bf16"), empty(x.shape, "bf16"), empty(shape + (2 * c,), "bf16")
+    assert L.tb_nn_avgpool2(ptr(X), ptr(o), *shape, c, 0, None) == 0
+    assert L.tb_nn_avgpool2(ptr(A), ptr(p), *shape, c, 1, None) == 0
+    assert L.tb_nn_up2_concat(ptr(A), ptr(X), ptr(q), *shape, c, c, None) == 0
+    s = np.zeros(cell, np.float32)
+    for k in range(8):
+        s = s + x[:, k >> 2::2, (k >> 1 & 1)::2, (k & 1)::2]
+    np.testing.assert_array_equal(host(o), U.bf16(s * np.float32(0.125)))
+    np.testing.assert_array_equal(host(p), U.bf16(U.up2(a) * np.float32(0.125)))
+    np.testing.assert_array_equal(host(q), np.concatenate([U.up2(a), x], -1))
+
+
+def test_pooling_of_more_rows_than_one_launch_has_blocks(L):
+    """2^24 + 2 pooled rows of one voxel and channel."""
+    log("pooling 2^24 rows")
+    n = (1 << 24) + 2
+    x = np.zeros((n, 8), np.float32)
+    x[::7, 3] = 8.0
+    x[-1] = 16.0
+    X, o = bf(x), empty((n,), "bf16")
+    assert L.tb_nn_avgpool2(ptr(X), ptr(o), n, 2, 2, 2, 1, 0, None) == 0
+    np.testing.assert_array_equal(host(o), x.mean(1))

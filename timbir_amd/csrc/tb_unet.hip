@@ -582,11 +582,12 @@ __global__ __launch_bounds__(64 * kSumRuns) void k_sum_parts(const float *__rest
   }
 }
 
-// The elementwise kernels below move 8 channels (16 bytes) per thread; those
-// over voxels take one row (n, z, y) per block, so that an index costs no
-// 64-bit division.  With one channel per thread the network input took 156 us,
-// the head 147, the pooling 36 on average for 2 x 16 x 256 x 256 voxels; now
-// 35, 23 and 17.
+// The elementwise kernels below move 8 channels (16 bytes) per thread.  Those
+// over voxels take one item (V channels of one voxel) after another and divide
+// its index by high products, so a 64-bit division costs nothing where they
+// are large and small or narrow volumes fill the chip too.  With one channel
+// per thread the network input took 156 us, the head 147, the pooling 36 on
+// average for 2 x 16 x 256 x 256 voxels; now 35, 23 and 17.
 // V: 8, or 1 where the channels or an address do not allow 16-byte accesses.
 template <int V>
 __device__ __forceinline__ void ldv(const bf16 *p, float (&o)[V]) {
@@ -608,18 +609,6 @@ __device__ __forceinline__ void stv(bf16 *p, const float (&o)[V]) {
   } else {
     p[0] = (bf16)o[0];
   }
-}
-
-struct Row {
-  int n, z, y;
-};
-__device__ __forceinline__ Row row_of(unsigned b, int D, int H) {
-  Row r;
-  const unsigned q = b / (unsigned)H;
-  r.y = (int)(b - q * (unsigned)H);
-  r.n = (int)(q / (unsigned)D);
-  r.z = (int)(q - (unsigned)r.n * (unsigned)D);
-  return r;
 }
 
 // Division of a flat index by one of the sizes behind it.  32 bits, for indices
@@ -715,68 +704,68 @@ __global__ void k_relu_bwd(const bf16 *__restrict__ y, bf16 *__restrict__ g, siz
     if (!((float)y[i] > 0.f)) g[i] = (bf16)0.f;
 }
 
-// 2x2x2 average pooling, forward and backward (block: one output row)
-template <int V>
+// 2x2x2 average pooling, forward and backward.  An item is V channels of an
+// output voxel; wo, ho, dp divide by the output's sides.
+template <int V, class Ix>
 __global__ __launch_bounds__(256) void k_avgpool2(const bf16 *__restrict__ in,
-                                                  bf16 *__restrict__ out, int D, int H, int W,
-                                                  int C) {
-  const Row r = row_of(blockIdx.x, D / 2, H / 2);
-  const int CG = C / V, items = W / 2 * CG;
-  const bf16 *src = in + (((size_t)r.n * D + 2 * r.z) * H + 2 * r.y) * (size_t)W * C;
-  bf16 *dst = out + (size_t)blockIdx.x * (W / 2) * C;
-  for (int i = threadIdx.x; i < items; i += 256) {
-    const int x = i / CG, c = (i - x * CG) * V;
+                                                  bf16 *__restrict__ out, int C, Ix total,
+                                                  Div<Ix> cg, Div<Ix> wo, Div<Ix> ho, Div<Ix> dp) {
+  for (Ix j = blockIdx.x * (Ix)blockDim.x + threadIdx.x; j < total;
+       j += (Ix)gridDim.x * blockDim.x) {
+    const Ix p = cg(j), q = wo(p), r = ho(q), n = dp(r);
+    const Ix c = (j - p * cg.d) * V, x = p - q * wo.d, y = q - r * ho.d, z = r - n * dp.d;
+    const Ix row = 2 * wo.d * (Ix)C, plane = 2 * ho.d * row;
+    const bf16 *src = in + ((n * dp.d + z) * 2 * plane + 2 * y * row + 2 * x * C + c);
     float s[V] = {};
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       float v[V];
-      ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + 2 * x + (k & 1)) * C + c, v);
+      ldv<V>(src + ((k >> 2) * plane + ((k >> 1) & 1) * row + (Ix)((k & 1) * C)), v);
 #pragma unroll
-      for (int q = 0; q < V; q++) s[q] += v[q];
+      for (int u = 0; u < V; u++) s[u] += v[u];
     }
 #pragma unroll
-    for (int q = 0; q < V; q++) s[q] *= 0.125f;
-    stv<V>(dst + (size_t)x * C + c, s);
+    for (int u = 0; u < V; u++) s[u] *= 0.125f;
+    stv<V>(out + (size_t)j * V, s);
   }
 }
 
-template <int V>
+template <int V, class Ix>
 __global__ __launch_bounds__(256) void k_avgpool2_bwd(const bf16 *__restrict__ gout,
-                                                      bf16 *__restrict__ gin, int D, int H, int W,
-                                                      int C) {
-  const Row r = row_of(blockIdx.x, D, H);
-  const int CG = C / V, items = W * CG;
-  const bf16 *src = gout + (((size_t)r.n * (D / 2) + r.z / 2) * (H / 2) + r.y / 2) * (size_t)(W / 2) * C;
-  bf16 *dst = gin + (size_t)blockIdx.x * W * C;
-  for (int i = threadIdx.x; i < items; i += 256) {
-    const int x = i / CG, c = (i - x * CG) * V;
+                                                      bf16 *__restrict__ gin, int C, Ix total,
+                                                      Div<Ix> cg, Div<Ix> wo, Div<Ix> ho,
+                                                      Div<Ix> dp) {
+  for (Ix j = blockIdx.x * (Ix)blockDim.x + threadIdx.x; j < total;
+       j += (Ix)gridDim.x * blockDim.x) {
+    const Ix p = cg(j), q = wo(p), r = ho(q), n = dp(r);
+    const Ix c = (j - p * cg.d) * V, x = p - q * wo.d, y = q - r * ho.d, z = r - n * dp.d;
     float v[V];
-    ldv<V>(src + (size_t)(x / 2) * C + c, v);
+    const Ix parent = ((n * (dp.d / 2) + z / 2) * (ho.d / 2) + y / 2) * (wo.d / 2) + x / 2;
+    ldv<V>(gout + (parent * C + c), v);
 #pragma unroll
-    for (int q = 0; q < V; q++) v[q] *= 0.125f;
-    stv<V>(dst + (size_t)x * C + c, v);
+    for (int u = 0; u < V; u++) v[u] *= 0.125f;
+    stv<V>(gin + (size_t)j * V, v);
   }
 }
 
 // out[v][0:Ca] = a[parent(v)][:] (nearest x2 upsampling of the coarse
 // features), out[v][Ca:Ca+Cb] = b[v][:] (the skip connection)
-template <int V>
+template <int V, class Ix>
 __global__ __launch_bounds__(256) void k_up2_concat(const bf16 *__restrict__ a,
                                                     const bf16 *__restrict__ b,
-                                                    bf16 *__restrict__ out, int D, int H, int W,
-                                                    int Ca, int Cb) {
-  const Row r = row_of(blockIdx.x, D, H);
-  const int C = Ca + Cb, CG = C / V, items = W * CG;
-  const bf16 *ra = a + (((size_t)r.n * (D / 2) + r.z / 2) * (H / 2) + r.y / 2) * (size_t)(W / 2) * Ca;
-  const bf16 *rb = b + (size_t)blockIdx.x * W * Cb;
-  bf16 *dst = out + (size_t)blockIdx.x * W * C;
-  for (int i = threadIdx.x; i < items; i += 256) {
-    const int x = i / CG, c = (i - x * CG) * V;
-    const bf16 *p = c < Ca ? ra + (size_t)(x / 2) * Ca + c : rb + (size_t)x * Cb + (c - Ca);
+                                                    bf16 *__restrict__ out, int Ca, int Cb,
+                                                    Ix total, Div<Ix> cg,
+                                                    Div<Ix> wo, Div<Ix> ho, Div<Ix> dp) {
+  for (Ix j = blockIdx.x * (Ix)blockDim.x + threadIdx.x; j < total;
+       j += (Ix)gridDim.x * blockDim.x) {
+    const Ix p = cg(j), q = wo(p), r = ho(q), n = dp(r);
+    const Ix c = (j - p * cg.d) * V, x = p - q * wo.d, y = q - r * ho.d, z = r - n * dp.d;
+    const Ix parent = ((n * (dp.d / 2) + z / 2) * (ho.d / 2) + y / 2) * (wo.d / 2) + x / 2;
+    const bf16 *src = c < (Ix)Ca ? a + (parent * Ca + c) : b + (p * Cb + (c - Ca));
     if constexpr (V == 8)
-      *reinterpret_cast<bf16x8 *>(dst + (size_t)x * C + c) = *reinterpret_cast<const bf16x8 *>(p);
+      *reinterpret_cast<bf16x8 *>(out + (size_t)j * 8) = *reinterpret_cast<const bf16x8 *>(src);
     else
-      dst[(size_t)x * C + c] = *p;
+      out[j] = *src;
   }
 }
 
@@ -796,21 +785,20 @@ __global__ __launch_bounds__(256) void k_up2_concat_bwd(const bf16 *__restrict__
        j += (Ix)gridDim.x * blockDim.x) {
     if (j < na) {
       const Ix p = ag(j), q = wc(p), r = hc(q), n = dc(r);
-      const int c = (int)(j - p * ag.d) * V, x = (int)(p - q * wc.d), y = (int)(q - r * hc.d),
-                z = (int)(r - n * dc.d);
-      const bf16 *src = g + ((((size_t)n * D + 2 * z) * H + 2 * y) * W + 2 * x) * C + c;
+      const Ix c = (j - p * ag.d) * V, x = p - q * wc.d, y = q - r * hc.d, z = r - n * dc.d;
+      const bf16 *src = g + ((((n * D + 2 * z) * H + 2 * y) * W + 2 * x) * C + c);
       float s[V] = {};
 #pragma unroll
       for (int k = 0; k < 8; k++) {
         float v[V];
-        ldv<V>(src + (((size_t)(k >> 2) * H + ((k >> 1) & 1)) * W + (k & 1)) * C, v);
+        ldv<V>(src + (((Ix)(k >> 2) * H + ((k >> 1) & 1)) * W + (k & 1)) * C, v);
 #pragma unroll
         for (int u = 0; u < V; u++) s[u] += v[u];
       }
       stv<V>(ga + (size_t)j * V, s);
     } else {
       const Ix i = j - na, v = bg(i);
-      const bf16 *src = g + (size_t)v * C + Ca + (size_t)(i - v * bg.d) * V;
+      const bf16 *src = g + (v * C + Ca + (i - v * bg.d) * V);
       if constexpr (V == 8)
         *reinterpret_cast<bf16x8 *>(gb + (size_t)i * 8) = *reinterpret_cast<const bf16x8 *>(src);
       else
@@ -1218,52 +1206,70 @@ extern "C" int tb_nn_relu_bwd(const void *y, void *g, int64_t count, void *strea
   return 0;
 }
 
-// blocks of the row kernels: one per row of an n x d x h volume
-static int row_blocks(long long n, long long d, long long h, unsigned *out) {
-  const long long r = n * d * h;
-  if (r > 0x7fffffffLL) return nn_fail("volume too large");
-  *out = r > 0 ? (unsigned)r : 0u;
-  return 0;
+// Blocks of the kernels over voxels' items: 32 a CU at most, so a thread of a
+// large volume takes several (concatenation's backward pass, 2 x 16 x 256 x 256
+// voxels, 32 + 32 channels: 111 us with a block for every 256 items, 95 so).
+static int item_grid(size_t n) { return std::min(grid1d(n), 8192); }
+
+// The kernels over voxels, by index type and channels a thread.  32-bit indices
+// serve volumes below 2^31 items.
+static bool small_index(int n, int d, int h, int wd, long long c) {
+  return (double)n * d * h * wd * (double)c < 2147483647.0;
+}
+
+template <int V, class Ix>
+static void avgpool2(const void *in, void *out, int n, int d, int h, int wd, int c, bool backward,
+                     hipStream_t s) {
+  const int k = backward ? 1 : 2;
+  d /= k, h /= k, wd /= k;  // the output's size
+  const size_t total = (size_t)n * d * h * wd * (c / V);
+  hipLaunchKernelGGL((backward ? k_avgpool2_bwd<V, Ix> : k_avgpool2<V, Ix>), dim3(item_grid(total)),
+                     dim3(256), 0, s, static_cast<const bf16 *>(in), static_cast<bf16 *>(out), c,
+                     (Ix)total, make_div<Ix>(c / V), make_div<Ix>(wd), make_div<Ix>(h),
+                     make_div<Ix>(d));
 }
 
 extern "C" int tb_nn_avgpool2(const void *in, void *out, int32_t n, int32_t d, int32_t h,
                               int32_t wd, int32_t c, int32_t backward, void *stream) {
   if (d % 2 || h % 2 || wd % 2) return nn_fail("tb_nn_avgpool2: odd size");
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || c <= 0) return 0;
   const bool vec = c % 8 == 0 && al16(in) && al16(out);
-  const int k = backward ? 1 : 2;
-  unsigned rows = 0;
-  if (row_blocks(n, d / k, h / k, &rows)) return -1;
-  if (!rows) return 0;
-  auto fn = backward ? (vec ? k_avgpool2_bwd<8> : k_avgpool2_bwd<1>)
-                     : (vec ? k_avgpool2<8> : k_avgpool2<1>);
-  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, s, static_cast<const bf16 *>(in),
-                     static_cast<bf16 *>(out), d, h, wd, c);
+  const bool small = small_index(n, d, h, wd, c);
+  auto fn = vec ? (small ? avgpool2<8, uint32_t> : avgpool2<8, uint64_t>)
+                : (small ? avgpool2<1, uint32_t> : avgpool2<1, uint64_t>);
+  fn(in, out, n, d, h, wd, c, backward != 0, static_cast<hipStream_t>(stream));
   NNCHK("tb_nn_avgpool2");
   return 0;
 }
 
+template <int V, class Ix>
+static void up2_concat(const void *a, const void *b, void *out, int n, int d, int h, int wd, int ca,
+                       int cb, hipStream_t s) {
+  const size_t total = (size_t)n * d * h * wd * ((ca + cb) / V);
+  hipLaunchKernelGGL((k_up2_concat<V, Ix>), dim3(item_grid(total)), dim3(256), 0, s,
+                     static_cast<const bf16 *>(a), static_cast<const bf16 *>(b),
+                     static_cast<bf16 *>(out), ca, cb, (Ix)total, make_div<Ix>((ca + cb) / V),
+                     make_div<Ix>(wd), make_div<Ix>(h), make_div<Ix>(d));
+}
+
 extern "C" int tb_nn_up2_concat(const void *a, const void *b, void *out, int32_t n, int32_t d,
                                 int32_t h, int32_t wd, int32_t ca, int32_t cb, void *stream) {
-  unsigned rows = 0;
-  if (row_blocks(n, d, h, &rows)) return -1;
-  if (!rows) return 0;
-  auto fn = ca % 8 == 0 && cb % 8 == 0 && al16(a) && al16(b) && al16(out) ? k_up2_concat<8>
-                                                                          : k_up2_concat<1>;
-  hipLaunchKernelGGL(fn, dim3(rows), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const bf16 *>(a), static_cast<const bf16 *>(b),
-                     static_cast<bf16 *>(out), d, h, wd, ca, cb);
+  if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || ca + cb <= 0) return 0;
+  const bool vec = ca % 8 == 0 && cb % 8 == 0 && al16(a) && al16(b) && al16(out);
+  const bool small = small_index(n, d, h, wd, (long long)ca + cb);
+  auto fn = vec ? (small ? up2_concat<8, uint32_t> : up2_concat<8, uint64_t>)
+                : (small ? up2_concat<1, uint32_t> : up2_concat<1, uint64_t>);
+  fn(a, b, out, n, d, h, wd, ca, cb, static_cast<hipStream_t>(stream));
   NNCHK("tb_nn_up2_concat");
   return 0;
 }
 
-// index type and channels a thread, by the items' number and the operands
 template <int V, class Ix>
 static void up2_concat_bwd(const void *g, void *ga, void *gb, int n, int d, int h, int wd, int ca,
                            int cb, hipStream_t s) {
   const size_t na = (size_t)n * (d / 2) * (h / 2) * (wd / 2) * (ca / V);
   const size_t total = na + (size_t)n * d * h * wd * (cb / V);
-  hipLaunchKernelGGL((k_up2_concat_bwd<V, Ix>), dim3(grid1d(total)), dim3(256), 0, s,
+  hipLaunchKernelGGL((k_up2_concat_bwd<V, Ix>), dim3(item_grid(total)), dim3(256), 0, s,
                      static_cast<const bf16 *>(g), static_cast<bf16 *>(ga),
                      static_cast<bf16 *>(gb), d, h, wd, ca, cb, (Ix)na, (Ix)total,
                      make_div<Ix>(ca / V), make_div<Ix>(cb / V), make_div<Ix>(wd / 2),
@@ -1272,8 +1278,9 @@ static void up2_concat_bwd(const void *g, void *ga, void *gb, int n, int d, int 
 
 extern "C" int tb_nn_up2_concat_bwd(const void *g, void *ga, void *gb, int32_t n, int32_t d,
                                     int32_t h, int32_t wd, int32_t ca, int32_t cb, void *stream) {
+  if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || ca + cb <= 0) return 0;
   const bool vec = ca % 8 == 0 && cb % 8 == 0 && al16(g) && al16(ga) && al16(gb);
-  const bool small = (size_t)n * d * h * wd * ((size_t)ca + cb) < 0x7fffffffu;
+  const bool small = small_index(n, d, h, wd, (long long)ca + cb);
   auto fn = vec ? (small ? up2_concat_bwd<8, uint32_t> : up2_concat_bwd<8, uint64_t>)
                 : (small ? up2_concat_bwd<1, uint32_t> : up2_concat_bwd<1, uint64_t>);
   fn(g, ga, gb, n, d, h, wd, ca, cb, static_cast<hipStream_t>(stream));
