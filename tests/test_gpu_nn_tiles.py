@@ -333,3 +333,40 @@ def test_pooling_of_more_rows_than_one_launch_has_blocks(L):
     X, o = bf(x), empty((n,), "bf16")
     assert L.tb_nn_avgpool2(ptr(X), ptr(o), n, 2, 2, 2, 1, 0, None) == 0
     np.testing.assert_array_equal(host(o), x.mean(1))
+
+
+@pytest.mark.parametrize("cin", [32, 64, 96, 128, 192])
+@pytest.mark.parametrize("cout", [32, 64, 96, 192])
+@pytest.mark.parametrize("shape", [(1, 2, 5, 64), (197, 1, 8, 64), (195, 2, 9, 33), (130, 4, 1, 20),
+                                   (23, 6, 3, 70)])
+def test_conv3d_forms_give_the_same_bits(L, cin, cout, shape):
+    """Launches small enough for 32 channels a wave, larger ones with 64 and 96
+    and with two strips, and rows too few for the staged kernel: bit for bit
+    the unstaged kernel's (the output stored at an odd address)."""
+    log(f"conv forms {shape} {cin}->{cout}")
+    rng = np.random.default_rng(cin + cout)
+    x, w = bf(rng.standard_normal(shape + (cin,))), bf(rng.standard_normal((27, cout, cin)) / 30)
+    bias, size = dev(rng.standard_normal(cout)), int(np.prod(shape)) * cout
+    y1, y2 = empty((size,), "bf16"), empty((size + 8,), "bf16")
+    assert L.tb_nn_conv3d(ptr(x), ptr(w), ptr(bias), ptr(y1), *shape, cin, cout, 0, 0, None) == 0
+    assert L.tb_nn_conv3d(ptr(x), ptr(w), ptr(bias), at(y2, 1, 2), *shape, cin, cout, 0, 0, None) == 0
+    assert np.abs(host(y1)).max() > 0
+    np.testing.assert_array_equal(host(y1), host(y2)[1:size + 1])
+
+
+@pytest.mark.parametrize("ca,cb", [(64, 32), (128, 64)])
+@pytest.mark.parametrize("cout", [32, 64, 96])
+@pytest.mark.parametrize("shape", [(2, 2, 6, 40), (100, 4, 6, 64), (70, 4, 10, 34), (150, 4, 2, 16)])
+def test_conv3d_up2cat_forms_give_the_same_bits(L, ca, cb, cout, shape):
+    log(f"conv up2cat forms {shape} {ca}+{cb}->{cout}")
+    rng = np.random.default_rng(ca + cout)
+    n, d, h, w_ = shape
+    a = bf(rng.standard_normal((n, d // 2, h // 2, w_ // 2, ca)))
+    b = bf(rng.standard_normal(shape + (cb,)))
+    w, size = bf(rng.standard_normal((27, cout, ca + cb)) / 30), int(np.prod(shape)) * cout
+    cat, y1, y2 = empty(shape + (ca + cb,), "bf16"), empty((size,), "bf16"), empty((size + 8,), "bf16")
+    assert L.tb_nn_up2_concat(ptr(a), ptr(b), ptr(cat), *shape, ca, cb, None) == 0
+    assert L.tb_nn_conv3d_up2cat(ptr(a), ptr(b), ptr(w), None, ptr(y1), *shape, ca, cb, cout, 1,
+                                 None) == 0
+    assert L.tb_nn_conv3d(ptr(cat), ptr(w), None, at(y2, 1, 2), *shape, ca + cb, cout, 1, 0, None) == 0
+    np.testing.assert_array_equal(host(y1), host(y2)[1:size + 1])

@@ -200,6 +200,7 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
   const int h0 = (int)(g % HB) * HT; g /= HB;
   const int d = g % D, n = g / D;
   const int co0 = ct * 16 * NB;
+  const int hw = h0 + __builtin_amdgcn_readfirstlane(wave) * SP * RPS;  // the wave's first row
   const int xq = row % (WT / 4), yr = row / (WT / 4);
   f32x4 acc[SP][4][NB];
 #pragma unroll
@@ -251,6 +252,8 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
     __syncthreads();
 #pragma unroll 1
     for (int dy = 0; dy < 3; dy++) {
+      // the wave's rows lie past the volume, or the tap's rows all outside it
+      if (hw >= H || hw + dy - 1 >= H || min(hw + SP * RPS, H) + dy < 2) continue;
       const bf16 *wt = wl + (size_t)(dz * 9 + dy * 3) * Cout * Cin;
       // voxels 4 q + t - 1 of chunk c, t = 0 .. 5; of the half-size tensor
       // their parents 2 q + u - 1, u = (t + 1) / 2
@@ -300,7 +303,6 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
         }
     }
   }
-  const int hw = h0 + wave * SP * RPS;  // the wave's first row
   if (hw == 0 || hw + SP * RPS >= H) {
     bool bad = false;
 #pragma unroll
@@ -1016,6 +1018,9 @@ static int grid1d(size_t n) {
   return (int)g;
 }
 
+// blocks of 256 threads in a launch: its threads are counted in 32 bits
+constexpr long long kMaxBlocks = 0xffffffffLL / 256;
+
 static bool al16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 extern "C" const char *tb_nn_last_error(void) { return g_nn_err.c_str(); }
@@ -1056,11 +1061,6 @@ extern "C" int tb_dev_synchronize(void) {
   return 0;
 }
 
-// The staged kernel's launch.  Output channels: 96 at once, else 64, else 32.
-// Strips of 64 x 1 voxels, or 32 x 2 where that leaves fewer lanes without a
-// voxel (and for 128 + 64 input channels, whose tile of 64 leaves one workgroup
-// per CU).  Two strips per wave for 32 output channels of 32 inputs, where the
-// weights' share of the L1 would otherwise bound.
 template <int CA, int CB, int NB, int SP, int WT>
 static int conv_tile(const void *a, const void *in, const void *w, const float *bias, void *out,
                      int n, int d, int h, int wd, int cout, int relu, int out_f32, hipStream_t s) {
@@ -1068,7 +1068,7 @@ static int conv_tile(const void *a, const void *in, const void *w, const float *
   auto fn = k_conv3d_tile<CA, CB, NB, SP, WT>;
   const long long blocks = (long long)n * d * ((h + T::HT - 1) / T::HT) * ((wd + WT - 1) / WT) *
                            (cout / (16 * NB));
-  if (blocks > 0x7fffffffLL) return nn_fail("tb_nn_conv3d: volume too large");
+  if (blocks > kMaxBlocks) return nn_fail("tb_nn_conv3d: volume too large");
   if (T::kBytes > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::kBytes);
@@ -1083,16 +1083,42 @@ static int conv_tile(const void *a, const void *in, const void *w, const float *
 
 using conv_fn = int (*)(const void *, const void *, const void *, const float *, void *, int, int,
                         int, int, int, int, int, hipStream_t);
+// A staged form: its launch, workgroups, and voxels of a plane with its rows and
+// columns filled up to whole tiles.  Strips of 64 x 1 voxels, or 32 x 2 where
+// that leaves fewer lanes without a voxel (and for 128 + 64 input channels,
+// whose tile of 64 leaves one workgroup per CU).
+struct ConvForm {
+  conv_fn fn;
+  long long blocks, slots;
+};
 template <int CA, int CB, int NB, int SP>
-static conv_fn conv_pick(int wd) {
-  const int a64 = (wd + 63) / 64 * 64, a32 = (wd + 31) / 32 * 32;
-  return a32 < a64 || CA == 4 ? conv_tile<CA, CB, NB, SP, 32> : conv_tile<CA, CB, NB, SP, 64>;
+static ConvForm conv_form(long long planes, int h, int wd, int cout) {
+  const bool narrow = CA == 4 || (wd + 31LL) / 32 * 32 < (wd + 63LL) / 64 * 64;
+  const long long WT = narrow ? 32 : 64, HT = 4 * SP * (64 / WT);
+  const long long th = (h + HT - 1) / HT, tw = (wd + WT - 1) / WT;
+  return {narrow ? conv_tile<CA, CB, NB, SP, 32> : conv_tile<CA, CB, NB, SP, 64>,
+          planes * th * tw * (cout / (16 * NB)), th * HT * tw * WT};
 }
+// More output channels a wave use a staged value more often, but a wave's chain
+// is longer: 32 channels while that leaves the chip with at most three workgroups
+// a CU (one where LDS holds one, from 128 input channels on), else 64, else 96.
+// 64 -> 64 channels, 16 planes of 16 x 16 voxels: 36 us with 64 channels a wave,
+// 23 with 32; 128 -> 128, 64 planes of 16 x 32: 66 and 82.  Two strips per wave for
+// 32 channels of 32 inputs, where the weights' share of the L1 would otherwise
+// bound, unless they fill up more rows.
 template <int CA, int CB>
-static conv_fn conv_pick(int cout, int wd) {
-  if (cout % 96 == 0) return conv_pick<CA, CB, 6, 1>(wd);
-  if (cout % 64 == 0) return conv_pick<CA, CB, 4, 1>(wd);
-  return conv_pick<CA, CB, 2, CA == 0 && CB == 1 ? 2 : 1>(wd);
+static ConvForm conv_pick(long long planes, int h, int wd, int cout) {
+  constexpr long long few = CA + CB >= 4 ? 256 : 768;
+  ConvForm f = conv_form<CA, CB, 2, 1>(planes, h, wd, cout);
+  if constexpr (CA == 0 && CB == 1) {
+    if (f.blocks > few && cout % 64 && cout % 96) {
+      const ConvForm g = conv_form<CA, CB, 2, 2>(planes, h, wd, cout);
+      if (g.slots <= f.slots) f = g;
+    }
+  }
+  if (f.blocks > few && cout % 64 == 0) f = conv_form<CA, CB, 4, 1>(planes, h, wd, cout);
+  if (f.blocks > few && cout % 96 == 0) f = conv_form<CA, CB, 6, 1>(planes, h, wd, cout);
+  return f;
 }
 
 extern "C" int tb_nn_conv3d(const void *in, const void *w, const float *bias, void *out,
@@ -1101,19 +1127,25 @@ extern "C" int tb_nn_conv3d(const void *in, const void *w, const float *bias, vo
   if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || cin % 32 || cout % 32 || cin <= 0 || cout <= 0)
     return nn_fail("tb_nn_conv3d: sizes must be positive, channels multiples of 32");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  conv_fn fn = cin == 32    ? conv_pick<0, 1>(cout, wd)
-               : cin == 64  ? conv_pick<0, 2>(cout, wd)
-               : cin == 96  ? conv_pick<0, 3>(cout, wd)
-               : cin == 128 ? conv_pick<0, 4>(cout, wd)
-               : cin == 192 ? conv_pick<0, 6>(cout, wd)
-                            : nullptr;
-  // the staged kernel stores 16 bytes at a time
-  if (fn && reinterpret_cast<uintptr_t>(out) % 16 == 0)
-    return fn(nullptr, in, w, bias, out, n, d, h, wd, cout, relu, out_f32, s);
+  const long long planes = (long long)n * d;
+  const ConvForm f = cin == 32    ? conv_pick<0, 1>(planes, h, wd, cout)
+                     : cin == 64  ? conv_pick<0, 2>(planes, h, wd, cout)
+                     : cin == 96  ? conv_pick<0, 3>(planes, h, wd, cout)
+                     : cin == 128 ? conv_pick<0, 4>(planes, h, wd, cout)
+                     : cin == 192 ? conv_pick<0, 6>(planes, h, wd, cout)
+                                  : ConvForm{nullptr, 0, 0};
+  // Unstaged: volumes of one to three rows that fill the chip, whose tiles are
+  // empty by half and more (512 planes of 1 x 32, 128 -> 128 channels: 81 us
+  // staged, 38 unstaged; 16 planes of it 18 and 23), other channels, an output
+  // that 16-byte stores do not allow, and more tiles than a launch holds.
+  const long long strips = (wd + 63LL) / 64 * 64 * h;
+  const bool empty = f.slots > 2 * strips || (f.slots == 2 * strips && (cin >= 96 || wd <= 8));
+  if (f.fn && al16(out) && !(empty && f.blocks >= 512) && f.blocks <= kMaxBlocks)
+    return f.fn(nullptr, in, w, bias, out, n, d, h, wd, cout, relu, out_f32, s);
   const int MB = 4, NB = 2;
-  const long long waves = (long long)n * d * h * ((wd + 16 * MB - 1) / (16 * MB)) * (cout / (16 * NB));
+  const long long waves = planes * h * ((wd + 16 * MB - 1) / (16 * MB)) * (cout / (16 * NB));
   const long long blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;
-  if (blocks > 0x7fffffffLL) return nn_fail("tb_nn_conv3d: volume too large");
+  if (blocks > kMaxBlocks) return nn_fail("tb_nn_conv3d: volume too large");
   hipLaunchKernelGGL((k_conv3d_fwd<4, 2>), dim3((unsigned)blocks), dim3(64 * kWavesPerBlock), 0,
                      s, static_cast<const bf16 *>(in), static_cast<const bf16 *>(w), bias, out, n,
                      d, h, wd, cin, cout, relu, out_f32);
@@ -1127,9 +1159,10 @@ extern "C" int tb_nn_conv3d_up2cat(const void *a, const void *b, const void *w, 
                                    void *stream) {
   if (n <= 0 || d <= 0 || h <= 0 || wd <= 0 || d % 2 || h % 2 || wd % 2 || cout <= 0 || cout % 32)
     return nn_fail("tb_nn_conv3d_up2cat: sizes must be positive and even, channels multiples of 32");
-  conv_fn fn = ca == 64 && cb == 32    ? conv_pick<2, 1>(cout, wd)
-               : ca == 128 && cb == 64 ? conv_pick<4, 2>(cout, wd)
-                                       : nullptr;
+  const long long planes = (long long)n * d;
+  const conv_fn fn = ca == 64 && cb == 32    ? conv_pick<2, 1>(planes, h, wd, cout).fn
+                     : ca == 128 && cb == 64 ? conv_pick<4, 2>(planes, h, wd, cout).fn
+                                             : nullptr;
   if (!fn) return nn_fail("tb_nn_conv3d_up2cat: 64 + 32 or 128 + 64 input channels");
   if (!al16(a) || !al16(b) || !al16(w) || !al16(out))
     return nn_fail("tb_nn_conv3d_up2cat: a, b, w and out must be 16-byte aligned");
