@@ -370,3 +370,15 @@ def test_conv3d_up2cat_forms_give_the_same_bits(L, ca, cb, cout, shape):
                                  None) == 0
     assert L.tb_nn_conv3d(ptr(cat), ptr(w), None, at(y2, 1, 2), *shape, ca + cb, cout, 1, 0, None) == 0
     np.testing.assert_array_equal(host(y1), host(y2)[1:size + 1])
+
+
+@pytest.mark.parametrize("shape,cin,cout,slices", [
+    ((3, 5, 1, 2), 32, 64, 4), ((40, 3, 2, 5), 64, 32, 7), ((1, 1, 1, 31), 96, 32, 256),
+    ((2, 2, 3, 5), 32, 32, 1),                                       # 32 voxels at a time
+    ((2, 5, 40, 70), 32, 32, 256), ((2, 4, 33, 66), 64, 96, 256), ((1, 9, 50, 31), 96, 32, 5),
+    ((6, 3, 17, 65), 32, 64, 2)])                                    # in tiles
+@pytest.mark.parametrize("off", [0, 1])
+def test_conv3d_wgrad_of_narrow_and_of_large_volumes(L, shape, cin, cout, slices, off):
+    """Either kernel of the weight gradient, to the bound of
+    test_conv3d_wgrad_tiles."""
+    test_conv3d_wgrad_tiles(L, shape, cin, cout, slices, off)

@@ -554,6 +554,74 @@ __global__ __launch_bounds__(kGThreads) void k_conv3d_wgrad(
   }
 }
 
+// The same for volumes whose tiles would be mostly empty (short rows, few of
+// them): a wave owns one tap, 16 MBO output and 16 NBI input channels and one of S
+// slices of the voxels in their order, 32 at a time, whatever row they lie in; its
+// sums go to part[s][tap][co][ci].
+template <int MBO, int NBI>
+__global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_wgrad_flat(
+    const bf16 *__restrict__ in, const bf16 *__restrict__ gout, float *__restrict__ part,
+    int N, int D, int H, int W, int Cin, int Cout, int S) {
+  const int lane = threadIdx.x & 63;
+  const long long g = (long long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  const int OT = Cout / (16 * MBO), IT = Cin / (16 * NBI);
+  const long long total = (long long)S * kTaps * OT * IT;
+  if (g >= total) return;
+  long long r = g;
+  const int it = (int)(r % IT); r /= IT;
+  const int ot = (int)(r % OT); r /= OT;
+  const int tap = (int)(r % kTaps);
+  const int s = (int)(r / kTaps);
+  const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
+  const int row = lane & 15, kq = lane >> 4;
+  const int co0 = ot * 16 * MBO, ci0 = it * 16 * NBI;
+  const long long nvox = (long long)N * D * H * W;
+  const long long nch = (nvox + 31) / 32;
+  const long long c_begin = nch * s / S, c_end = nch * (s + 1) / S;
+  f32x4 acc[MBO][NBI];
+#pragma unroll
+  for (int a = 0; a < MBO; a++)
+#pragma unroll
+    for (int b = 0; b < NBI; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (long long c = c_begin; c < c_end; c++) {
+    bf16x8 av[MBO], bv[NBI];
+#pragma unroll
+    for (int a = 0; a < MBO; a++) av[a] = zero8();
+#pragma unroll
+    for (int b = 0; b < NBI; b++) bv[b] = zero8();
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const long long v = c * 32 + kq * 8 + i;
+      if (v >= nvox) break;
+      long long q = v;
+      const int x = (int)(q % W); q /= W;
+      const int y = (int)(q % H); q /= H;
+      const int z = (int)(q % D);
+      const int nn = (int)(q / D);
+#pragma unroll
+      for (int a = 0; a < MBO; a++) av[a][i] = gout[(size_t)v * Cout + co0 + 16 * a + row];
+      const int zz = z + dz, yy = y + dy, xx = x + dx;
+      if (zz >= 0 && zz < D && yy >= 0 && yy < H && xx >= 0 && xx < W) {
+        const size_t u = (((size_t)nn * D + zz) * H + yy) * (size_t)W + xx;
+#pragma unroll
+        for (int b = 0; b < NBI; b++) bv[b][i] = in[u * Cin + ci0 + 16 * b + row];
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < MBO; a++)
+#pragma unroll
+      for (int b = 0; b < NBI; b++) acc[a][b] = mfma(av[a], bv[b], acc[a][b]);
+  }
+  float *dst = part + ((size_t)s * kTaps + tap) * Cout * Cin;
+#pragma unroll
+  for (int a = 0; a < MBO; a++)
+#pragma unroll
+    for (int b = 0; b < NBI; b++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        dst[(size_t)(co0 + 16 * a + 4 * kq + j) * Cin + ci0 + 16 * b + row] = acc[a][b][j];
+}
+
 // out[i] = sum_s part[s][i]: 16 runs of slices side by side, each in order,
 // then the runs in order.  Block: 64 entries.  (One thread per entry walked the
 // slices one load at a time: 68 us on average over a training step's sums, 15
@@ -1207,6 +1275,27 @@ extern "C" int tb_nn_conv3d_wgrad(const void *in, const void *gout, float *gw, f
   // partial sums: as many as have work, the units shared out evenly
   long long S = std::max<long long>(1, std::min<long long>({(long long)slices, units, want}));
   S = std::max<long long>(1, (units + (units + S - 1) / S - 1) / std::max<long long>((units + S - 1) / S, 1));
+  // A workgroup stages a plane (a unit of several has one and a half more) in about
+  // the time in which a wave of the flat kernel walks 1.25 chunks of 32 voxels (4.6
+  // and 3.7 us); 256 workgroups run at once, and about 2000 such waves.  Volumes of
+  // short rows, few rows or few slices are sooner done by chunks: 512 planes of 1 x 2
+  // voxels, 4 slices, 32 -> 32 channels take 663 us in tiles and 37 by chunks; 16
+  // planes of 48 x 48, 256 slices, 30 and 75.
+  const long long chunks = ((long long)n * d * h * wd + 31) / 32;
+  const long long SF = std::max<long long>(1, std::min<long long>(slices, chunks));
+  const double flat = 1.25 * (double)((chunks + SF - 1) / SF) *
+                      std::max(1.0, (double)(SF * kTaps * pairs) / 2000.0);
+  const double tile = (double)((units + S - 1) / S) * (U.per + (d > 1 ? 1.5 : 0.5)) *
+                      (double)((S * pairs + 255) / 256);
+  const long long flat_blocks = (SF * kTaps * pairs + kWavesPerBlock - 1) / kWavesPerBlock;
+  if (flat < tile && flat_blocks <= kMaxBlocks) {
+    hipLaunchKernelGGL((k_conv3d_wgrad_flat<2, 2>), dim3((unsigned)flat_blocks),
+                       dim3(64 * kWavesPerBlock), 0, s, static_cast<const bf16 *>(in),
+                       static_cast<const bf16 *>(gout), part, n, d, h, wd, cin, cout, (int)SF);
+    sum_parts(part, gw, nw, (int)SF, s);
+    NNCHK("tb_nn_conv3d_wgrad");
+    return 0;
+  }
   const size_t lds = (size_t)(3 * 2 * (kGH + 2) * (kGW + 2) + 2 * kGH * kGW) * 16 * sizeof(bf16);
   auto fn = al16(in) && al16(gout) ? k_conv3d_wgrad<true> : k_conv3d_wgrad<false>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn),
