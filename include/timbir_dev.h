@@ -424,7 +424,7 @@ int tb_nn_head_bwd(const void *h, const float *w, const float *gout, void *gh, f
  * fp64 sums of squares of `blocks` blocks. */
 int tb_nn_mse(const float *out, const float *target, float *gout, double *part, int32_t blocks,
               int64_t nvox, void *stream);
-/* out[i] = sum over s < slices of part[s * count + i], in order. */
+/* out[i] = sum over s < slices of part[s * count + i], in a fixed order. */
 int tb_nn_sum_parts(const float *part, float *out, int64_t count, int32_t slices, void *stream);
 /* Adam step `step` (from 1) on fp32 parameters p with gradient g and moments
  * m, v; wb (may be NULL) receives the bf16 copy. */

@@ -382,3 +382,16 @@ def test_conv3d_wgrad_of_narrow_and_of_large_volumes(L, shape, cin, cout, slices
     """Either kernel of the weight gradient, to the bound of
     test_conv3d_wgrad_tiles."""
     test_conv3d_wgrad_tiles(L, shape, cin, cout, slices, off)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 32768, 32769, 131072, 131073, 200001])
+@pytest.mark.parametrize("slices", [1, 7, 8, 16, 17, 70])
+def test_sum_of_partial_sums(L, n, slices):
+    """Every number of runs and their remainders: within 1e-6 of the sum of
+    magnitudes of the float64 sums (at most 70 fp32 terms)."""
+    log(f"sum parts n={n} slices={slices}")
+    v = np.random.default_rng(n + slices).standard_normal((slices, n)).astype(np.float32)
+    part, out = dev(v), empty((n,))
+    assert L.tb_nn_sum_parts(ptr(part), ptr(out), n, slices, None) == 0
+    want = v.astype(np.float64)
+    assert (np.abs(host(out) - want.sum(0)) <= 1e-6 * np.abs(want).sum(0)).all()

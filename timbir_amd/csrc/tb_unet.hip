@@ -622,33 +622,40 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_wgrad_flat(
         dst[(size_t)(co0 + 16 * a + 4 * kq + j) * Cin + ci0 + 16 * b + row] = acc[a][b][j];
 }
 
-// out[i] = sum_s part[s][i]: 16 runs of slices side by side, each in order,
-// then the runs in order.  Block: 64 entries.  (One thread per entry walked the
-// slices one load at a time: 68 us on average over a training step's sums, 15
-// in this form.)
-constexpr int kSumRuns = 16;
-__global__ __launch_bounds__(64 * kSumRuns) void k_sum_parts(const float *__restrict__ part,
-                                                             float *__restrict__ out, size_t n,
-                                                             int S) {
-  __shared__ float sh[kSumRuns][64];
-  const int col = threadIdx.x & 63, run = threadIdx.x >> 6;
-  const int per = (S + kSumRuns - 1) / kSumRuns;
+// out[i] = sum_s part[s][i]: RUNS runs of slices side by side, each in order with
+// eight loads in flight, then the runs in order.  Block: E entries.
+template <int RUNS, int E>
+__global__ __launch_bounds__(E *RUNS) void k_sum_parts(const float *__restrict__ part,
+                                                       float *__restrict__ out, size_t n, int S) {
+  __shared__ float sh[RUNS][E];
+  const int col = threadIdx.x % E, run = threadIdx.x / E;
+  const int per = (S + RUNS - 1) / RUNS;
   const int s0 = min(run * per, S), s1 = min(s0 + per, S);
-  for (size_t i0 = blockIdx.x * (size_t)64; i0 < n; i0 += (size_t)gridDim.x * 64) {
+  for (size_t i0 = blockIdx.x * (size_t)E; i0 < n; i0 += (size_t)gridDim.x * E) {
     const size_t i = i0 + col;
     float acc = 0.f;
     if (i < n) {
-#pragma unroll 8
-      for (int s = s0; s < s1; s++) acc += part[(size_t)s * n + i];
-    }
-    __syncthreads();
-    sh[run][col] = acc;
-    __syncthreads();
-    if (run == 0 && i < n) {
+      int s = s0;
+      for (; s + 8 <= s1; s += 8) {
+        float v[8];
 #pragma unroll
-      for (int r = 1; r < kSumRuns; r++) acc += sh[r][col];
-      out[i] = acc;
+        for (int k = 0; k < 8; k++) v[k] = part[(size_t)(s + k) * n + i];
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc += v[k];
+      }
+#pragma unroll 1
+      for (; s < s1; s++) acc += part[(size_t)s * n + i];
     }
+    if constexpr (RUNS > 1) {
+      __syncthreads();
+      sh[run][col] = acc;
+      __syncthreads();
+      if (run == 0) {
+#pragma unroll
+        for (int r = 1; r < RUNS; r++) acc += sh[r][col];
+      }
+    }
+    if (run == 0 && i < n) out[i] = acc;
   }
 }
 
@@ -1246,9 +1253,20 @@ extern "C" int tb_nn_conv3d_flip(const void *w, void *wt, int32_t cin, int32_t c
   return 0;
 }
 
+template <int RUNS, int E>
+static void sum_parts_runs(const float *part, float *out, size_t n, int slices, hipStream_t s) {
+  const unsigned blocks =
+      (unsigned)std::min<size_t>(std::max<size_t>((n + E - 1) / E, 1), 65536);
+  hipLaunchKernelGGL((k_sum_parts<RUNS, E>), dim3(blocks), dim3(E * RUNS), 0, s, part, out, n,
+                     slices);
+}
+// As many runs as give the chip its 2^19 threads: 27648 entries of 256 slices take
+// 9 us in one run, 4 in 16; 331776 entries of 32 slices 8 in one, 20 in 16.  (One
+// thread per entry and one load at a time took 26 and 11.)
 static void sum_parts(const float *part, float *out, size_t n, int slices, hipStream_t s) {
-  const unsigned blocks = (unsigned)std::min<size_t>(std::max<size_t>((n + 63) / 64, 1), 65536);
-  hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(64 * kSumRuns), 0, s, part, out, n, slices);
+  if (n <= (1u << 19) / 16) sum_parts_runs<16, 64>(part, out, n, slices, s);
+  else if (n <= (1u << 19) / 4) sum_parts_runs<4, 64>(part, out, n, slices, s);
+  else sum_parts_runs<1, 256>(part, out, n, slices, s);
 }
 
 extern "C" int tb_nn_conv3d_wgrad(const void *in, const void *gout, float *gw, float *part,
