@@ -395,3 +395,27 @@ def test_sum_of_partial_sums(L, n, slices):
     assert L.tb_nn_sum_parts(ptr(part), ptr(out), n, slices, None) == 0
     want = v.astype(np.float64)
     assert (np.abs(host(out) - want.sum(0)) <= 1e-6 * np.abs(want).sum(0)).all()
+
+
+@pytest.mark.parametrize("c", [8, 32, 200, 1024, 4200, 3, 70, 600])
+@pytest.mark.parametrize("nv,slices", [(1, 1), (5, 9), (700, 2), (900, 300)])
+def test_sums_over_voxels_of_any_width(L, c, nv, slices):
+    """The bias gradient and the head's: channel groups of every size of a
+    block and more than one block holds, more slices than voxels; within 1e-5
+    of the sum of magnitudes, the activation gradient bit for bit."""
+    log(f"channel sums c={c} nv={nv} slices={slices}")
+    rng = np.random.default_rng(c + nv)
+    x = U.bf16(rng.standard_normal((nv, c)).astype(np.float32))
+    w, g = (rng.standard_normal(k).astype(np.float32) for k in (c, nv))
+    xt, wt, gt, out, part = bf(x), dev(w), dev(g), empty((c,)), empty((slices * (c + 1),))
+    assert L.tb_nn_channel_sum(ptr(xt), ptr(out), ptr(part), slices, nv, c, None) == 0
+    ref = x.astype(np.float64)
+    assert (np.abs(host(out) - ref.sum(0)) <= 1e-5 * np.abs(ref).sum(0)).all()
+    gh, hb = empty((nv, c), "bf16"), empty((c + 1,))
+    assert L.tb_nn_head_bwd(ptr(xt), ptr(wt), ptr(gt), ptr(gh), ptr(part), slices, nv, c, 2.0,
+                            None) == 0
+    assert L.tb_nn_sum_parts(ptr(part), ptr(hb), c + 1, slices, None) == 0
+    gs = g * np.float32(0.5)
+    np.testing.assert_array_equal(host(gh), U.bf16(gs[:, None] * w[None]))
+    terms = np.concatenate([ref, np.ones((nv, 1))], 1) * gs[:, None].astype(np.float64)
+    assert (np.abs(host(hb) - terms.sum(0)) <= 1e-5 * np.abs(terms).sum(0)).all()

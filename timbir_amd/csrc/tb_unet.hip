@@ -717,23 +717,43 @@ static Div<Ix> make_div(long long d) {
   return r;
 }
 
-// A block's per-channel sums, combined over its threads: thread t holds V
-// channels of group t % nc in acc, the threads past a whole number of groups
-// nothing
+// A block's sums by channel: thread t holds V channels of group t % nc of one of
+// the block's vs voxels, t / nc, of which the first nd have any.  All its channels
+// go through LDS at once, then as many threads an output as the block has add
+// parts of the voxels, and one adds the parts: two short chains.  (A channel at a
+// time and one thread an output, a head's backward pass of 64 voxels took 40 us, 5
+// so.)  sh: BS V + BS floats.
 template <int V, int BS>
-__device__ __forceinline__ void block_channel_sum(const float (&acc)[V], int nc, float *sh,
+__device__ __forceinline__ void block_channel_sum(const float (&acc)[V], int nc, int nd, float *sh,
                                                   float *out) {
-  const int per = BS / nc * nc;
+  const int t = threadIdx.x, no = nc * V;
+  __syncthreads();
 #pragma unroll
-  for (int k = 0; k < V; k++) {
-    __syncthreads();
-    sh[threadIdx.x] = acc[k];
-    __syncthreads();
-    if ((int)threadIdx.x < nc) {
+  for (int k = 0; k < V; k++) sh[t * V + k] = acc[k];
+  __syncthreads();
+  const int parts = min(min(BS / no, 16), nd);
+  if (parts <= 1) {
+    for (int o = t; o < no; o += BS) {
       float s = 0.f;
-      for (int t = threadIdx.x; t < per; t += nc) s += sh[t];
-      out[threadIdx.x * V + k] = s;
+      for (int d = 0; d < nd; d++) s += sh[d * no + o];
+      out[o] = s;
     }
+    return;
+  }
+  float *sp = sh + BS * V;
+  const int o = t % no, p = t / no;
+  if (p < parts) {
+    float s = 0.f;
+#pragma unroll 4
+    for (int d = p; d < nd; d += parts) s += sh[d * no + o];
+    sp[t] = s;
+  }
+  __syncthreads();
+  if (p == 0) {
+    float s = sp[o];
+#pragma unroll 4
+    for (int q = 1; q < parts; q++) s += sp[q * no + o];
+    out[o] = s;
   }
 }
 
@@ -745,7 +765,7 @@ template <int V>
 __global__ __launch_bounds__(256) void k_channel_sum(const bf16 *__restrict__ g,
                                                      float *__restrict__ part, long long nvox,
                                                      int C, int S) {
-  __shared__ float sh[256];
+  __shared__ float sh[256 * V + 256];
   const int s = blockIdx.x, CG = C / V;
   const long long v0 = nvox * s / S, v1 = nvox * (s + 1) / S;
   for (int c0 = 0; c0 < CG; c0 += 256) {
@@ -761,7 +781,8 @@ __global__ __launch_bounds__(256) void k_channel_sum(const bf16 *__restrict__ g,
         for (int k = 0; k < V; k++) acc[k] += x[k];
       }
     }
-    block_channel_sum<V, 256>(acc, nc, sh, part + (size_t)s * C + c0 * V);
+    block_channel_sum<V, 256>(acc, nc, (int)min((long long)vs, v1 - v0), sh,
+                              part + (size_t)s * C + c0 * V);
   }
 }
 
@@ -973,51 +994,49 @@ __global__ void k_mse(const float *__restrict__ out, const float *__restrict__ t
 // the weight sums, once a thread per channel walking the slice's voxels, were
 // the whole of its 417 us for 4 x 8 x 128 x 128 voxels; now 55.
 // S 0: gh alone, the blocks sharing its voxels; C 0: the bias gradient alone.
-template <int V>
-__global__ __launch_bounds__(512) void k_head_bwd(const bf16 *__restrict__ h,
-                                                  const float *__restrict__ w,
-                                                  const float *__restrict__ gout,
-                                                  bf16 *__restrict__ gh, float *__restrict__ part,
-                                                  long long nvox, int C, int S, float inv_scale) {
-  __shared__ float sh[512];
+template <int V, int BS>
+__global__ __launch_bounds__(BS) void k_head_bwd(const bf16 *__restrict__ h,
+                                                 const float *__restrict__ w,
+                                                 const float *__restrict__ gout,
+                                                 bf16 *__restrict__ gh, float *__restrict__ part,
+                                                 long long nvox, int C, int S, float inv_scale) {
+  __shared__ float sh[BS * V + BS];
   const int s = blockIdx.x, CG = C / V;
   const long long v0 = nvox * s / gridDim.x, v1 = nvox * (s + 1) / gridDim.x;
-  for (int c0 = 0; c0 == 0 || c0 < CG; c0 += 512) {
-    const int nc = max(min(512, CG - c0), 1), vs = 512 / nc;
+  for (int c0 = 0; c0 == 0 || c0 < CG; c0 += BS) {
+    const int nc = max(min(BS, CG - c0), 1), vs = BS / nc;
     const int cg = (int)threadIdx.x % nc, dv = (int)threadIdx.x / nc, c = (c0 + cg) * V;
-    float acc[V] = {}, wc[V] = {}, gs = 0.f;
+    const int nd = (int)min((long long)vs, v1 - v0);
+    const long long begin = dv < vs ? v0 + dv : v1;
+    float gs = 0.f;
     if (CG > 0) {
+      float acc[V] = {}, wc[V];
 #pragma unroll
       for (int k = 0; k < V; k++) wc[k] = w[c + k];
-    }
-    if (dv < vs) {
 #pragma unroll 4
-      for (long long v = v0 + dv; v < v1; v += vs) {
+      for (long long v = begin; v < v1; v += vs) {
         const float g = gout[v] * inv_scale;
-        if (CG > 0) {
-          float x[V], o[V];
-          ldv<V>(h + (size_t)v * C + c, x);
+        float x[V], o[V];
+        ldv<V>(h + (size_t)v * C + c, x);
 #pragma unroll
-          for (int k = 0; k < V; k++) {
-            o[k] = g * wc[k];
-            acc[k] += g * x[k];
-          }
-          stv<V>(gh + (size_t)v * C + c, o);
+        for (int k = 0; k < V; k++) {
+          o[k] = g * wc[k];
+          acc[k] += g * x[k];
         }
+        stv<V>(gh + (size_t)v * C + c, o);
         gs += g;
       }
+      if (S > 0) block_channel_sum<V, BS>(acc, nc, nd, sh, part + (size_t)s * (C + 1) + c0 * V);
+    } else {
+      for (long long v = begin; v < v1; v += vs) gs += gout[v] * inv_scale;
     }
-    if (S <= 0) continue;
-    if (CG > 0) block_channel_sum<V, 512>(acc, nc, sh, part + (size_t)s * (C + 1) + c0 * V);
-    if (c0 == 0) {
+    if (c0 == 0 && S > 0) {
+      // the bias, which the first thread of each voxel has
       __syncthreads();
-      sh[threadIdx.x] = gs;
+      if (cg == 0) sh[dv] = gs;
       __syncthreads();
-      if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int k = 0; k < vs; k++) t += sh[k * nc];
-        part[(size_t)s * (C + 1) + C] = t;
-      }
+      const float bias[1] = {sh[threadIdx.x]};
+      block_channel_sum<1, BS>(bias, 1, nd, sh, part + (size_t)s * (C + 1) + C);
     }
   }
 }
@@ -1466,9 +1485,14 @@ extern "C" int tb_nn_head(const void *h, const float *w, const float *b, const f
 extern "C" int tb_nn_head_bwd(const void *h, const float *w, const float *gout, void *gh,
                               float *part, int32_t slices, int64_t nvox, int32_t c, float scale,
                               void *stream) {
-  auto fn = c % 8 == 0 && al16(h) && al16(gh) ? k_head_bwd<8> : k_head_bwd<1>;
+  // one wave a slice where it has no more to do (2048 slices of 5000 voxels x 32
+  // channels: 9 us with eight, 4 with one)
+  const bool vec = c % 8 == 0 && al16(h) && al16(gh);
   const int blocks = slices > 0 ? slices : grid1d((size_t)(nvox + 127) / 128);
-  hipLaunchKernelGGL(fn, dim3(blocks), dim3(512), 0, static_cast<hipStream_t>(stream),
+  const bool one = (nvox / blocks + 1) * (double)(vec ? c / 8 : c) <= 64.0;
+  auto fn = vec ? (one ? k_head_bwd<8, 64> : k_head_bwd<8, 512>)
+                : (one ? k_head_bwd<1, 64> : k_head_bwd<1, 512>);
+  hipLaunchKernelGGL(fn, dim3(blocks), dim3(one ? 64 : 512), 0, static_cast<hipStream_t>(stream),
                      static_cast<const bf16 *>(h), w, gout, static_cast<bf16 *>(gh), part,
                      (long long)nvox, c, slices, 1.f / scale);
   NNCHK("tb_nn_head_bwd");
