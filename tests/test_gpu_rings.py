@@ -2,12 +2,18 @@
 neighbours and records of a voxel are in flight while they are updated, voxel
 lists shorter than a group, and entries at the generalized-Huber threshold,
 where the rounded decision hands over to the exact one."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
 import timbir_amd as tb
 from oracle import pyorc
 from timbir_amd import datagen
+
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+from test_gpu_parity import check_kernel  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +81,38 @@ def test_huber_threshold(kern, T):
         g.close()
     finally:
         tb.set_options(kernel=old)
+
+
+@pytest.mark.parametrize("raster", [0, 1])
+@pytest.mark.parametrize("kern,N,nz,views,mult", [
+    (4, 4, 2, 400, (1, 1)), (4, 8, 2, 700, (1, 1)),                            # records RD 2: 2 and 4 views a lane
+    (4, 10, 4, 90, (2, 2)), (4, 16, 4, 170, (2, 2)), (4, 8, 4, 300, (2, 2)),   # 5 bins x 2 rows, 15 slots, 2 views
+    (4, 16, 8, 100, (4, 4)), (4, 20, 8, 180, (4, 4)), (4, 24, 4, 90, (4, 2)),  # 9 bins x 4 rows: RD 4; 2 rows
+    (3, 10, 4, 40, (2, 2)), (3, 22, 4, 90, (2, 2)), (0, 16, 8, 60, (4, 4))])
+def test_voxels_in_flight_of_wide_columns(kern, N, nz, views, mult, raster):
+    """test_voxels_in_flight for the record rings of two and four records, the
+    columns of several rows, several views a lane and the exchange of 15 slots:
+    lists shorter than the rings, to the same bounds."""
+    print(f"in flight N={N} nz={nz} views={views} mult={mult} raster={raster} kernel={kern}", flush=True)
+    scan = datagen.tiny(N=N, nz=nz, n_frames=2, n_views=2 * views, sig_s=0.005, sig_t=0.01,
+                        convg_thresh=0.0, quad_convex=0, c_s=1.0, c_t=1.0)
+    old = tb.get_options()
+    tb.set_options(hicd_order=raster, kernel=kern)
+    try:
+        o = pyorc.Problem(scan, mult_xy=mult[0], mult_z=mult[1],
+                          opt=pyorc.options(schedule=pyorc.SCHED_COLOUR, hicd_order=raster))
+        g = tb.Stage(scan, mult_xy=mult[0], mult_z=mult[1])
+        o.init_error_sino()
+        g.init_error_sino()
+        for it in range(1, 4):
+            o.icd_iteration(it)
+            g.icd_iteration(it)
+            xo, xg = o.obj(), g.object()
+            rmse = np.sqrt(np.mean((xg - xo) ** 2)) / (xo.max() - xo.min())
+            assert rmse < 1e-4, (it, rmse)
+            eo, eg = o.err(), g.error_sino()
+            assert np.abs(eg - eo).max() <= 1e-4 * np.abs(eo).max()
+        check_kernel(g, kern)
+        g.close()
+    finally:
+        tb.set_options(kernel=old.kernel, hicd_order=old.hicd_order)
