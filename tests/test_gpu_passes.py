@@ -152,3 +152,37 @@ def test_fbp_of_a_groups_remainder(N, nz, shift):
     """The numbers of slices in the last group that test_fbp_groups_and_edges
     has not, each its own kernel and row stride, to the same bound."""
     test_fbp_groups_and_edges(N, nz, shift)
+
+
+@pytest.mark.parametrize("where", ["one", "pair", "ends"])
+def test_prior_cost_at_infinities_and_the_largest_values(where):
+    """The numpy statement's value where the fast form's FP32 range ends: a
+    difference with an infinity and of two infinities (both NaN there), and of
+    the largest finite values of either sign (within 1e-12, as above)."""
+    print(f"prior cost {where}", flush=True)
+    scan = scan_of(9, 2, n_frames=2, n_views=12)
+    st = tb.Stage(scan)
+    x = np.random.default_rng(2).normal(0, 1, st.obj_shape).astype(np.float32)
+    if where == "ends":
+        x = (np.sign(x) * np.finfo(np.float32).max).astype(np.float32)
+    else:
+        x[0, 1, 4, 4] = np.inf
+        if where == "pair":
+            x[0, 1, 4, 5] = np.inf
+    st.set_object(x)
+    got = st.cost()[2]
+    i, f = st.info, st.sfilt
+    st.close()
+    with np.errstate(invalid="ignore", over="ignore"):
+        xd, ref = x.astype(np.float64), 0.0
+        for dz, dy, dx in [(a, b, c) for a in (0, 1) for b in (-1, 0, 1) for c in (-1, 0, 1)
+                           if (a, b, c) > (0, 0, 0)]:
+            a = xd[:, :2 - dz, max(0, -dy):9 - max(0, dy), max(0, -dx):9 - max(0, dx)]
+            b = xd[:, dz:, max(0, dy):9 - max(0, -dy), max(0, dx):9 - max(0, -dx)]
+            ref += f[dz + 1, dy + 1, dx + 1] * mathref.rho(a - b, i["sigS_q"], i["sigS_qp"],
+                                                           i["c_s"]).sum()
+        ref += i["tfilt"] * mathref.rho(xd[:-1] - xd[1:], i["sigT_q"], i["sigT_qp"], i["c_t"]).sum()
+    if where == "ends":
+        assert np.isfinite(ref) and abs(got - ref) <= 1e-12 * abs(ref), (got, ref)
+    else:
+        assert np.isnan(ref) and np.isnan(got), (got, ref)
