@@ -126,8 +126,9 @@ __global__ void k_upsample(const float *__restrict__ in, float *__restrict__ out
 // numbered view-major inside each XCD's share (block b runs on XCD b mod
 // 8), so one XCD's L2 holds the objects of few frames.
 //
-// Bound: FP64 arithmetic.  A column is nonzero at bin j only where the pixel's
-// centre projects within 64 OffsetR = delta_xy / sqrt(2) + delta_r / 2 of the
+// Bound: vector issue (52% of the cycles at four an instruction, half of them
+// FP64 arithmetic and a third conversions).  A column is nonzero at bin j only
+// where the pixel's centre projects within 64 OffsetR = delta_xy / sqrt(2) + delta_r / 2 of the
 // bin's centre, and there calcAMatrixColumnforAngle's other limits (first and
 // last bin, the detector's ends) hold by 0.29 delta_xy, so a thread visits
 // only the columns of a row inside that reach (widened by 1e-6 of a pixel) and
@@ -294,7 +295,8 @@ __global__ __launch_bounds__(kFwdT) void k_forward(KP P, const int *__restrict__
 //     f of q at the pixel's ray, linearly interpolated between bin centres;
 //     zero outside the reconstruction mask.
 //
-// Bound: FP64 arithmetic and the L1 reads of q.  The filter keeps the kernel's
+// Bound: vector issue, 88% of the filter's cycles and 67% of the back-
+// projection's, a third to a half of it FP64.  The filter keeps the kernel's
 // odd taps in LDS (no division per tap), takes `per` slices of a view at once
 // and gives a thread kFbpF outputs of one parity, which share each sample and
 // all but one tap.  The back-projection's geometry (ray, bin, fraction)
@@ -404,7 +406,8 @@ __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict_
           ld_slices<NZ>(qv + (size_t)j0 * NZ, a);
           ld_slices<NZ>(qv + (size_t)j0 * NZ + NZ, b);
 #pragma unroll
-          for (int i = 0; i < NZ; i++) acc[i] = fma(t, (double)b[i], fma(1.0 - t, (double)a[i], acc[i]));
+          for (int i = 0; i < NZ; i++)
+            acc[i] = fma(t, (double)b[i], fma(1.0 - t, (double)a[i], acc[i]));
         } else if (j0 == -1 || j0 == P.N_r - 1) {
           // one of the two bins is off the detector
           const float *a = qv + (size_t)max(j0, 0) * NZ;
@@ -876,9 +879,11 @@ __device__ __forceinline__ double qggmrf_value_fast(double d, double inv_sq, dou
 // outside the volume is the voxel with itself (value zero), so every lane runs
 // the 14 pairs side by side.  A voxel with a value the fast form does not
 // hold for, and every voxel when c is not positive, takes the plain one.
-// FP64 arithmetic bounds it: with pow, three FP64 divisions per pair and
-// 64-bit index divisions Stage.cost took 3.49 ms for 512 x 512 x 16 slices x 8
-// frames and 512 views, with this form 0.90 ms; reading the object takes 0.03.
+// Vector issue bounds it (60% of the cycles at four an instruction, half of them
+// FP64 arithmetic; conversions and the FP32 units take more than four): with pow,
+// three FP64 divisions per pair and 64-bit index divisions Stage.cost took 3.49
+// ms for 512 x 512 x 16 slices x 8 frames and 512 views, with this form 0.90 ms;
+// reading the object takes 0.03.
 __global__ __launch_bounds__(256) void k_cost_prior(KP P, double sSq, double sSqp, double cs,
                                                     double sTq, double sTqp, double ct,
                                                     const double *__restrict__ sfilt, double tfilt,
@@ -1022,8 +1027,8 @@ __global__ __launch_bounds__(kVscThreads) void k_vsc_select(KP P, const float *_
     }
   };
   // fn(pixel, value, mask bit) over the wave's range, step by step, in every
-  // lane of the wave.  A lane past the range holds all ones: above every value in the ranking, so that no rank counts it,
-  // and a NaN, above no threshold.
+  // lane of the wave.  A lane past the range holds all ones: above every value
+  // in the ranking, so that no rank counts it, and a NaN, above no threshold.
   auto walk = [&](bool with_mask, auto fn) {
     for (int i0 = w0; R ? i0 == w0 : i0 < w1; i0 += 64 * U) {
       if (!R) load(i0, with_mask);

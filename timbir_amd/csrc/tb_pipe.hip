@@ -1170,7 +1170,8 @@ template __global__ void k_icd_mw_m<5, 2, 2, 3>(const KP *, const int4 *, int, i
 // hidden altogether.  Before and after waiting for everything at each
 // voxel, a pass: 192 x 192, 5 bins x 2 rows, 128 views, 32 cells 60.8 and
 // 57.9 ms; twelve 128 x 128 and 192 x 192 problems of 180 views, 24 cells a
-// launch 72.3 and 66.9 ms; 512 x 512, 128 views, 256 cells 90.7 and 88.9 ms.
+// launch 72.3 and 66.9 ms; 512 x 512, 128 views, 256 cells 90.7 and 88.9 ms (49 of
+// them with every row in the L2: the chain).
 // ---------------------------------------------------------------------------
 template <int MZ>
 __device__ __forceinline__ void ld_rows(const float *p, float (&o)[MZ]) {

@@ -167,9 +167,12 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_conv3d_fwd(
 // the bits are the same.  Rows above and below the volume are zeros in LDS; a
 // weight that is infinite or NaN makes those NaN, so a wave that finds such a
 // sum in the volume's first or last row takes conv_strip for its strips, which
-// leaves those taps out.  2 x 16 x 256 x 256 voxels, before and now: 32 -> 32
-// channels 0.38 and 0.18 ms (650 TFLOP/s); 64 + 32 -> 32 with its
-// concatenation 1.6 and 0.46 ms (750 TFLOP/s).
+// leaves those taps out.
+//   What bounds it: staging and sums take turns behind barriers with two or three
+// waves a SIMD; matrix cores, other vector instructions and LDS are each busy for
+// less than a third of the cycles.  2 x 16 x 256 x 256 voxels, before and now: 32
+// -> 32 channels 0.38 and 0.19 ms (600 TFLOP/s); 64 + 32 -> 32 with its
+// concatenation 1.6 and 0.47 ms (710 TFLOP/s).
 template <int CA, int CB, int SP, int WT>
 struct ConvTile {
   static constexpr int RPS = 64 / WT, HT = 4 * SP * RPS;
@@ -396,7 +399,7 @@ __global__ void k_conv_flip(const bf16 *__restrict__ w, bf16 *__restrict__ wt, i
 // cores' rate).  The two row groups are added at the end, the slices by
 // k_sum_parts: the order is fixed.  Reading 2 bytes per lane and load from
 // global memory, one tap at a time, took 654 us on average over the layers of
-// a training step on 4 x 8 x 128 x 128 voxels, in this form 44 (600 TFLOP/s).
+// a training step on 4 x 8 x 128 x 128 voxels, in this form 45 (580 TFLOP/s).
 // ---------------------------------------------------------------------------
 constexpr int kGH = 16, kGW = 32, kGThreads = 768;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -664,7 +667,7 @@ __global__ __launch_bounds__(E *RUNS) void k_sum_parts(const float *__restrict__
 // its index by high products, so a 64-bit division costs nothing where they
 // are large and small or narrow volumes fill the chip too.  With one channel
 // per thread the network input took 156 us, the head 147, the pooling 36 on
-// average for 2 x 16 x 256 x 256 voxels; now 35, 23 and 17.
+// average for 2 x 16 x 256 x 256 voxels; now 39, 23 and 16.
 // V: 8, or 1 where the channels or an address do not allow 16-byte accesses.
 template <int V>
 __device__ __forceinline__ void ldv(const bf16 *p, float (&o)[V]) {
@@ -760,7 +763,7 @@ __device__ __forceinline__ void block_channel_sum(const float (&acc)[V], int nc,
 // part[s][c] = sum over the voxels of slice s of g[v][c] (bias gradient): the
 // block's threads hold channel groups and step over the slice's voxels side by
 // side (one thread per channel, all voxels in turn: 163 us on average over the
-// layers of a training step on 4 x 8 x 128 x 128 voxels, 18 in this form)
+// layers of a training step on 4 x 8 x 128 x 128 voxels, 6 in this form)
 template <int V>
 __global__ __launch_bounds__(256) void k_channel_sum(const bf16 *__restrict__ g,
                                                      float *__restrict__ part, long long nvox,
@@ -992,7 +995,7 @@ __global__ void k_mse(const float *__restrict__ out, const float *__restrict__ t
 // and bias gradients per slice of voxels: part[s][c] = sum gout[v] h[v][c] /
 // scale (c < C), part[s][C] = sum gout[v] / scale.  One pass, block = slice:
 // the weight sums, once a thread per channel walking the slice's voxels, were
-// the whole of its 417 us for 4 x 8 x 128 x 128 voxels; now 55.
+// the whole of its 417 us for 4 x 8 x 128 x 128 voxels; now 17.
 // S 0: gh alone, the blocks sharing its voxels; C 0: the bias gradient alone.
 template <int V, int BS>
 __global__ __launch_bounds__(BS) void k_head_bwd(const bf16 *__restrict__ h,
