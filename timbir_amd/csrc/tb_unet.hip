@@ -253,10 +253,9 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
       }
     }
     __syncthreads();
+    if (hw >= H) continue;  // the wave's rows lie past the volume
 #pragma unroll 1
     for (int dy = 0; dy < 3; dy++) {
-      // the wave's rows lie past the volume, or the tap's rows all outside it
-      if (hw >= H || hw + dy - 1 >= H || min(hw + SP * RPS, H) + dy < 2) continue;
       const bf16 *wt = wl + (size_t)(dz * 9 + dy * 3) * Cout * Cin;
       // voxels 4 q + t - 1 of chunk c, t = 0 .. 5; of the half-size tensor
       // their parents 2 q + u - 1, u = (t + 1) / 2
@@ -1231,13 +1230,15 @@ extern "C" int tb_nn_conv3d(const void *in, const void *w, const float *bias, vo
                      : cin == 128 ? conv_pick<0, 4>(planes, h, wd, cout)
                      : cin == 192 ? conv_pick<0, 6>(planes, h, wd, cout)
                                   : ConvForm{nullptr, 0, 0};
-  // Unstaged: volumes of one to three rows that fill the chip, whose tiles are
-  // empty by half and more (512 planes of 1 x 32, 128 -> 128 channels: 81 us
-  // staged, 38 unstaged; 16 planes of it 18 and 23), other channels, an output
-  // that 16-byte stores do not allow, and more tiles than a launch holds.
+  // Unstaged: planes of one row, two thirds of whose taps lie outside (4 planes of
+  // one voxel, 128 -> 128 channels: 27 us staged, 16 unstaged; not one long row
+  // alone), volumes of two or three rows that fill the chip, whose tiles are empty
+  // by half and more (512 planes of 2 x 4, 128 -> 64: 74 and 42), other channels, an
+  // output that 16-byte stores do not allow, and more tiles than a launch holds.
   const long long strips = (wd + 63LL) / 64 * 64 * h;
   const bool empty = f.slots > 2 * strips || (f.slots == 2 * strips && (cin >= 96 || wd <= 8));
-  if (f.fn && al16(out) && !(empty && f.blocks >= 512) && f.blocks <= kMaxBlocks)
+  const bool unstaged = (h == 1 && (planes > 1 || wd <= 32)) || (empty && f.blocks >= 512);
+  if (f.fn && al16(out) && !unstaged && f.blocks <= kMaxBlocks)
     return f.fn(nullptr, in, w, bias, out, n, d, h, wd, cout, relu, out_f32, s);
   const int MB = 4, NB = 2;
   const long long waves = planes * h * ((wd + 16 * MB - 1) / (16 * MB)) * (cout / (16 * NB));
