@@ -186,3 +186,26 @@ def test_prior_cost_at_infinities_and_the_largest_values(where):
         assert np.isfinite(ref) and abs(got - ref) <= 1e-12 * abs(ref), (got, ref)
     else:
         assert np.isnan(ref) and np.isnan(got), (got, ref)
+
+
+def test_fbp_of_more_frames_than_one_launch_has_blocks():
+    """2^24 + 3 frames of 4 x 4 pixels, the views all in frame 2^24 - 1: its
+    back-projection stands there, equal to that of one such frame alone, and
+    every other frame is zero."""
+    print("fbp of 2^24 frames", flush=True)
+    F, at = (1 << 24) + 3, (1 << 24) - 1
+    one = datagen.tiny(N=4, nz=1, n_frames=1, n_views=8)
+    st = tb.Stage(one)
+    st.init_fbp()
+    want = st.object()
+    st.close()
+    many = dict(one, recon_num=F, recon_times=np.arange(F + 1, dtype=np.float64).astype(np.float32),
+                proj_times=np.full(8, at, np.float32))
+    st = tb.Stage(many)
+    st.init_fbp()
+    got = st.object()
+    st.close()
+    assert np.abs(want).max() > 0
+    np.testing.assert_array_equal(got[at], want[0])
+    got[at] = 0.0
+    assert not got.any()

@@ -23,7 +23,7 @@ __global__ void k_to_ref_layout(KP, const float *, float *);
 __global__ void k_fwd_interleave(KP, float4 *);
 __global__ void k_fbp_filter(KP, float *, int);
 template <int NZ>
-__global__ void k_fbp_back(KP, const float *, int, int);
+__global__ void k_fbp_back(KP, const float *, int, int, int);
 __global__ void k_forward(KP, const int *, const float4 *, float *, int);
 __global__ void k_upsample(const float *, float *, int, int, int, int, int);
 template <int NT>
@@ -76,6 +76,7 @@ __global__ void k_mag_sum(KP, double *);
 __global__ void k_fill_f64(double *, size_t, double);
 __global__ void k_fill_f32(float *, size_t, float);
 __global__ void k_fill_u64(unsigned long long *, size_t);
+template <int T>
 __global__ void k_build_order(KP, int);
 }  // namespace tb
 
@@ -863,19 +864,24 @@ extern "C" int tb_init_fbp(tb_stage *st) {
   HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_fbp_filter),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   HIPCHK(dalloc(&q, (size_t)st->N_z * st->N_p * st->N_r));
-  hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, ngroups), dim3(512), lds, st->stream, P, q, per);
+  // (a launch's threads along an axis are counted in 32 bits)
+  const int ft = st->N_p < (1 << 23) ? 512 : 256;
+  hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, ngroups), dim3(ft), lds, st->stream, P, q, per);
   // the groups of kFwdZ slices, then the remainder's
   static_assert(kFwdZ == 8, "one kernel for each number of slices");
-  void (*const back[kFwdZ + 1])(KP, const float *, int, int) = {
+  void (*const back[kFwdZ + 1])(KP, const float *, int, int, int) = {
       nullptr,       k_fbp_back<1>, k_fbp_back<2>, k_fbp_back<3>, k_fbp_back<4>,
       k_fbp_back<5>, k_fbp_back<6>, k_fbp_back<7>, k_fbp_back<8>};
-  const size_t runs = (st->nxy() + 255) / 256 * st->N_time;
+  const size_t runs = (st->nxy() + 255) / 256;
   const int full = st->N_z / kFwdZ, rest = st->N_z % kFwdZ;
-  if (full)
-    hipLaunchKernelGGL(back[kFwdZ], dim3((unsigned)(runs * full)), dim3(256), 0, st->stream, P, q,
-                       0, full);
-  if (rest)
-    hipLaunchKernelGGL(back[rest], dim3((unsigned)runs), dim3(256), 0, st->stream, P, q, full, 1);
+  auto launch = [&](int nz, int g0, int groups) {
+    const size_t F = st->N_time, most = std::max<size_t>(1, ((size_t)1 << 23) / (runs * groups));
+    for (size_t f0 = 0; f0 < F; f0 += most)
+      hipLaunchKernelGGL(back[nz], dim3((unsigned)(std::min(most, F - f0) * runs * groups)),
+                         dim3(256), 0, st->stream, P, q, g0, groups, (int)f0);
+  };
+  if (full) launch(kFwdZ, 0, full);
+  if (rest) launch(rest, full, 1);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess) err = hipStreamSynchronize(st->stream);
   (void)hipFree(q);
@@ -971,7 +977,11 @@ extern "C" int tb_variance_update(tb_stage *st) {
 static int ensure_order(tb_stage *st, int iter) {
   if (st->ord_iter == iter) return 0;
   KP P = st->kp();
-  hipLaunchKernelGGL(k_build_order, dim3(st->N_time * st->N_z), dim3(1024), 0, st->stream, P, iter);
+  const int cells = st->N_time * st->N_z;
+  if (cells < (1 << 22))
+    hipLaunchKernelGGL(k_build_order<1024>, dim3(cells), dim3(1024), 0, st->stream, P, iter);
+  else
+    hipLaunchKernelGGL(k_build_order<256>, dim3(cells), dim3(256), 0, st->stream, P, iter);
   HIPCHK(hipGetLastError());
   st->ord_iter = iter;
   return 0;

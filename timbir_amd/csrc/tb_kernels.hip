@@ -360,8 +360,8 @@ __global__ __launch_bounds__(512) void k_fbp_filter(KP P, float *__restrict__ q,
   }
 }
 
-// thread: one pixel of one frame, the NZ slices of a group (blocks: frame, group
-// g0 .. g0 + ngroups - 1, run of pixels)
+// thread: one pixel of one frame, the NZ slices of a group (blocks: frame from f0
+// on, group g0 .. g0 + ngroups - 1, run of pixels)
 template <int NZ>
 __device__ __forceinline__ void ld_slices(const float *p, float (&o)[NZ]) {
   if constexpr (NZ % 4 == 0) {
@@ -377,10 +377,10 @@ __device__ __forceinline__ void ld_slices(const float *p, float (&o)[NZ]) {
 }
 template <int NZ>
 __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q, int g0,
-                                                  int ngroups) {
+                                                  int ngroups, int f0) {
   const int Nxy = P.N_x * P.N_y;
-  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, f = fg / ngroups,
-            g = g0 + fg - f * ngroups;
+  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, fl = fg / ngroups,
+            g = g0 + fg - fl * ngroups, f = f0 + fl;
   const int vb = P.view_off[f], nv = P.view_off[f + 1] - vb;
   const float *qg = q + (size_t)g * kFwdZ * P.N_p * P.N_r;
   float *ob = P.obj + ((size_t)f * P.N_z + g * kFwdZ) * Nxy;
@@ -421,14 +421,14 @@ __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict_
     for (int i = 0; i < NZ; i++) ob[(size_t)i * Nxy + pix] = in ? (float)(acc[i] * kPi / nv) : 0.0f;
   }
 }
-template __global__ void k_fbp_back<1>(KP, const float *, int, int);
-template __global__ void k_fbp_back<2>(KP, const float *, int, int);
-template __global__ void k_fbp_back<3>(KP, const float *, int, int);
-template __global__ void k_fbp_back<4>(KP, const float *, int, int);
-template __global__ void k_fbp_back<5>(KP, const float *, int, int);
-template __global__ void k_fbp_back<6>(KP, const float *, int, int);
-template __global__ void k_fbp_back<7>(KP, const float *, int, int);
-template __global__ void k_fbp_back<8>(KP, const float *, int, int);
+template __global__ void k_fbp_back<1>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<2>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<3>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<4>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<5>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<6>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<7>(KP, const float *, int, int, int);
+template __global__ void k_fbp_back<8>(KP, const float *, int, int, int);
 
 // ---------------------------------------------------------------------------
 // Voxel update: one workgroup per cell of one colour, voxels in sequence.

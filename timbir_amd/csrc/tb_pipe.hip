@@ -45,10 +45,11 @@ namespace tb {
 // column records and neighbours).  One workgroup per cell, of 16 waves: what
 // bounds it is the run of appends, each behind a barrier, one for as many
 // pixels as the workgroup has threads (four cells of 128 x 128 or 192 x 192
-// pixels, mean: 135 us with 4 waves, 56 with 16).
-constexpr int kOrdThreads = 1024;
-__global__ __launch_bounds__(kOrdThreads) void k_build_order(KP P, int iter) {
-  constexpr int NW = kOrdThreads / 64;
+// pixels, mean: 135 us with 4 waves, 56 with 16).  T threads: 1024, or 256 where
+// the cells' threads would exceed a launch's 2^32.
+template <int T>
+__global__ __launch_bounds__(T) void k_build_order(KP P, int iter) {
+  constexpr int NW = T / 64;
   const int cell = blockIdx.x;
   const int f = cell / P.N_z, z = cell - f * P.N_z;
   const int Nxy = P.N_x * P.N_y;
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(kOrdThreads) void k_build_order(KP P, int iter) {
   if (P.hicd_order == 1) {
     for (int j = 0; j < P.K; j++) {
       if (threadIdx.x == 0) off[j] = min(base, P.ord_cap);
-      for (int start = 0; start < Nxy; start += kOrdThreads) {
+      for (int start = 0; start < Nxy; start += T) {
         const int pix = start + threadIdx.x;
         bool ok = false;
         if (pix < Nxy && P.mask[pix] == 1) {
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(kOrdThreads) void k_build_order(KP P, int iter) {
       }
     }
   } else {
-    for (int start = 0; start < Nxy; start += kOrdThreads) {
+    for (int start = 0; start < Nxy; start += T) {
       const int n = start + threadIdx.x;
       int pix = 0;
       bool ok = false;
@@ -105,6 +106,8 @@ __global__ __launch_bounds__(kOrdThreads) void k_build_order(KP P, int iter) {
   }
   if (threadIdx.x == 0) off[P.K] = min(base, P.ord_cap);
 }
+template __global__ void k_build_order<1024>(KP, int);
+template __global__ void k_build_order<256>(KP, int);
 
 __device__ __forceinline__ void wait_vm_all() {
   __builtin_amdgcn_sched_barrier(0);
