@@ -116,3 +116,40 @@ def test_voxels_in_flight_of_wide_columns(kern, N, nz, views, mult, raster):
         g.close()
     finally:
         tb.set_options(kernel=old.kernel, hicd_order=old.hicd_order)
+
+
+@pytest.mark.parametrize("kern", [2, 3, 4, 8])
+@pytest.mark.parametrize("seed", [0, 1, 2])
+@pytest.mark.parametrize("side", [-1, 1])
+def test_huber_side_inside_the_band(kern, seed, side):
+    """Products that round, e^2 w off T^2 by 2.5e-7 to 9e-7 of it: inside the
+    rounded decision's band and four times outside what huber_sel may err by
+    (2^-24).  Every entry takes its side, to the tolerance above."""
+    from fractions import Fraction
+    rng = np.random.default_rng(seed)
+    while True:
+        T, e = np.float32(rng.uniform(1, 5)), np.float32(rng.uniform(0.05, 0.5))
+        w = np.float32(float(T) ** 2 / float(e) ** 2 * (1 + side * rng.uniform(2.5e-7, 9e-7)))
+        off = Fraction(float(e)) ** 2 * Fraction(float(w)) / Fraction(float(T)) ** 2 - 1
+        if 2.5e-7 <= side * off <= 9e-7 and Fraction(float(e)) ** 2 != Fraction(float(e * e)):
+            break
+    print(f"huber band e={e!r} w={w!r} T={T!r} off={float(off):.2e} kernel={kern}", flush=True)
+    scan = datagen.tiny(N=16, nz=2, n_frames=1, n_views=24, sig_s=0.005, sig_t=0.01,
+                        quad_convex=0, c_s=1.0, c_t=1.0)
+    scan["projections"] = np.full_like(scan["projections"], e)
+    scan["weights"] = np.full_like(scan["weights"], w)
+    scan["huber_T"] = float(T)
+    old = tb.get_options().kernel
+    tb.set_options(kernel=kern)
+    try:
+        o = pyorc.Problem(scan, opt=pyorc.options(schedule=pyorc.SCHED_COLOUR))
+        g = tb.Stage(scan)
+        o.init_error_sino()
+        g.init_error_sino()
+        vo = o.voxel_update(0, 1, 8, 8)
+        vg = g.voxel_update(0, 1, 8, 8)
+        assert abs(vg - vo) <= 2e-5 * abs(vo), (vg, vo)
+        check_kernel(g, kern)
+        g.close()
+    finally:
+        tb.set_options(kernel=old)
