@@ -22,8 +22,8 @@ __global__ void k_transpose_in(KP, const float *, const float *, double);
 __global__ void k_to_ref_layout(KP, const float *, float *);
 __global__ void k_fwd_interleave(KP, float4 *);
 __global__ void k_fbp_filter(KP, float *, int);
-template <int NZ>
-__global__ void k_fbp_back(KP, const float *, int, int, int);
+template <bool FULL, int REST>
+__global__ void k_fbp_back(KP, const float *, int);
 __global__ void k_forward(KP, const int *, const float4 *, float *, int);
 __global__ void k_upsample(const float *, float *, int, int, int, int, int);
 template <int NT>
@@ -867,21 +867,19 @@ extern "C" int tb_init_fbp(tb_stage *st) {
   // (a launch's threads along an axis are counted in 32 bits)
   const int ft = st->N_p < (1 << 23) ? 512 : 256;
   hipLaunchKernelGGL(k_fbp_filter, dim3(st->N_p, ngroups), dim3(ft), lds, st->stream, P, q, per);
-  // the groups of kFwdZ slices, then the remainder's
-  static_assert(kFwdZ == 8, "one kernel for each number of slices");
-  void (*const back[kFwdZ + 1])(KP, const float *, int, int, int) = {
-      nullptr,       k_fbp_back<1>, k_fbp_back<2>, k_fbp_back<3>, k_fbp_back<4>,
-      k_fbp_back<5>, k_fbp_back<6>, k_fbp_back<7>, k_fbp_back<8>};
-  const size_t runs = (st->nxy() + 255) / 256;
-  const int full = st->N_z / kFwdZ, rest = st->N_z % kFwdZ;
-  auto launch = [&](int nz, int g0, int groups) {
-    const size_t F = st->N_time, most = std::max<size_t>(1, ((size_t)1 << 23) / (runs * groups));
-    for (size_t f0 = 0; f0 < F; f0 += most)
-      hipLaunchKernelGGL(back[nz], dim3((unsigned)(std::min(most, F - f0) * runs * groups)),
-                         dim3(256), 0, st->stream, P, q, g0, groups, (int)f0);
-  };
-  if (full) launch(kFwdZ, 0, full);
-  if (rest) launch(rest, full, 1);
+  static_assert(kFwdZ == 8, "a kernel for each remainder");
+  using back_fn = void (*)(KP, const float *, int);
+  static const back_fn back[2][kFwdZ] = {
+      {nullptr, k_fbp_back<false, 1>, k_fbp_back<false, 2>, k_fbp_back<false, 3>,
+       k_fbp_back<false, 4>, k_fbp_back<false, 5>, k_fbp_back<false, 6>, k_fbp_back<false, 7>},
+      {k_fbp_back<true, 0>, k_fbp_back<true, 1>, k_fbp_back<true, 2>, k_fbp_back<true, 3>,
+       k_fbp_back<true, 4>, k_fbp_back<true, 5>, k_fbp_back<true, 6>, k_fbp_back<true, 7>}};
+  const size_t per_frame = (st->nxy() + 255) / 256 * ngroups, F = st->N_time;
+  const size_t most = std::max<size_t>(1, ((size_t)1 << 23) / per_frame);
+  for (size_t f0 = 0; f0 < F; f0 += most)
+    hipLaunchKernelGGL(back[st->N_z >= kFwdZ][st->N_z % kFwdZ],
+                       dim3((unsigned)(std::min(most, F - f0) * per_frame)), dim3(256), 0,
+                       st->stream, P, q, (int)f0);
   hipError_t err = hipGetLastError();
   if (err == hipSuccess) err = hipStreamSynchronize(st->stream);
   (void)hipFree(q);

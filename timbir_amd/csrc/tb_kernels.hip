@@ -360,8 +360,6 @@ __global__ __launch_bounds__(512) void k_fbp_filter(KP P, float *__restrict__ q,
   }
 }
 
-// thread: one pixel of one frame, the NZ slices of a group (blocks: frame from f0
-// on, group g0 .. g0 + ngroups - 1, run of pixels)
 template <int NZ>
 __device__ __forceinline__ void ld_slices(const float *p, float (&o)[NZ]) {
   if constexpr (NZ % 4 == 0) {
@@ -375,16 +373,15 @@ __device__ __forceinline__ void ld_slices(const float *p, float (&o)[NZ]) {
     for (int i = 0; i < NZ; i++) o[i] = p[i];
   }
 }
+
+// one pixel of frame f, the NZ slices of group g
 template <int NZ>
-__global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q, int g0,
-                                                  int ngroups, int f0) {
+__device__ __forceinline__ void fbp_pixel(const KP &P, const float *__restrict__ q, int f, int g,
+                                          int pix) {
   const int Nxy = P.N_x * P.N_y;
-  const int runs = (Nxy + 255) / 256, fg = blockIdx.x / runs, fl = fg / ngroups,
-            g = g0 + fg - fl * ngroups, f = f0 + fl;
   const int vb = P.view_off[f], nv = P.view_off[f + 1] - vb;
   const float *qg = q + (size_t)g * kFwdZ * P.N_p * P.N_r;
   float *ob = P.obj + ((size_t)f * P.N_z + g * kFwdZ) * Nxy;
-  const int pix = (blockIdx.x - fg * runs) * 256 + (int)threadIdx.x;
   if (pix < Nxy) {
     const int row = pix / P.N_x, col = pix - row * P.N_x;
     double acc[NZ];
@@ -421,14 +418,37 @@ __global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict_
     for (int i = 0; i < NZ; i++) ob[(size_t)i * Nxy + pix] = in ? (float)(acc[i] * kPi / nv) : 0.0f;
   }
 }
-template __global__ void k_fbp_back<1>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<2>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<3>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<4>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<5>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<6>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<7>(KP, const float *, int, int, int);
-template __global__ void k_fbp_back<8>(KP, const float *, int, int, int);
+
+// blocks: frame from f0 on, group of slices, run of pixels.  All groups in one
+// launch, FULL of them of kFwdZ slices and then one of REST (one launch for each
+// kind: 93 us for 120 x 120 x 12 slices x 2 frames and 160 views, 58 for both)
+template <bool FULL, int REST>
+__global__ __launch_bounds__(256) void k_fbp_back(KP P, const float *__restrict__ q, int f0) {
+  const int runs = (P.N_x * P.N_y + 255) / 256, ngroups = (P.N_z + kFwdZ - 1) / kFwdZ;
+  const int fg = blockIdx.x / runs, fl = fg / ngroups, g = fg - fl * ngroups;
+  const int pix = (blockIdx.x - fg * runs) * 256 + (int)threadIdx.x;
+  if constexpr (FULL && REST > 0) {
+    if (g + 1 < ngroups) fbp_pixel<kFwdZ>(P, q, f0 + fl, g, pix);
+    else fbp_pixel<REST>(P, q, f0 + fl, g, pix);
+  } else {
+    fbp_pixel<FULL ? kFwdZ : REST>(P, q, f0 + fl, g, pix);
+  }
+}
+template __global__ void k_fbp_back<true, 0>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 1>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 1>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 2>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 2>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 3>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 3>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 4>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 4>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 5>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 5>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 6>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 6>(KP, const float *, int);
+template __global__ void k_fbp_back<true, 7>(KP, const float *, int);
+template __global__ void k_fbp_back<false, 7>(KP, const float *, int);
 
 // ---------------------------------------------------------------------------
 // Voxel update: one workgroup per cell of one colour, voxels in sequence.
