@@ -253,7 +253,10 @@ __global__ __launch_bounds__(256) void k_conv3d_tile(
       }
     }
     __syncthreads();
-    if (hw >= H) continue;  // the wave's rows lie past the volume
+    // a wave past a volume of fewer rows than a tile (not of a last tile alone: its
+    // waves' early end costs the tall volumes' launches more than it saves, 64 -> 64
+    // channels of 16 planes of 114 x 106 144 us with it and 136 without)
+    if (h0 == 0 && hw >= H) continue;
 #pragma unroll 1
     for (int dy = 0; dy < 3; dy++) {
       const bf16 *wt = wl + (size_t)(dz * 9 + dy * 3) * Cout * Cin;
@@ -1201,7 +1204,7 @@ static ConvForm conv_form(long long planes, int h, int wd, int cout) {
 // 64 -> 64 channels, 16 planes of 16 x 16 voxels: 36 us with 64 channels a wave,
 // 23 with 32; 128 -> 128, 64 planes of 16 x 32: 66 and 82.  Two strips per wave for
 // 32 channels of 32 inputs, where the weights' share of the L1 would otherwise
-// bound, unless they fill up more rows.
+// bound, unless they fill up a quarter more rows.
 template <int CA, int CB>
 static ConvForm conv_pick(long long planes, int h, int wd, int cout) {
   constexpr long long few = CA + CB >= 4 ? 256 : 768;
@@ -1209,7 +1212,7 @@ static ConvForm conv_pick(long long planes, int h, int wd, int cout) {
   if constexpr (CA == 0 && CB == 1) {
     if (f.blocks > few && cout % 64 && cout % 96) {
       const ConvForm g = conv_form<CA, CB, 2, 2>(planes, h, wd, cout);
-      if (g.slots <= f.slots) f = g;
+      if (g.slots <= f.slots * 5 / 4) f = g;
     }
   }
   if (f.blocks > few && cout % 64 == 0) f = conv_form<CA, CB, 4, 1>(planes, h, wd, cout);
